@@ -339,6 +339,57 @@ int hsd_seq_rollback(int32_t* seq, int64_t n_drop, int64_t nslab, void* stream);
 /* seq[idx] += delta on the stream (host-known adjustments, e.g. the head's prefill rows). */
 int hsd_seq_add(int32_t* seq, int64_t idx, int64_t delta, void* stream);
 
+/* ------------------------------------------------------------------ prompt chunks
+ * The projections of a prompt chunk on the matrix cores (hsd/model.py:259-279 runs a prompt
+ * in chunks; the block arithmetic is hsd_linear's and hsd_moe_up_relu2's, the summation order
+ * the matrix cores').
+ * hsd_rows_prep: the prologue of hsd_linear (x_kind HSD_X_BF16, HSD_X_RMS or HSD_X_GATED_Z,
+ * the same bits) for T rows -> xp [T, I] bf16. hs non-null: xp's inputs in the order
+ * 0 4 1 5 2 6 3 7 of every 8 and hs [T, 2 GP] bf16, GP = ceil(I/64/8)*8: every 64-input
+ * group's sum as hi + lo (zero past I/64); hs null: the natural order.
+ * I a multiple of 64 (8 without hs; 512 for the gated norm), at most 6144. */
+int hsd_rows_prep(const void* x, int64_t x_ld, int x_kind, const uint16_t* norm_w, float eps,
+                  uint16_t* xp, uint16_t* hs, int64_t T, int64_t I, void* stream);
+
+/* y [T, O] = xn W^T in bf16, W 4-bit (stock layout), from hsd_rows_prep's xp and hs; res
+ * non-null: y = bf16(res + bf16(xn W^T)) (y may be res). I a multiple of 128. */
+int hsd_gemm_q4(const uint16_t* xp, const uint16_t* hs, const uint32_t* w, const uint16_t* s,
+                const uint16_t* b, uint16_t* y, int64_t y_ld, const uint16_t* res, int64_t res_ld,
+                int64_t T, int64_t O, int64_t I, void* stream);
+
+/* y [T, O] = x W^T in bf16 with a bf16 weight [O, I]; permuted: x in hsd_rows_prep's order. */
+int hsd_gemm_bf16(const uint16_t* x, int64_t x_ld, int permuted, const uint16_t* w, uint16_t* y,
+                  int64_t y_ld, int64_t T, int64_t O, int64_t I, void* stream);
+
+/* hsd_prefill_tiles without a workspace, with ntiles[0] = the routed tiles in use. */
+int hsd_moe_tiles(const int32_t* sel, int64_t T, int64_t topk, int64_t E, int64_t tt,
+                  int32_t* tile_e, int32_t* tile_slot, int32_t* ntiles, int32_t* dev_status,
+                  void* stream);
+
+/* hsd_moe_up_relu2 for a chunk: hcat [T, topk*F + FS] from hsd_rows_prep's xp and hs and
+ * hsd_moe_tiles' lists (tt 32 or 64); the slots of experts outside [0, E) are not written.
+ * hsum (nullable, [T, topk + 1, 2 GPH] bf16, GPH = ceil(max(F, FS)/64/8)*8): the sum of every
+ * 64 neurons of a slot's h as hi + lo, for hsd_moe_down_gemm (entries past a slot's groups
+ * are not written). D a multiple of 128. */
+int hsd_moe_up_gemm(const uint16_t* xp, const uint16_t* hs, const int32_t* tile_e,
+                    const int32_t* tile_slot, const int32_t* ntiles, const uint32_t* w1,
+                    const uint16_t* s1, const uint16_t* b1, const uint32_t* sw1,
+                    const uint16_t* ss1, const uint16_t* sb1, uint16_t* hcat, uint16_t* hsum, int64_t T,
+                    int64_t D, int64_t F, int64_t FS, int64_t topk, int64_t E, int64_t tt, void* stream);
+
+/* y = bf16(res + bf16(the MoE down projection)) of a chunk (hsd_sparse_down_residual's result
+ * with the matrix cores' summation order), every row of the neuron-major layout read, from
+ * hsd_moe_up_gemm's hcat and hsum and the same lists. A slot whose expert is outside [0, E) adds
+ * nothing. y may be res. D a multiple of 128. workspace: hsd_moe_down_workspace_bytes. */
+size_t hsd_moe_down_workspace_bytes(int64_t T, int64_t D, int64_t topk);
+int hsd_moe_down_gemm(const uint16_t* hcat, const uint16_t* hsum, const int32_t* sel,
+                      const float* gains, const int32_t* tile_e, const int32_t* tile_slot,
+                      const int32_t* ntiles, const uint32_t* pw, const uint16_t* ps,
+                      const uint16_t* pb, const uint32_t* spw, const uint16_t* sps,
+                      const uint16_t* spb, const uint16_t* res, int64_t res_ld, uint16_t* y,
+                      int64_t y_ld, int64_t T, int64_t D, int64_t F, int64_t FS, int64_t topk,
+                      int64_t E, int64_t tt, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------ prefill
  * Replaces hsd/prefill.py:247-278 `build_tiles(sel, E, tt)`: slots t*topk+k stably
  * sorted by expert (ties by slot id), ceil(count/tt) tiles per expert, then

@@ -1,0 +1,90 @@
+"""A prompt chunk's layers: many consecutive token rows at once (hsd/model.py:259-279 runs a
+prompt in chunks through the blocks).
+
+`prep` normalises the rows once per projection (the bits of nn.linear's prologue), `gemm`
+multiplies them with a 4-bit or bf16 weight, and `moe_up` runs every expert's up projection
+with ReLU^2 over the (token, slot) pairs sorted by expert. The arithmetic is nn.linear's and
+moe.up_relu2's with the matrix cores' summation order.
+"""
+from __future__ import annotations
+
+import torch
+
+from . import _native as N
+from .prefill import num_tiles
+
+
+def group_pitch(I):
+    """Group sums per row and half: I/64 rounded up to 8."""
+    return (I // 64 + 7) // 8 * 8
+
+
+class Rows:
+    """Prepared rows: xp [T, I] bf16 and, for 4-bit weights, the group sums hs [T, 2 GP]."""
+
+    def __init__(self, xp, hs):
+        self.xp, self.hs = xp, hs
+
+
+def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
+    """x [T, I]: bf16 rows (norm: the RMS norm's weight), or with gated_z mamba's z rows (f32,
+    I + I/16 values per row) and the gated norm's weight. sums: for 4-bit weights."""
+    T, I = x.shape
+    kind = N.X_GATED_Z if gated_z else N.X_RMS if norm is not None else N.X_BF16
+    xp = torch.empty((T, I), dtype=torch.bfloat16, device=x.device)
+    hs = torch.empty((T, 2 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
+    N.call("hsd_rows_prep", N.ptr(x), x.stride(0), kind, N.ptr(norm), float(eps), N.ptr(xp), N.ptr(hs), T, I,
+           N.stream(x.device))
+    return Rows(xp, hs)
+
+
+def gemm(rows: Rows, W, residual=None, out=None):
+    """bf16 y [T, O] = xn W^T (W: nn.QWeight); residual: y = bf16(residual + bf16(xn W^T))
+    (4-bit weights; out may be residual)."""
+    T = rows.xp.shape[0]
+    y = out if out is not None else torch.empty((T, W.O), dtype=torch.bfloat16, device=rows.xp.device)
+    st = N.stream(rows.xp.device)
+    if W.q4:
+        N.call("hsd_gemm_q4", N.ptr(rows.xp), N.ptr(rows.hs), N.ptr(W.w), N.ptr(W.scales), N.ptr(W.biases), N.ptr(y),
+               y.stride(0), N.ptr(residual), 0 if residual is None else residual.stride(0), T, W.O, W.I, st)
+    else:
+        N.call("hsd_gemm_bf16", N.ptr(rows.xp), rows.xp.stride(0), 0 if rows.hs is None else 1, N.ptr(W.w), N.ptr(y),
+               y.stride(0), T, W.O, W.I, st)
+    return y
+
+
+def moe_tiles(sel, E, tt, status=None):
+    """prefill.build_tiles' lists and the routed tiles in use: (tile_e, tile_slot, ntiles [1])."""
+    T, K = sel.shape
+    NT = num_tiles(T, K, E, tt)
+    t = torch.empty(NT * (tt + 1) + 1, dtype=torch.int32, device=sel.device)
+    tile_e, tile_slot, ntiles = t[:NT], t[NT:NT * (tt + 1)], t[NT * (tt + 1):]
+    N.call("hsd_moe_tiles", N.ptr(sel), T, K, E, tt, N.ptr(tile_e), N.ptr(tile_slot), N.ptr(ntiles), N.ptr(status),
+           N.stream(sel.device))
+    return tile_e, tile_slot, ntiles
+
+
+def moe_up(rows: Rows, tiles, w1, s1, b1, sw1, ss1, sb1, *, topk, tt):
+    """moe.up_relu2 of a chunk -> (hcat [T, topk*F + FS] bf16, its 64-neuron group sums)."""
+    T, D = rows.xp.shape
+    E, F, FS = w1.shape[0], w1.shape[1], sw1.shape[0]
+    hcat = torch.empty((T, topk * F + FS), dtype=torch.bfloat16, device=rows.xp.device)
+    hsum = torch.empty((T, topk + 1, 2 * group_pitch(max(F, FS))), dtype=torch.bfloat16, device=rows.xp.device)
+    N.call("hsd_moe_up_gemm", N.ptr(rows.xp), N.ptr(rows.hs), N.ptr(tiles[0]), N.ptr(tiles[1]), N.ptr(tiles[2]),
+           N.ptr(N.as_words(w1)), N.ptr(s1), N.ptr(b1), N.ptr(N.as_words(sw1)), N.ptr(ss1), N.ptr(sb1), N.ptr(hcat),
+           N.ptr(hsum), T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
+    return hcat, hsum
+
+
+def moe_down(x, hcat, hsum, sel, gains, tiles, pw, ps, pb, spw, sps, spb, *, topk, tt, out=None):
+    """bf16(x + bf16(the MoE down projection)) of a chunk, every row of the neuron-major layout
+    read (out may be x)."""
+    T, D = x.shape
+    E, F, FS = pw.shape[0], pw.shape[1], spw.shape[0]
+    y = out if out is not None else torch.empty((T, D), dtype=torch.bfloat16, device=x.device)
+    nb = N.lib().hsd_moe_down_workspace_bytes(T, D, topk)
+    ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
+    N.call("hsd_moe_down_gemm", N.ptr(hcat), N.ptr(hsum), N.ptr(sel), N.ptr(gains), N.ptr(tiles[0]), N.ptr(tiles[1]),
+           N.ptr(tiles[2]), N.ptr(N.as_words(pw)), N.ptr(ps), N.ptr(pb), N.ptr(N.as_words(spw)), N.ptr(sps), N.ptr(spb),
+           N.ptr(x), x.stride(0), N.ptr(y), y.stride(0), T, D, F, FS, topk, E, tt, N.ptr(ws), nb, N.stream(x.device))
+    return y

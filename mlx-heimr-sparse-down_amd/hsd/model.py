@@ -31,10 +31,11 @@ import numpy as np
 import torch
 
 from . import _native as N
-from . import layout, mamba as M, nn
+from . import chunk, layout, mamba as M, nn
 from .moe import route_up_relu2, router_topk, up_relu2
 
 NSLAB = 4          # Mamba checkpoint ring: a verify of up to 3 rows
+CHUNK_MIN = 4      # more token rows than this run as a chunk on the matrix cores
 ROWS = (1, 3)      # row counts with preallocated buffers: decode, verify / prefill steps
 
 
@@ -301,11 +302,14 @@ class MoEBlock:
         return self.prefill_sparse(x) if mode == "sparse" else self.decode_dense(x)
 
     def prefill_sparse(self, x, tt=32):
-        """model.py:156-175: x [T, D] -> x + the MoE output, the down projection as the
-        grouped MFMA GEMM over each expert tile's union of live rows (tiles, unions and
-        the GEMM on the device)."""
+        """model.py:156-175: x [T, D] -> x + the MoE output (a new tensor): the up projections
+        and the down projection as grouped matrix products over the tiles of each expert's
+        tokens. A few rows: the decode front end, and the down projection over each tile's
+        union of live rows (tiles, unions and the GEMM on the device)."""
         from . import prefill as P
         c = self.cfg
+        if c.hidden % 128 == 0 and x.shape[0] > CHUNK_MIN:
+            return self._chunk(N.contig(x), tt)
         hcat, sel, gains = self._front_packed(x)
         tiles = P.build_tiles(sel, c.n_experts, tt)
         union = P.build_union(hcat, tiles[0], tiles[1], F=c.moe_inter, FS=c.shared_inter, topk=c.topk,
@@ -314,6 +318,23 @@ class MoEBlock:
                                   F=c.moe_inter, FS=c.shared_inter, D=c.hidden, topk=c.topk, E=c.n_experts, tt=tt,
                                   tiles=tiles, union=union)
         return x + y.to(x.dtype)
+
+    def _chunk(self, x, tt, out=None):
+        """A prompt chunk's rows on the matrix cores (hsd.chunk): the projections run over the
+        tiles of (token, slot) pairs sorted by expert, so an expert's weights are read once
+        per tile and not once per token, and every down row of a tile (with the tokens of a
+        tile nearly every row has a live one). No row's result depends on the zeros of another,
+        so both modes are the same bits."""
+        c = self.cfg
+        rows = chunk.prep(x, norm=self.norm_w, eps=c.eps)
+        logits = chunk.gemm(rows, self.gate)
+        sel, gains = router_topk(logits, self.e_bias, topk=c.topk, routed_scale=c.routed_scale, norm_topk=c.norm_topk)
+        tiles = chunk.moe_tiles(sel, c.n_experts, tt)
+        hcat, hsum = chunk.moe_up(rows, tiles, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, topk=c.topk, tt=tt)
+        if self.trace is not None:                       # calibration / statistics only
+            self.trace.append(float((hcat == 0).float().mean().item()))
+        return chunk.moe_down(x, hcat, hsum, sel, gains, tiles, self.pw, self.ps, self.pb, self.spw, self.sps, self.spb,
+                              topk=c.topk, tt=tt, out=out)
 
     def nbytes(self):
         t = [self.gate.w, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, self.pw, self.ps, self.pb,
