@@ -390,6 +390,34 @@ int hsd_moe_down_gemm(const uint16_t* hcat, const uint16_t* hsum, const int32_t*
                       int64_t y_ld, int64_t T, int64_t D, int64_t F, int64_t FS, int64_t topk,
                       int64_t E, int64_t tt, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The mixers of a prompt chunk: T consecutive rows at positions P = *pos .. of a prompt of
+ * Ttot tokens; the rows past it (V = clamp(Ttot - P, 0, T) are inside) leave nothing behind.
+ * hsd_mamba_scan: T rows of hsd_mamba_ssm_gated (the same bits) without the per-row
+ * checkpoints: the state after row V - 1 goes to slab (cur + V) % nslab (V == 0: nothing).
+ * workspace: hsd_mamba_scan_workspace_bytes. */
+size_t hsd_mamba_scan_workspace_bytes(int64_t T, int64_t H, int64_t P, int64_t N, int64_t G);
+int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const uint16_t* dt_raw, int64_t dt_ld,
+                   const uint16_t* gate, int64_t gate_ld, const uint16_t* conv_w,
+                   const uint16_t* conv_b, const float* A_log, const float* dt_bias, const float* Dp,
+                   float* ssm_slabs, uint16_t* conv_slabs, const int32_t* cur, int64_t nslab,
+                   const int32_t* pos, float* z, int64_t z_ld, int64_t T, int64_t Ttot, int64_t H,
+                   int64_t P, int64_t N, int64_t G, float dt_lo, float dt_hi, int32_t* dev_status,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
+/* hsd_attn_decode for a chunk: the keys and values of rows 0 .. V-1 (qkv's k | v columns) go
+ * to the cache at P .., then out [T, HQ*HD] (null: the cache only) = causal attention of
+ * every row over keys 0 .. P+r. HD = 128, HQ/HKV a multiple of 4. P < 0 or P + V > smax:
+ * HSD_STATUS_BAD_STATE, nothing written to the cache, out 0. */
+int hsd_attn_prompt(const uint16_t* qkv, int64_t qkv_ld, int64_t T, int64_t Ttot, uint16_t* k_cache,
+                    uint16_t* v_cache, int64_t smax, const int32_t* pos, uint16_t* out,
+                    int64_t out_ld, int64_t HQ, int64_t HKV, int64_t HD, float scale,
+                    int32_t* dev_status, void* stream);
+
+/* hsd_gather_tokens and hsd_prefill_advance for any number of rows. */
+int hsd_prompt_tokens(const int32_t* src, int64_t n, const int32_t* seq, int64_t offset, int64_t count,
+                      int32_t* dst, void* stream);
+int hsd_prompt_advance(int32_t* seq, int64_t T, int64_t B, int64_t nslab, void* stream);
+
 /* ------------------------------------------------------------------ prefill
  * Replaces hsd/prefill.py:247-278 `build_tiles(sel, E, tt)`: slots t*topk+k stably
  * sorted by expert (ties by slot id), ceil(count/tt) tiles per expert, then

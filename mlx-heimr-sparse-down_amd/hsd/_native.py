@@ -108,6 +108,13 @@ _SIGS = {
     "hsd_gemm_q4": (_c_int, [_vp] * 6 + [_c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "hsd_gemm_bf16": (_c_int, [_vp, _c_i64, _c_int, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "hsd_moe_tiles": (_c_int, [_vp] + [_c_i64] * 4 + [_vp] * 5),
+    "hsd_mamba_scan_workspace_bytes": (_c_size, [_c_i64] * 5),
+    "hsd_mamba_scan": (_c_int, [_vp, _c_i64, _vp, _c_i64, _vp, _c_i64] + [_vp] * 8 + [_c_i64, _vp, _vp, _c_i64]
+                       + [_c_i64] * 6 + [_c_float] * 2 + [_vp, _vp, _c_size, _vp]),
+    "hsd_attn_prompt": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _c_i64, _vp, _vp] + [_c_i64] * 4
+                        + [_c_float, _vp, _vp]),
+    "hsd_prompt_tokens": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _vp]),
+    "hsd_prompt_advance": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp]),
     "hsd_moe_up_gemm": (_c_int, [_vp] * 13 + [_c_i64] * 7 + [_vp]),
     "hsd_moe_down_workspace_bytes": (_c_size, [_c_i64] * 3),
     "hsd_moe_down_gemm": (_c_int, [_vp] * 14 + [_c_i64, _vp, _c_i64] + [_c_i64] * 7 + [_vp, _c_size, _vp]),

@@ -4,9 +4,14 @@ prompt in chunks through the blocks).
 `prep` normalises the rows once per projection (the bits of nn.linear's prologue), `gemm`
 multiplies them with a 4-bit or bf16 weight, and `moe_up` runs every expert's up projection
 with ReLU^2 over the (token, slot) pairs sorted by expert. The arithmetic is nn.linear's and
-moe.up_relu2's with the matrix cores' summation order.
+moe.up_relu2's with the matrix cores' summation order. `scan` and `attention` are the
+Mamba-2 recurrence and the causal attention of the chunk's rows at positions *pos .. of a
+prompt of `total` tokens.
 """
 from __future__ import annotations
+
+import ctypes
+import math
 
 import torch
 
@@ -88,3 +93,34 @@ def moe_down(x, hcat, hsum, sel, gains, tiles, pw, ps, pb, spw, sps, spb, *, top
            N.ptr(tiles[2]), N.ptr(N.as_words(pw)), N.ptr(ps), N.ptr(pb), N.ptr(N.as_words(spw)), N.ptr(sps), N.ptr(spb),
            N.ptr(x), x.stride(0), N.ptr(y), y.stride(0), T, D, F, FS, topk, E, tt, N.ptr(ws), nb, N.stream(x.device))
     return y
+
+
+def scan(mixer, proj, cache, pos, total, status=None):
+    """mamba.ssm_rows(..., gated=True) of a chunk from the in_proj output [T, 2*H*P + 2*G*N + H]:
+    -> z [T, H*P] f32 (a view of rows of H*P + H*P/16 values); the state after the chunk goes to
+    the ring slab the advanced ring index names."""
+    T = proj.shape[0]
+    H, P, Nst, G = mixer.num_heads, mixer.head_dim, mixer.ssm_state_size, mixer.n_groups
+    DI, CD = mixer.intermediate_size, mixer.conv_dim
+    z = torch.empty((T, DI + DI // 16), dtype=torch.float32, device=proj.device)
+    nb = N.lib().hsd_mamba_scan_workspace_bytes(T, H, P, Nst, G)
+    ws = torch.empty(nb, dtype=torch.uint8, device=proj.device)
+    base, es, ld = proj.data_ptr(), proj.element_size(), proj.stride(0)
+    lo, hi = mixer.time_step_limit
+    N.call("hsd_mamba_scan", ctypes.c_void_p(base + DI * es), ld, ctypes.c_void_p(base + (DI + CD) * es), ld, N.ptr(proj),
+           ld, N.ptr(N.contig(mixer.conv_w)), N.ptr(N.contig(mixer.conv_b)), N.ptr(N.contig(mixer.A_log)),
+           N.ptr(N.contig(mixer.dt_bias)), N.ptr(N.contig(mixer.D)), N.ptr(cache.ssm), N.ptr(cache.conv),
+           N.ptr(cache.cur), cache.nslab, N.ptr(pos), N.ptr(z), z.stride(0), T, total, H, P, Nst, G, float(lo), float(hi),
+           N.ptr(status), N.ptr(ws), nb, N.stream(proj.device))
+    return z[:, :DI]
+
+
+def attention(qkv, kv, pos, total, *, n_heads, n_kv_heads, head_dim=128, cache_only=False, status=None):
+    """nn.attention of a chunk: the rows' keys and values into the cache, then causal attention
+    -> [T, HQ*HD] bf16 (None with cache_only)."""
+    T = qkv.shape[0]
+    out = None if cache_only else torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
+    N.call("hsd_attn_prompt", N.ptr(qkv), qkv.stride(0), T, total, N.ptr(kv.k), N.ptr(kv.v), kv.smax, N.ptr(pos),
+           N.ptr(out), 0 if out is None else out.stride(0), n_heads, n_kv_heads, head_dim, 1.0 / math.sqrt(head_dim),
+           N.ptr(status), N.stream(qkv.device))
+    return out

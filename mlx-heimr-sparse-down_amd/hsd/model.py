@@ -36,6 +36,7 @@ from .moe import route_up_relu2, router_topk, up_relu2
 
 NSLAB = 4          # Mamba checkpoint ring: a verify of up to 3 rows
 CHUNK_MIN = 4      # more token rows than this run as a chunk on the matrix cores
+CHUNK_ROWS = 2048  # prompt rows per chunk (the reference's chunk, model.py:259)
 ROWS = (1, 3)      # row counts with preallocated buffers: decode, verify / prefill steps
 
 
@@ -150,6 +151,13 @@ class MambaBlock:
         nn.linear(z, self.out_proj, norm=self.mixer.norm_w, eps=self.eps, gated_z=True, residual=x, out=x)
         return x
 
+    def chunk(self, x, cache: M.MambaCache, pos, total, status=None):
+        """x [T, D] (updated in place): a prompt chunk's rows."""
+        proj = chunk.gemm(chunk.prep(x, norm=self.norm_w, eps=self.eps), self.in_proj)
+        z = chunk.scan(self.mixer, proj, cache, pos, total, status=status)
+        chunk.gemm(chunk.prep(z, norm=self.mixer.norm_w, eps=self.eps, gated_z=True), self.out_proj, residual=x, out=x)
+        return x
+
     def nbytes(self):
         return self.in_proj.nbytes() + self.out_proj.nbytes()
 
@@ -176,6 +184,15 @@ class AttnBlock:
         o = nn.attention(qkv, kv, pos, n_heads=c.attn_heads, n_kv_heads=c.kv_heads, head_dim=c.head_dim,
                          out=buf["att"][:B], workspace=buf["ws_attn"], status=status)
         nn.linear(o, self.o_proj, residual=x, out=x)
+        return x
+
+    def chunk(self, x, kv: nn.KVCache, pos, total, status=None):
+        """x [T, D] (updated in place): a prompt chunk's rows."""
+        c = self.cfg
+        qkv = chunk.gemm(chunk.prep(x, norm=self.norm_w, eps=c.eps), self.qkv)
+        o = chunk.attention(qkv, kv, pos, total, n_heads=c.attn_heads, n_kv_heads=c.kv_heads, head_dim=c.head_dim,
+                            status=status)
+        chunk.gemm(chunk.prep(o), self.o_proj, residual=x, out=x)
         return x
 
     def nbytes(self):
@@ -335,6 +352,12 @@ class MoEBlock:
             self.trace.append(float((hcat == 0).float().mean().item()))
         return chunk.moe_down(x, hcat, hsum, sel, gains, tiles, self.pw, self.ps, self.pb, self.spw, self.sps, self.spb,
                               topk=c.topk, tt=tt, out=out)
+
+    def chunk(self, x):
+        """x [T, D] (updated in place): a prompt chunk's rows. 64-slot tiles once an expert has
+        about that many tokens (they share the nibbles' unpacking between two row blocks)."""
+        c = self.cfg
+        return self._chunk(x, 64 if x.shape[0] * c.topk >= 48 * c.n_experts else 32, out=x)
 
     def nbytes(self):
         t = [self.gate.w, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, self.pw, self.ps, self.pb,
@@ -601,7 +624,36 @@ class NemotronModel:
             nn.linear(x, self.lm_head, norm=hd.final_norm, eps=c.eps, argmax_keys=keys, xn_out=buf["hn"][:B])
         return x
 
-    # ---- prefill (model.py:259-279), in steps of 3 rows through the decode kernels
+    # ---- prefill (model.py:259-279): chunks of CHUNK_ROWS rows on the matrix cores, or (few
+    # tokens, shapes those kernels do not take) steps of 3 rows through the decode kernels
+    def _chunkable(self):
+        c = self.cfg
+        return (c.hidden % 128 == 0 and c.hidden <= 3072 and c.moe_inter % 64 == 0 and c.shared_inter % 64 == 0
+                and c.mamba_inner % 512 == 0 and c.mamba_inner <= 6144 and c.mamba_head_dim % 16 == 0
+                and c.ssm_state == 128 and c.head_dim == 128 and c.attn_heads % (4 * c.kv_heads) == 0
+                and c.attn_heads * c.head_dim <= 6144 and c.topk <= 8 and c.n_experts <= 256)
+
+    def _prefill_chunk(self, prompt_dev, T, B, cache, with_head):
+        """B rows from the cache's position on -> their residual stream [B, D]."""
+        st, seq, c = N.stream(self.device), cache.seq, self.cfg
+        ids = torch.empty(B, dtype=torch.int32, device=self.device)
+        N.call("hsd_prompt_tokens", N.ptr(prompt_dev), T, N.ptr(seq), 0, B, N.ptr(ids), st)
+        x = self.embed(ids, status=cache.status)
+        for t, blk, lc in zip(c.pattern, self.blocks, cache.layers):
+            if t == "E":
+                blk.chunk(x)
+            else:
+                blk.chunk(x, lc, cache.pos, T, status=cache.status)
+        if with_head:
+            N.call("hsd_prompt_tokens", N.ptr(prompt_dev), T, N.ptr(seq), 1, B, N.ptr(ids), st)
+            hd = self.mtp
+            pair = nn.head_input(ids, x, self.embedding, hd.enorm, hd.hnorm, eps=c.eps, status=cache.status)
+            hx = chunk.gemm(chunk.prep(pair, sums=False), hd.eh_proj)
+            hd.attn.chunk(hx, cache.head_kv, cache.head_pos, T - 1, status=cache.status)
+            hd.moe.chunk(hx)
+        N.call("hsd_prompt_advance", N.ptr(seq), T, B, NSLAB, st)
+        return x
+
     def _prefill_step(self, prompt_dev, T, cache, with_head):
         buf = self._bufs[3]
         ids = buf["ids"][:3]
@@ -618,8 +670,7 @@ class NemotronModel:
     def prefill(self, tokens, cache: ModelCache, with_head=None, graph=True):
         """tokens [T] (host ints or a tensor) -> the residual stream of the last position
         [1, D] (pre norm_f), with every cache advanced by T rows (and, with the MTP head,
-        its cache holding the rows (h_p, tok_{p+1}), p < T-1). The steps of 3 rows replay
-        one captured graph."""
+        its cache holding the rows (h_p, tok_{p+1}), p < T-1)."""
         with_head = (self.mtp is not None) if with_head is None else with_head
         prompt = torch.as_tensor(tokens, dtype=torch.int32).to(self.device)
         T = int(prompt.numel())
@@ -628,6 +679,10 @@ class NemotronModel:
             # the last 3-row step writes attention rows up to 3 * nsteps - 1
             raise N.HSDError(f"a {T}-token prompt needs {3 * nsteps} attention cache rows (3-row prefill steps); "
                              f"max_seq is {self.cfg.max_seq}")
+        if T > 3 and self._chunkable():
+            for r in range(0, T, CHUNK_ROWS):
+                x = self._prefill_chunk(prompt, T, min(CHUNK_ROWS, T - r), cache, with_head)
+            return x[-1:]
         if graph and nsteps > 2:
             g = self._capture(lambda: self._prefill_step(prompt, T, cache, with_head))
             for _ in range(nsteps):

@@ -1,0 +1,134 @@
+"""GPU: the mixers of a prompt chunk (hsd.chunk.scan, hsd.chunk.attention) and the chunked
+prompt against the decode kernels' row-by-row runs.
+
+* scan: bit-identical to mamba.ssm_rows in steps of up to 3 rows (the same arithmetic per row):
+  z, the 16-channel sums, the state and the conv window;
+* attention: the cache rows bit-exact, the outputs against float64 attention. The kernel sums
+  exact bf16 products in fp32, keeps 16 bits of each probability and rounds once to bf16:
+  half a bf16 ulp (2^-9) plus 2^-16 of the values' scale, doubled for the fp32 exponentials;
+* prefill: both modes equal bits, and the caches near a run in 3-row steps. Two correct runs
+  differ by bf16 roundings (a few 1e-3 after these layers) and, where a token's sixth and
+  seventh experts are nearly tied, by one of six gains of that block's update of that row:
+  with updates of at most the residual's size, sqrt(2)/6 of a row, which over T >= 4 rows
+  and the blocks after it stays below 0.12/sqrt(T) + 2e-2 for one such token in four."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from hsd import _native as N
+from hsd import chunk, mamba as M, nn
+from hsd import model as Mdl
+
+pytestmark = pytest.mark.gpu
+
+
+def gen(dev, seed):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    return g
+
+
+def mixer_and_state(dev, seed):
+    blk = Mdl.MambaBlock(Mdl.ModelConfig(hidden=512, mtp=False), Mdl._Init(seed, dev))
+    g = gen(dev, seed)
+    m = blk.mixer
+    conv = torch.randn((3, m.conv_dim), device=dev, generator=g).to(torch.bfloat16)
+    ssm = torch.randn((m.num_heads, m.head_dim, m.ssm_state_size), device=dev, generator=g) * 0.1
+    return m, conv, ssm, g
+
+
+@pytest.mark.parametrize("T,cur0,pos0,total", [(1, 0, 0, 1), (2, 3, 0, 2), (15, 1, 0, 15), (16, 0, 0, 16), (17, 2, 0, 17),
+                                               (33, 0, 5, 30), (40, 1, 9, 9)])
+def test_scan_equals_rows(dev, T, cur0, pos0, total):
+    m, conv, ssm, g = mixer_and_state(dev, T)
+    width = 2 * m.intermediate_size + 2 * m.n_groups * m.ssm_state_size + m.num_heads
+    proj = torch.randn((T, width), device=dev, generator=g).to(torch.bfloat16)
+    cur = torch.full((1,), cur0, dtype=torch.int32, device=dev)
+    pos = torch.full((1,), pos0, dtype=torch.int32, device=dev)
+    ca = M.MambaCache(m, dev, nslab=4, cur=cur, conv_state=conv, ssm_state=ssm)
+    cb = M.MambaCache(m, dev, nslab=4, cur=cur.clone(), conv_state=conv, ssm_state=ssm)
+    z = chunk.scan(m, proj, ca, pos, total)
+    V = min(max(total - pos0, 0), T)
+    DI = m.intermediate_size
+    for r in range(0, V, 3):
+        n = min(3, V - r)
+        zr = M.ssm_rows(m, proj[r:r + n], cb, gated=True)
+        full = torch.as_strided(zr, (n, DI + DI // 16), (DI + DI // 16, 1))
+        got = torch.as_strided(z, (T, DI + DI // 16), (DI + DI // 16, 1))[r:r + n]
+        assert torch.equal(got.view(torch.int32), full.view(torch.int32)), r
+        N.call("hsd_mamba_select_row", N.ptr(cb.cur), None, n, n, 4, None, N.stream(dev))
+    d = (cur0 + V) % 4
+    assert int(cb.cur.item()) == d and int(ca.cur.item()) == cur0
+    assert torch.equal(ca.ssm[d].view(torch.int32), cb.ssm[d].view(torch.int32))
+    assert torch.equal(ca.conv[d].view(torch.int16), cb.conv[d].view(torch.int16))
+
+
+@pytest.mark.parametrize("T,pos0,total", [(1, 0, 1), (31, 0, 31), (33, 0, 33), (65, 0, 65), (130, 7, 137), (70, 100, 160)])
+def test_attention(dev, T, pos0, total):
+    HQ, HKV, HD, smax = 8, 2, 128, 192
+    g = gen(dev, T)
+    qkv = torch.randn((T, (HQ + 2 * HKV) * HD), device=dev, generator=g).to(torch.bfloat16)
+    kv = nn.KVCache(HKV, smax, dev, HD)
+    for t in (kv.k, kv.v):
+        t[:, :pos0] = torch.randn((HKV, pos0, HD), device=dev, generator=g).to(torch.bfloat16)
+    kv.v[:, total:] = float("nan")           # never read
+    pos = torch.full((1,), pos0, dtype=torch.int32, device=dev)
+    o = chunk.attention(qkv, kv, pos, total, n_heads=HQ, n_kv_heads=HKV, head_dim=HD)
+    V = min(total - pos0, T)
+    k, v = (qkv[:V, (HQ + i * HKV) * HD:(HQ + (i + 1) * HKV) * HD].view(V, HKV, HD).transpose(0, 1) for i in (0, 1))
+    assert torch.equal(kv.k[:, pos0:pos0 + V].view(torch.int16), k.contiguous().view(torch.int16))
+    assert torch.equal(kv.v[:, pos0:pos0 + V].view(torch.int16), v.contiguous().view(torch.int16))
+    assert bool(torch.isnan(kv.v[:, total:].float()).all())
+    q = qkv[:V, :HQ * HD].view(V, HQ, HD).double().cpu()
+    kd, vd = kv.k.double().cpu(), kv.v.double().cpu()
+    for r in (0, V // 2, V - 1):
+        n = pos0 + r + 1
+        for h in range(HQ):
+            s = (kd[h // (HQ // HKV), :n] @ q[r, h]) / math.sqrt(HD)
+            ref = torch.softmax(s, 0) @ vd[h // (HQ // HKV), :n]
+            got = o[r, h * HD:(h + 1) * HD].double().cpu()
+            assert float(((got - ref).abs() - 2.0 ** -8 * ref.abs()).max()) <= 2.0 ** -15 * 8, (r, h)
+
+
+def test_attention_refuses_overflow(dev):
+    HQ, HKV, HD, smax = 8, 2, 128, 64
+    qkv = torch.ones((40, (HQ + 2 * HKV) * HD), dtype=torch.bfloat16, device=dev)
+    kv = nn.KVCache(HKV, smax, dev, HD)
+    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    pos = torch.full((1,), 30, dtype=torch.int32, device=dev)
+    o = chunk.attention(qkv, kv, pos, 70, n_heads=HQ, n_kv_heads=HKV, head_dim=HD, status=status)
+    assert int(status.item()) == N.STATUS_BAD_STATE
+    assert float(kv.k.float().abs().max()) == 0 and float(o.float().abs().max()) == 0
+
+
+CFG = Mdl.ModelConfig(hidden=512, pattern="MEM*EME", vocab=4096, n_experts=16, topk=6, moe_inter=256, shared_inter=512,
+                      max_seq=256, mtp=True)
+
+
+@pytest.mark.parametrize("T", [4, 33, 70])
+def test_chunked_prefill(dev, T):
+    m = Mdl.NemotronModel(CFG, seed=5, device=dev, calibrate=False)
+    prompt = np.random.default_rng(T).integers(0, CFG.vocab, T).astype(np.int32)
+    caches, xs = [], []
+    for mode, steps in (("sparse", False), ("dense", False), ("sparse", True)):
+        m.set_mode(mode)
+        m._chunkable = (lambda: False) if steps else (lambda: True)
+        c = m.make_cache(cap=8)
+        xs.append(m.prefill(prompt, c, graph=False).clone())
+        assert int(c.status.item()) == 0
+        caches.append(c)
+    a, b, s = caches
+    assert torch.equal(xs[0].view(torch.int16), xs[1].view(torch.int16))
+    assert torch.equal(a.seq, b.seq) and torch.equal(a.seq, s.seq)
+    assert a.state()[N.SEQ_POS] == T and a.state()[N.SEQ_HEAD_POS] == T - 1
+    cur = int(a.cur.item())
+    tensors = lambda c: [t for lc in c.layers if lc is not None for t in                          # noqa: E731
+                         ((lc.ssm[cur], lc.conv[cur]) if hasattr(lc, "ssm") else (lc.k[:, :T], lc.v[:, :T]))] + \
+        [c.head_kv.k[:, :T - 1], c.head_kv.v[:, :T - 1]]
+    for u, v, w in zip(tensors(a), tensors(b), tensors(s)):
+        assert torch.equal(u, v)
+        u, w = u.double(), w.double()
+        assert float((u - w).norm() / w.norm()) < 0.12 / math.sqrt(T) + 2e-2
+    assert float((xs[0].double() - xs[2].double()).norm() / xs[2].double().norm()) < 0.24 + 2e-2   # one row
