@@ -99,12 +99,14 @@ __global__ __launch_bounds__(256) void k_conv_rows(const uint16_t* __restrict__ 
 // Bound by the vector unit's issue (about 30 instructions per row and wavefront, one
 // wavefront per SIMD): rows are a serial chain of one fma.
 constexpr int kTS = 16;
-__global__ __launch_bounds__(256) void k_scan(
+__global__ __launch_bounds__(256, 1) void k_scan(
     const float* __restrict__ co, const float* __restrict__ dtA, const uint16_t* __restrict__ cin, int64_t cin_ld,
     const uint16_t* __restrict__ gate, int64_t gate_ld, const float* __restrict__ Dp, float* __restrict__ ssm,
     uint16_t* __restrict__ convs, const int32_t* __restrict__ cur_ptr, const int32_t* __restrict__ pos, int nslab,
     float* __restrict__ z, int64_t z_ld, int T, int Ttot, int H, int P, int G, int32_t* __restrict__ status) {
-  __shared__ __attribute__((aligned(16))) float Bs[2][kTS][kN], Cs[2][kTS][kN];
+  // a lane's 8 B (C) elements as two float4, the 16 lanes' first ones, then their second
+  // ones: consecutive lanes read consecutive 16 bytes (no bank conflicts)
+  __shared__ __attribute__((aligned(16))) f32x4 Bs[2][kTS][2][kN / 8], Cs[2][kTS][2][kN / 8];
   __shared__ __attribute__((aligned(16))) float xs[2][kTS][kPB];
   __shared__ float ds[2][kTS][2];
   __shared__ float ys[kTS][kPB + 1];
@@ -174,7 +176,7 @@ __global__ __launch_bounds__(256) void k_scan(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int idx = tid + 256 * i, r = idx >> 6, q = idx & 63;
-      *reinterpret_cast<f32x4*>(q < 32 ? &Bs[b][r][4 * q] : &Cs[b][r][4 * (q - 32)]) = rb[i];
+      (q < 32 ? Bs[b][r][q & 1] : Cs[b][r][q & 1])[(q & 31) >> 1] = rb[i];
     }
     if (tid < 64) *reinterpret_cast<f32x4*>(&xs[b][tid >> 2][4 * (tid & 3)]) = rx;
     if (tid < 32) ds[b][tid >> 1][tid & 1] = rd;
@@ -187,13 +189,24 @@ __global__ __launch_bounds__(256) void k_scan(
     __syncthreads();                               // stage b in LDS, ys read
     load(t0 + kTS);                                // past the chunk: its last row again, unused
     const int n = min(kTS, T - t0);
-    auto row = [&](int r) {
-      const float4 B0 = *reinterpret_cast<const float4*>(&Bs[b][r][8 * c8]);
-      const float4 B1 = *reinterpret_cast<const float4*>(&Bs[b][r][8 * c8 + 4]);
-      const float4 C0 = *reinterpret_cast<const float4*>(&Cs[b][r][8 * c8]);
-      const float4 C1 = *reinterpret_cast<const float4*>(&Cs[b][r][8 * c8 + 4]);
-      const float x = xs[b][r][pl];
-      const float xdt = x * ds[b][r][0], a = ds[b][r][1];
+    // a row's inputs; the next kPF rows' are read while kPF rows are computed (one wavefront
+    // per SIMD: nothing else hides the LDS latency)
+    struct In {
+      f32x4 B0, B1, C0, C1;
+      float x, dt, a;
+    };
+    auto fetch = [&](In& v, int r) {
+      v.B0 = Bs[b][r][0][c8];
+      v.B1 = Bs[b][r][1][c8];
+      v.C0 = Cs[b][r][0][c8];
+      v.C1 = Cs[b][r][1][c8];
+      v.x = xs[b][r][pl];
+      v.dt = ds[b][r][0];
+      v.a = ds[b][r][1];
+    };
+    auto row = [&](const In& v, int r) {
+      const f32x4 B0 = v.B0, B1 = v.B1, C0 = v.C0, C1 = v.C1;
+      const float x = v.x, xdt = x * v.dt, a = v.a;
       S0.x = fmaf(a, S0.x, xdt * B0.x);
       S0.y = fmaf(a, S0.y, xdt * B0.y);
       S0.z = fmaf(a, S0.z, xdt * B0.z);
@@ -222,12 +235,25 @@ __global__ __launch_bounds__(256) void k_scan(
       *reinterpret_cast<float4*>(dst + 4) = S1;
     };
     if (n == kTS && (V - 1 < t0 || V - 1 >= t0 + kTS - 1)) {
-#pragma unroll 4
-      for (int r = 0; r < kTS; ++r) row(r);
+      constexpr int kPF = 4;
+      In in[2][kPF];
+#pragma unroll
+      for (int u = 0; u < kPF; ++u) fetch(in[0][u], u);
+#pragma unroll
+      for (int r0 = 0; r0 < kTS; r0 += kPF) {
+#pragma unroll
+        for (int u = 0; u < kPF; ++u)
+          if (r0 + kPF < kTS) fetch(in[(r0 / kPF + 1) & 1][u], r0 + kPF + u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < kPF; ++u) row(in[(r0 / kPF) & 1][u], r0 + u);
+      }
       if (V - 1 == t0 + kTS - 1) save();
     } else {
       for (int r = 0; r < n; ++r) {
-        row(r);
+        In v;
+        fetch(v, r);
+        row(v, r);
         if (t0 + r == V - 1) save();
       }
     }
