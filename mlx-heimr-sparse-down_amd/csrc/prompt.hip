@@ -189,6 +189,7 @@ __global__ __launch_bounds__(256, 1) void k_scan(
     __syncthreads();                               // stage b in LDS, ys read
     load(t0 + kTS);                                // past the chunk: its last row again, unused
     const int n = min(kTS, T - t0);
+    float yk = 0.0f;
     // a row's inputs; the next kPF rows' are read while kPF rows are computed (one wavefront
     // per SIMD: nothing else hides the LDS latency)
     struct In {
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(256, 1) void k_scan(
     };
     auto row = [&](const In& v, int r) {
       const f32x4 B0 = v.B0, B1 = v.B1, C0 = v.C0, C1 = v.C1;
-      const float x = v.x, xdt = x * v.dt, a = v.a;
+      const float xdt = v.x * v.dt, a = v.a;
       S0.x = fmaf(a, S0.x, xdt * B0.x);
       S0.y = fmaf(a, S0.y, xdt * B0.y);
       S0.z = fmaf(a, S0.z, xdt * B0.z);
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256, 1) void k_scan(
       y += dpp_f32<0x4E>(y);
       y += dpp_f32<0x141>(y);
       y += dpp_f32<0x140>(y);
-      if (c8 == 0) ys[r][pl] = y + x * Dh;
+      yk = c8 == r ? y : yk;                       // lane c8 keeps row c8's (a select, no branch per row)
     };
     auto save = [&]() {
       float* dst = ssm + (size_t)dst_slab * slab + soff;
@@ -257,6 +258,7 @@ __global__ __launch_bounds__(256, 1) void k_scan(
         if (t0 + r == V - 1) save();
       }
     }
+    ys[c8][pl] = yk + xs[b][c8][pl] * Dh;
     __syncthreads();                               // ys complete
     {
       const int r = tid >> 4, c = tid & 15;
