@@ -1,4 +1,5 @@
-"""ctypes binding of libhsd.so (the gfx950 HIP kernels behind a C ABI).
+"""Binding of libhsd.so (the gfx950 HIP kernels behind a C ABI): the library loaded with
+ctypes, its entry points called through the native module _hsdcall (csrc/pycall.cpp).
 
 The library is built in-tree (`make` in the package root, or `__graft_entry__.build()`)
 and loaded from next to this package. There is no fallback: if the library is missing
@@ -44,6 +45,7 @@ def capture_guard():
             gc.enable()
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
 _c_int, _c_i64, _c_size, _c_float, _vp = ctypes.c_int, ctypes.c_int64, ctypes.c_size_t, ctypes.c_float, ctypes.c_void_p
 
 # name -> (restype, [argtypes]); every pointer is passed as void*.
@@ -147,12 +149,34 @@ def lib():
     return _lib
 
 
+_entries = None
+
+
+def _bind():
+    """The entry points as native functions (bound once to the loaded library's addresses)."""
+    global _entries
+    L = lib()
+    try:
+        from . import _hsdcall
+    except ImportError as e:
+        raise HSDError("hsd/_hsdcall.so is not built or does not load (make -C mlx-heimr-sparse-down_amd all, or "
+                       f"__graft_entry__.build()): {e}") from e
+    addr = lambda n: ctypes.cast(getattr(L, n), _vp).value  # noqa: E731
+    names = [n for n in _SIGS if hasattr(_hsdcall, n)]
+    _hsdcall.bind(HSDError, addr("hsd_last_error"), {n: addr(n) for n in names})
+    _entries = {n: getattr(_hsdcall, n) for n in names}
+    return _entries
+
+
+def entry(name):
+    """The entry point as a native function: its pointer arguments take None, device tensors,
+    ints or ctypes pointers; it raises HSDError with hsd_last_error() on a negative status."""
+    return (_entries or _bind())[name]
+
+
 def call(name, *args):
-    """Call an entry point; raise HSDError with hsd_last_error() on a negative status."""
-    rc = getattr(lib(), name)(*args)
-    if rc != 0:
-        raise HSDError(f"{name} -> {rc}: {lib().hsd_last_error().decode(errors='replace')}")
-    return rc
+    """Call an entry point (see entry)."""
+    return (_entries or _bind())[name](*args)
 
 
 def ptr(t):
@@ -166,7 +190,8 @@ def ptr(t):
 
 def stream(device=None):
     """The current torch stream of `device` as a hipStream_t."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = None if device is None else device.index if isinstance(device, torch.device) else torch.device(device).index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 _DT = {torch.bfloat16: DT_BF16, torch.float16: DT_F16, torch.float32: DT_F32}

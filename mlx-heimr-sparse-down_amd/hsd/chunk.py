@@ -38,7 +38,7 @@ def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
     kind = N.X_GATED_Z if gated_z else N.X_RMS if norm is not None else N.X_BF16
     xp = torch.empty((T, I), dtype=torch.bfloat16, device=x.device)
     hs = torch.empty((T, 2 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
-    N.call("hsd_rows_prep", N.ptr(x), x.stride(0), kind, N.ptr(norm), float(eps), N.ptr(xp), N.ptr(hs), T, I,
+    N.call("hsd_rows_prep", x, x.stride(0), kind, norm, float(eps), xp, hs, T, I,
            N.stream(x.device))
     return Rows(xp, hs)
 
@@ -50,10 +50,10 @@ def gemm(rows: Rows, W, residual=None, out=None):
     y = out if out is not None else torch.empty((T, W.O), dtype=torch.bfloat16, device=rows.xp.device)
     st = N.stream(rows.xp.device)
     if W.q4:
-        N.call("hsd_gemm_q4", N.ptr(rows.xp), N.ptr(rows.hs), N.ptr(W.w), N.ptr(W.scales), N.ptr(W.biases), N.ptr(y),
-               y.stride(0), N.ptr(residual), 0 if residual is None else residual.stride(0), T, W.O, W.I, st)
+        N.call("hsd_gemm_q4", rows.xp, rows.hs, W.w, W.scales, W.biases, y,
+               y.stride(0), residual, 0 if residual is None else residual.stride(0), T, W.O, W.I, st)
     else:
-        N.call("hsd_gemm_bf16", N.ptr(rows.xp), rows.xp.stride(0), 0 if rows.hs is None else 1, N.ptr(W.w), N.ptr(y),
+        N.call("hsd_gemm_bf16", rows.xp, rows.xp.stride(0), 0 if rows.hs is None else 1, W.w, y,
                y.stride(0), T, W.O, W.I, st)
     return y
 
@@ -64,7 +64,7 @@ def moe_tiles(sel, E, tt, status=None):
     NT = num_tiles(T, K, E, tt)
     t = torch.empty(NT * (tt + 1) + 1, dtype=torch.int32, device=sel.device)
     tile_e, tile_slot, ntiles = t[:NT], t[NT:NT * (tt + 1)], t[NT * (tt + 1):]
-    N.call("hsd_moe_tiles", N.ptr(sel), T, K, E, tt, N.ptr(tile_e), N.ptr(tile_slot), N.ptr(ntiles), N.ptr(status),
+    N.call("hsd_moe_tiles", sel, T, K, E, tt, tile_e, tile_slot, ntiles, status,
            N.stream(sel.device))
     return tile_e, tile_slot, ntiles
 
@@ -75,9 +75,9 @@ def moe_up(rows: Rows, tiles, w1, s1, b1, sw1, ss1, sb1, *, topk, tt):
     E, F, FS = w1.shape[0], w1.shape[1], sw1.shape[0]
     hcat = torch.empty((T, topk * F + FS), dtype=torch.bfloat16, device=rows.xp.device)
     hsum = torch.empty((T, topk + 1, 2 * group_pitch(max(F, FS))), dtype=torch.bfloat16, device=rows.xp.device)
-    N.call("hsd_moe_up_gemm", N.ptr(rows.xp), N.ptr(rows.hs), N.ptr(tiles[0]), N.ptr(tiles[1]), N.ptr(tiles[2]),
-           N.ptr(N.as_words(w1)), N.ptr(s1), N.ptr(b1), N.ptr(N.as_words(sw1)), N.ptr(ss1), N.ptr(sb1), N.ptr(hcat),
-           N.ptr(hsum), T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
+    N.call("hsd_moe_up_gemm", rows.xp, rows.hs, tiles[0], tiles[1], tiles[2],
+           N.as_words(w1), s1, b1, N.as_words(sw1), ss1, sb1, hcat,
+           hsum, T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
     return hcat, hsum
 
 
@@ -87,11 +87,11 @@ def moe_down(x, hcat, hsum, sel, gains, tiles, pw, ps, pb, spw, sps, spb, *, top
     T, D = x.shape
     E, F, FS = pw.shape[0], pw.shape[1], spw.shape[0]
     y = out if out is not None else torch.empty((T, D), dtype=torch.bfloat16, device=x.device)
-    nb = N.lib().hsd_moe_down_workspace_bytes(T, D, topk)
+    nb = N.call("hsd_moe_down_workspace_bytes", T, D, topk)
     ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
-    N.call("hsd_moe_down_gemm", N.ptr(hcat), N.ptr(hsum), N.ptr(sel), N.ptr(gains), N.ptr(tiles[0]), N.ptr(tiles[1]),
-           N.ptr(tiles[2]), N.ptr(N.as_words(pw)), N.ptr(ps), N.ptr(pb), N.ptr(N.as_words(spw)), N.ptr(sps), N.ptr(spb),
-           N.ptr(x), x.stride(0), N.ptr(y), y.stride(0), T, D, F, FS, topk, E, tt, N.ptr(ws), nb, N.stream(x.device))
+    N.call("hsd_moe_down_gemm", hcat, hsum, sel, gains, tiles[0], tiles[1],
+           tiles[2], N.as_words(pw), ps, pb, N.as_words(spw), sps, spb,
+           x, x.stride(0), y, y.stride(0), T, D, F, FS, topk, E, tt, ws, nb, N.stream(x.device))
     return y
 
 
@@ -103,15 +103,15 @@ def scan(mixer, proj, cache, pos, total, status=None):
     H, P, Nst, G = mixer.num_heads, mixer.head_dim, mixer.ssm_state_size, mixer.n_groups
     DI, CD = mixer.intermediate_size, mixer.conv_dim
     z = torch.empty((T, DI + DI // 16), dtype=torch.float32, device=proj.device)
-    nb = N.lib().hsd_mamba_scan_workspace_bytes(T, H, P, Nst, G)
+    nb = N.call("hsd_mamba_scan_workspace_bytes", T, H, P, Nst, G)
     ws = torch.empty(nb, dtype=torch.uint8, device=proj.device)
     base, es, ld = proj.data_ptr(), proj.element_size(), proj.stride(0)
     lo, hi = mixer.time_step_limit
-    N.call("hsd_mamba_scan", ctypes.c_void_p(base + DI * es), ld, ctypes.c_void_p(base + (DI + CD) * es), ld, N.ptr(proj),
-           ld, N.ptr(N.contig(mixer.conv_w)), N.ptr(N.contig(mixer.conv_b)), N.ptr(N.contig(mixer.A_log)),
-           N.ptr(N.contig(mixer.dt_bias)), N.ptr(N.contig(mixer.D)), N.ptr(cache.ssm), N.ptr(cache.conv),
-           N.ptr(cache.cur), cache.nslab, N.ptr(pos), N.ptr(z), z.stride(0), T, total, H, P, Nst, G, float(lo), float(hi),
-           N.ptr(status), N.ptr(ws), nb, N.stream(proj.device))
+    N.call("hsd_mamba_scan", ctypes.c_void_p(base + DI * es), ld, ctypes.c_void_p(base + (DI + CD) * es), ld, proj,
+           ld, N.contig(mixer.conv_w), N.contig(mixer.conv_b), N.contig(mixer.A_log),
+           N.contig(mixer.dt_bias), N.contig(mixer.D), cache.ssm, cache.conv,
+           cache.cur, cache.nslab, pos, z, z.stride(0), T, total, H, P, Nst, G, float(lo), float(hi),
+           status, ws, nb, N.stream(proj.device))
     return z[:, :DI]
 
 
@@ -120,7 +120,7 @@ def attention(qkv, kv, pos, total, *, n_heads, n_kv_heads, head_dim=128, cache_o
     -> [T, HQ*HD] bf16 (None with cache_only)."""
     T = qkv.shape[0]
     out = None if cache_only else torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
-    N.call("hsd_attn_prompt", N.ptr(qkv), qkv.stride(0), T, total, N.ptr(kv.k), N.ptr(kv.v), kv.smax, N.ptr(pos),
-           N.ptr(out), 0 if out is None else out.stride(0), n_heads, n_kv_heads, head_dim, 1.0 / math.sqrt(head_dim),
-           N.ptr(status), N.stream(qkv.device))
+    N.call("hsd_attn_prompt", qkv, qkv.stride(0), T, total, kv.k, kv.v, kv.smax, pos,
+           out, 0 if out is None else out.stride(0), n_heads, n_kv_heads, head_dim, 1.0 / math.sqrt(head_dim),
+           status, N.stream(qkv.device))
     return out

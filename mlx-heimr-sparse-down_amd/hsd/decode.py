@@ -55,16 +55,15 @@ def sparse_down(h, sel, gains, pw, ps, pb, spw, sps, spb, *, F, FS, D, topk,
     E = pw.shape[0]
     od = out_dtype or h.dtype
     y = torch.empty((B, D), dtype=od, device=h.device)
-    nbytes = N.lib().hsd_sparse_down_workspace_bytes(B, D, F, FS, topk)
-    ws = _workspace(nbytes, h.device, workspace)
+    ws = _workspace(N.call("hsd_sparse_down_workspace_bytes", B, D, F, FS, topk), h.device, workspace)
     if live_masks is not None and (live_masks.dtype != torch.int64 or not live_masks.is_contiguous()
                                    or live_masks.numel() < B * (topk * F // 64 + FS // 64)):
         raise N.HSDError("live_masks must be a contiguous int64 tensor of B*(topk*F/64 + FS/64) entries")
-    N.call("hsd_sparse_down_decode", N.ptr(h), N.dtype_tag(h.dtype), N.ptr(sel), N.ptr(gains),
-           N.ptr(N.as_words(N.contig(pw))), N.ptr(N.contig(ps)), N.ptr(N.contig(pb)),
-           N.ptr(N.as_words(N.contig(spw))), N.ptr(N.contig(sps)), N.ptr(N.contig(spb)),
-           N.ptr(y), N.dtype_tag(od), B, D, F, FS, topk, E, 1 if dense else 0,
-           N.ptr(live_masks), N.ptr(status), N.ptr(ws), ws.numel(), N.stream(h.device))
+    N.call("hsd_sparse_down_decode", h, N.dtype_tag(h.dtype), sel, gains,
+           N.as_words(N.contig(pw)), N.contig(ps), N.contig(pb),
+           N.as_words(N.contig(spw)), N.contig(sps), N.contig(spb),
+           y, N.dtype_tag(od), B, D, F, FS, topk, E, 1 if dense else 0,
+           live_masks, status, ws, ws.numel(), N.stream(h.device))
     return y
 
 
@@ -79,8 +78,8 @@ def dense_down(h, sel, gains, w, s, b, sw, ss, sb, *, F, FS, D, topk, out_dtype=
     gains = N.contig(gains.to(torch.float32))
     od = out_dtype or h.dtype
     y = torch.empty((B, D), dtype=od, device=h.device)
-    N.call("hsd_dense_down_decode", N.ptr(h), N.dtype_tag(h.dtype), N.ptr(sel), N.ptr(gains),
-           N.ptr(N.as_words(N.contig(w))), N.ptr(N.contig(s)), N.ptr(N.contig(b)),
-           N.ptr(N.as_words(N.contig(sw))), N.ptr(N.contig(ss)), N.ptr(N.contig(sb)),
-           N.ptr(y), N.dtype_tag(od), B, D, F, FS, topk, w.shape[0], N.ptr(status), N.stream(h.device))
+    N.call("hsd_dense_down_decode", h, N.dtype_tag(h.dtype), sel, gains,
+           N.as_words(N.contig(w)), N.contig(s), N.contig(b),
+           N.as_words(N.contig(sw)), N.contig(ss), N.contig(sb),
+           y, N.dtype_tag(od), B, D, F, FS, topk, w.shape[0], status, N.stream(h.device))
     return y

@@ -35,7 +35,7 @@ def nibble_transpose(w: torch.Tensor) -> torch.Tensor:
     batch = 1
     for d in lead:
         batch *= d
-    N.call("hsd_permute_nibbles", N.ptr(words), N.ptr(out), batch, R, CW, N.stream(w.device))
+    N.call("hsd_permute_nibbles", words, out, batch, R, CW, N.stream(w.device))
     return out.view(w.dtype) if w.dtype != torch.int32 else out
 
 
@@ -48,7 +48,7 @@ def transpose_last2(x: torch.Tensor) -> torch.Tensor:
     batch = 1
     for d in lead:
         batch *= d
-    N.call("hsd_transpose_u16", N.ptr(x), N.ptr(out), batch, R, C, N.stream(x.device))
+    N.call("hsd_transpose_u16", x, out, batch, R, C, N.stream(x.device))
     return out
 
 

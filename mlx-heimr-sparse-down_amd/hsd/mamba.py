@@ -93,7 +93,7 @@ def verify_rows(mixer: Mamba2Mixer, proj, cache: MambaCache, out_dtype=torch.bfl
     if ld != DI + CD + H:
         raise N.HSDError(f"proj has {ld} columns, expected {DI + CD + H}")
     y = torch.empty((L, DI), dtype=out_dtype, device=proj.device)
-    ws = _workspace(N.lib().hsd_mamba_workspace_bytes(L, H, P), proj.device, workspace)
+    ws = _workspace(N.call("hsd_mamba_workspace_bytes", L, H, P), proj.device, workspace)
     base = proj.data_ptr()
     es = proj.element_size()
     import ctypes
@@ -102,11 +102,11 @@ def verify_rows(mixer: Mamba2Mixer, proj, cache: MambaCache, out_dtype=torch.bfl
     dt_p = ctypes.c_void_p(base + (DI + CD) * es)
     lo, hi = mixer.time_step_limit
     N.call("hsd_mamba_verify", conv_p, ld, dt_p, ld, gate_p, ld,
-           N.ptr(N.contig(mixer.conv_w)), N.ptr(N.contig(mixer.conv_b)), N.ptr(N.contig(mixer.A_log)),
-           N.ptr(N.contig(mixer.dt_bias)), N.ptr(N.contig(mixer.D)), N.ptr(N.contig(mixer.norm_w)),
-           N.ptr(cache.ssm), N.ptr(cache.conv), N.ptr(cache.cur), cache.nslab, N.ptr(y),
+           N.contig(mixer.conv_w), N.contig(mixer.conv_b), N.contig(mixer.A_log),
+           N.contig(mixer.dt_bias), N.contig(mixer.D), N.contig(mixer.norm_w),
+           cache.ssm, cache.conv, cache.cur, cache.nslab, y,
            N.dtype_tag(out_dtype), L, H, P, Nst, G, mixer.norm_group, float(mixer.eps), float(lo),
-           float(hi), N.ptr(status), N.ptr(ws), ws.numel(), N.stream(proj.device))
+           float(hi), status, ws, ws.numel(), N.stream(proj.device))
     return y
 
 
@@ -136,17 +136,17 @@ def ssm_rows(mixer: Mamba2Mixer, proj, cache: MambaCache, out=None, status=None,
             out = torch.empty((L, zw), dtype=torch.float32, device=proj.device)
         if out.dtype != torch.float32 or out.shape[0] < L or out.stride(1) != 1 or out.stride(0) < zw:
             raise N.HSDError(f"ssm_rows(gated=True) needs f32 rows of at least {zw} values")
-        N.call("hsd_mamba_ssm_gated", conv_p, proj.stride(0), dt_p, proj.stride(0), N.ptr(proj), proj.stride(0),
-               N.ptr(N.contig(mixer.conv_w)), N.ptr(N.contig(mixer.conv_b)), N.ptr(N.contig(mixer.A_log)),
-               N.ptr(N.contig(mixer.dt_bias)), N.ptr(N.contig(mixer.D)), N.ptr(cache.ssm), N.ptr(cache.conv),
-               N.ptr(cache.cur), cache.nslab, N.ptr(out), out.stride(0), L, H, P, Nst, G, float(lo), float(hi),
-               N.ptr(status), N.stream(proj.device))
+        N.call("hsd_mamba_ssm_gated", conv_p, proj.stride(0), dt_p, proj.stride(0), proj, proj.stride(0),
+               N.contig(mixer.conv_w), N.contig(mixer.conv_b), N.contig(mixer.A_log),
+               N.contig(mixer.dt_bias), N.contig(mixer.D), cache.ssm, cache.conv,
+               cache.cur, cache.nslab, out, out.stride(0), L, H, P, Nst, G, float(lo), float(hi),
+               status, N.stream(proj.device))
         return out[:L, :DI]
     y = out if out is not None else torch.empty((L, DI), dtype=torch.float32, device=proj.device)
-    N.call("hsd_mamba_ssm", conv_p, proj.stride(0), dt_p, proj.stride(0), N.ptr(N.contig(mixer.conv_w)),
-           N.ptr(N.contig(mixer.conv_b)), N.ptr(N.contig(mixer.A_log)), N.ptr(N.contig(mixer.dt_bias)),
-           N.ptr(N.contig(mixer.D)), N.ptr(cache.ssm), N.ptr(cache.conv), N.ptr(cache.cur), cache.nslab, N.ptr(y), L,
-           H, P, Nst, G, float(lo), float(hi), N.ptr(status), N.stream(proj.device))
+    N.call("hsd_mamba_ssm", conv_p, proj.stride(0), dt_p, proj.stride(0), N.contig(mixer.conv_w),
+           N.contig(mixer.conv_b), N.contig(mixer.A_log), N.contig(mixer.dt_bias),
+           N.contig(mixer.D), cache.ssm, cache.conv, cache.cur, cache.nslab, y, L,
+           H, P, Nst, G, float(lo), float(hi), status, N.stream(proj.device))
     return y
 
 
@@ -168,8 +168,11 @@ def mamba_verify(block, x3, cache, records):
         buf = dict(proj=torch.empty((L, block.in_proj.O), dtype=torch.bfloat16, device=x.device),
                    y_pre=torch.empty((L, m.intermediate_size + m.intermediate_size // 16), dtype=torch.float32,
                                      device=x.device))
-        out = x.clone()
-        block.rows(out, buf, cache)
+        if hasattr(block, "rows_into") and x.data_ptr() % 16 == 0:
+            out = block.rows_into(x, buf, cache, torch.empty_like(x))
+        else:
+            out = x.clone()
+            block.rows(out, buf, cache)
         records.append((cache, L))
         return out[None]
     m = getattr(block, "mixer", block)
@@ -191,6 +194,6 @@ def mamba_rollback(records, n_keep, n_keep_dev=None, status=None):
         seen.add(id(cache.cur))
         if n_keep_dev is None and not 0 <= n_keep <= L:
             raise N.HSDError(f"n_keep {n_keep} outside [0, {L}]")
-        N.call("hsd_mamba_select_row", N.ptr(cache.cur), N.ptr(n_keep_dev),
-               0 if n_keep_dev is not None else int(n_keep), L, cache.nslab, N.ptr(status),
+        N.call("hsd_mamba_select_row", cache.cur, n_keep_dev,
+               0 if n_keep_dev is not None else int(n_keep), L, cache.nslab, status,
                N.stream(cache.cur.device))

@@ -143,13 +143,17 @@ class MambaBlock:
 
     def rows(self, x, buf, cache: M.MambaCache, status=None):
         """x [B, D] (updated in place). status: optional device int32 [1] (HSD_STATUS_*)."""
+        return self.rows_into(x, buf, cache, x, status=status)
+
+    def rows_into(self, x, buf, cache: M.MambaCache, out, status=None):
+        """rows with the result in out (16-byte aligned rows like x's; may be x)."""
         B = x.shape[0]
         proj = nn.linear(x, self.in_proj, norm=self.norm_w, eps=self.eps, out=buf["proj"][:B])
         # the gate applied in the SSM kernel, which also leaves each 16 channels' sum of z^2
         # for out_proj's gated norm (no silu, no gate loads in its prologue)
         z = M.ssm_rows(self.mixer, proj, cache, out=buf["y_pre"][:B], gated=True, status=status)
-        nn.linear(z, self.out_proj, norm=self.mixer.norm_w, eps=self.eps, gated_z=True, residual=x, out=x)
-        return x
+        nn.linear(z, self.out_proj, norm=self.mixer.norm_w, eps=self.eps, gated_z=True, residual=x, out=out)
+        return out
 
     def chunk(self, x, cache: M.MambaCache, pos, total, status=None):
         """x [T, D] (updated in place): a prompt chunk's rows."""
@@ -259,10 +263,10 @@ class MoEBlock:
         if self.trace is not None:                       # calibration / statistics only
             self.trace.append(float((hcat == 0).float().mean().item()))
         ws = buf["ws_down"]
-        N.call("hsd_sparse_down_residual", N.ptr(hcat), N.DT_BF16, N.ptr(sel), N.ptr(gains),
-               N.ptr(N.as_words(self.pw)), N.ptr(self.ps), N.ptr(self.pb), N.ptr(N.as_words(self.spw)),
-               N.ptr(self.sps), N.ptr(self.spb), N.ptr(x), N.ptr(x), B, c.hidden, c.moe_inter, c.shared_inter, c.topk,
-               c.n_experts, 1 if dense else 0, None, N.ptr(status), N.ptr(ws), ws.numel(), N.stream(x.device))
+        N.call("hsd_sparse_down_residual", hcat, N.DT_BF16, sel, gains,
+               N.as_words(self.pw), self.ps, self.pb, N.as_words(self.spw),
+               self.sps, self.spb, x, x, B, c.hidden, c.moe_inter, c.shared_inter, c.topk,
+               c.n_experts, 1 if dense else 0, None, status, ws, ws.numel(), N.stream(x.device))
         return x
 
     # ---- the reference's per-block call surface (model.py:110-175) on fresh buffers: any
@@ -295,13 +299,14 @@ class MoEBlock:
     def _down_residual(self, x, hcat, sel, gains, dense):
         c = self.cfg
         B = x.shape[0]
-        out = N.contig(x).clone()
-        nb = N.lib().hsd_sparse_down_workspace_bytes(B, c.hidden, c.moe_inter, c.shared_inter, c.topk)
+        x = N.contig(x)
+        out = torch.empty_like(x)
+        nb = N.call("hsd_sparse_down_workspace_bytes", B, c.hidden, c.moe_inter, c.shared_inter, c.topk)
         ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-        N.call("hsd_sparse_down_residual", N.ptr(hcat), N.DT_BF16, N.ptr(sel), N.ptr(gains),
-               N.ptr(N.as_words(self.pw)), N.ptr(self.ps), N.ptr(self.pb), N.ptr(N.as_words(self.spw)),
-               N.ptr(self.sps), N.ptr(self.spb), N.ptr(out), N.ptr(out), B, c.hidden, c.moe_inter, c.shared_inter,
-               c.topk, c.n_experts, 1 if dense else 0, None, None, N.ptr(ws), ws.numel(), N.stream(x.device))
+        N.call("hsd_sparse_down_residual", hcat, N.DT_BF16, sel, gains,
+               N.as_words(self.pw), self.ps, self.pb, N.as_words(self.spw),
+               self.sps, self.spb, x, out, B, c.hidden, c.moe_inter, c.shared_inter,
+               c.topk, c.n_experts, 1 if dense else 0, None, None, ws, ws.numel(), N.stream(x.device))
         return out
 
     def decode_sparse(self, x):
@@ -477,8 +482,8 @@ class NemotronModel:
     def _make_buffers(self, B):
         c, dev = self.cfg, self.device
         e = lambda *s, dt=torch.bfloat16: torch.zeros(s, dtype=dt, device=dev)
-        ws_down = N.lib().hsd_sparse_down_workspace_bytes(B, c.hidden, c.moe_inter, c.shared_inter, c.topk)
-        ws_attn = N.lib().hsd_attn_workspace_bytes(B, c.attn_heads, c.max_seq)
+        ws_down = N.call("hsd_sparse_down_workspace_bytes", B, c.hidden, c.moe_inter, c.shared_inter, c.topk)
+        ws_attn = N.call("hsd_attn_workspace_bytes", B, c.attn_heads, c.max_seq)
         return dict(x=e(B, c.hidden), xn=e(B, c.hidden), proj=e(B, c.in_proj_dim),
                     y_pre=e(B, c.mamba_inner + c.mamba_inner // 16, dt=torch.float32), qkv=e(B, c.qkv_dim),
                     att=e(B, c.attn_heads * c.head_dim), logits=e(B, c.n_experts),
@@ -611,7 +616,7 @@ class NemotronModel:
             nn.attention(qkv, kv, pos, n_heads=c.attn_heads, n_kv_heads=c.kv_heads, head_dim=c.head_dim,
                          out=comb[:, D:], workspace=buf["ws_attn"], status=status)
             one = b1["hcomb"]
-            N.call("hsd_seq_select_row", N.ptr(comb), comb.stride(0), N.ptr(seq), N.ptr(one), comb.shape[1],
+            N.call("hsd_seq_select_row", comb, comb.stride(0), seq, one, comb.shape[1],
                    N.stream(self.device))
             x1 = one[:, :D]
             nn.linear(one[:, D:], a.o_proj, residual=x1, out=x1)
@@ -637,7 +642,7 @@ class NemotronModel:
         """B rows from the cache's position on -> their residual stream [B, D]."""
         st, seq, c = N.stream(self.device), cache.seq, self.cfg
         ids = torch.empty(B, dtype=torch.int32, device=self.device)
-        N.call("hsd_prompt_tokens", N.ptr(prompt_dev), T, N.ptr(seq), 0, B, N.ptr(ids), st)
+        N.call("hsd_prompt_tokens", prompt_dev, T, seq, 0, B, ids, st)
         x = self.embed(ids, status=cache.status)
         for t, blk, lc in zip(c.pattern, self.blocks, cache.layers):
             if t == "E":
@@ -645,27 +650,27 @@ class NemotronModel:
             else:
                 blk.chunk(x, lc, cache.pos, T, status=cache.status)
         if with_head:
-            N.call("hsd_prompt_tokens", N.ptr(prompt_dev), T, N.ptr(seq), 1, B, N.ptr(ids), st)
+            N.call("hsd_prompt_tokens", prompt_dev, T, seq, 1, B, ids, st)
             hd = self.mtp
             pair = nn.head_input(ids, x, self.embedding, hd.enorm, hd.hnorm, eps=c.eps, status=cache.status)
             hx = chunk.gemm(chunk.prep(pair, sums=False), hd.eh_proj)
             hd.attn.chunk(hx, cache.head_kv, cache.head_pos, T - 1, status=cache.status)
             hd.moe.chunk(hx)
-        N.call("hsd_prompt_advance", N.ptr(seq), T, B, NSLAB, st)
+        N.call("hsd_prompt_advance", seq, T, B, NSLAB, st)
         return x
 
     def _prefill_step(self, prompt_dev, T, cache, with_head):
         buf = self._bufs[3]
         ids = buf["ids"][:3]
-        N.call("hsd_gather_tokens", N.ptr(prompt_dev), T, N.ptr(cache.seq), 0, 3, N.ptr(ids), N.stream(self.device))
+        N.call("hsd_gather_tokens", prompt_dev, T, cache.seq, 0, 3, ids, N.stream(self.device))
         x = self.embed(ids, out=buf["x"], status=cache.status)
         self.layers(x, buf, cache)
         if with_head:
             pend = buf["pend"][:3]
-            N.call("hsd_gather_tokens", N.ptr(prompt_dev), T, N.ptr(cache.seq), 1, 3, N.ptr(pend),
+            N.call("hsd_gather_tokens", prompt_dev, T, cache.seq, 1, 3, pend,
                    N.stream(self.device))
             self.mtp_rows(x, pend, buf, cache.head_kv, cache.head_pos, status=cache.status)
-        N.call("hsd_prefill_advance", N.ptr(cache.seq), T, 3, NSLAB, N.stream(self.device))
+        N.call("hsd_prefill_advance", cache.seq, T, 3, NSLAB, N.stream(self.device))
 
     def prefill(self, tokens, cache: ModelCache, with_head=None, graph=True):
         """tokens [T] (host ints or a tensor) -> the residual stream of the last position
@@ -717,7 +722,7 @@ class NemotronModel:
         x = self.embed(cache.seq[N.SEQ_TOK:N.SEQ_TOK + 1], out=buf["x"], status=cache.status)
         self.layers(x, buf, cache)
         self.head_keys(x, buf, buf["keys"])
-        N.call("hsd_decode_advance", N.ptr(buf["keys"]), self.slots, N.ptr(cache.seq), N.ptr(cache.out_tokens),
+        N.call("hsd_decode_advance", buf["keys"], self.slots, cache.seq, cache.out_tokens,
                cache.cap, NSLAB, N.stream(self.device))
 
     def step(self, x, cache):
@@ -732,10 +737,10 @@ class NemotronModel:
         # the advance of a decode step, then POS / CUR / STEPS back: the prompt's rows are
         # already in the caches
         st = N.stream(self.device)
-        N.call("hsd_decode_advance", N.ptr(buf["keys"]), self.slots, N.ptr(cache.seq), N.ptr(cache.out_tokens),
+        N.call("hsd_decode_advance", buf["keys"], self.slots, cache.seq, cache.out_tokens,
                cache.cap, NSLAB, st)
-        N.call("hsd_seq_rollback", N.ptr(cache.seq), 1, NSLAB, st)
-        N.call("hsd_seq_add", N.ptr(cache.seq), N.SEQ_STEPS, -1, st)
+        N.call("hsd_seq_rollback", cache.seq, 1, NSLAB, st)
+        N.call("hsd_seq_add", cache.seq, N.SEQ_STEPS, -1, st)
 
     def session(self, prompt, *, mtp=False, cap=4096, script=None, accepts=None, graph=True):
         """A generation after its prompt: the prompt prefilled (and the first token chosen),
@@ -773,8 +778,8 @@ class NemotronModel:
         if xb.data_ptr() != x.data_ptr():
             xb.copy_(x)
         self.layers(xb, buf, cache)
-        N.call("hsd_seq_add", N.ptr(cache.seq), N.SEQ_POS, B, N.stream(self.device))
-        N.call("hsd_mamba_select_row", N.ptr(cache.cur), None, B, B, NSLAB, None, N.stream(self.device))
+        N.call("hsd_seq_add", cache.seq, N.SEQ_POS, B, N.stream(self.device))
+        N.call("hsd_mamba_select_row", cache.cur, None, B, B, NSLAB, None, N.stream(self.device))
         return xb
 
     def rollback(self, cache, n_keep, B):
@@ -782,7 +787,7 @@ class NemotronModel:
         Mamba rings back to the checkpoint of row n_keep - 1)."""
         if n_keep == B:
             return
-        N.call("hsd_seq_rollback", N.ptr(cache.seq), B - n_keep, NSLAB, N.stream(self.device))
+        N.call("hsd_seq_rollback", cache.seq, B - n_keep, NSLAB, N.stream(self.device))
 
     # ---- MTP speculative decoding (model.py:366-443)
     def _mtp_step(self, cache, script=None, accepts=None):
@@ -803,15 +808,15 @@ class NemotronModel:
         # one launch writes the ids and their embedding rows
         ids = b3["ids"]
         emb = self.embedding
-        N.call("hsd_verify_input", N.ptr(b3["d1"]), N.ptr(b1["keys2"]), self.slots, 2, N.ptr(cache.seq),
-               N.ptr(script), 0 if script is None else script.numel(), N.ptr(accepts),
-               0 if accepts is None else accepts.numel(), c.vocab, N.ptr(emb.w), N.ptr(emb.scales),
-               N.ptr(emb.biases), c.hidden, N.ptr(ids), N.ptr(b3["x"]), b3["x"].stride(0), N.ptr(cache.status), st)
+        N.call("hsd_verify_input", b3["d1"], b1["keys2"], self.slots, 2, cache.seq,
+               script, 0 if script is None else script.numel(), accepts,
+               0 if accepts is None else accepts.numel(), c.vocab, emb.w, emb.scales,
+               emb.biases, c.hidden, ids, b3["x"], b3["x"].stride(0), cache.status, st)
         x = b3["x"][:3]
         self.layers(x, b3, cache)
         self.head_keys(x, b3, b3["keys"])
-        N.call("hsd_spec_accept", N.ptr(b3["keys"]), b3["keys"].stride(0), self.slots, 2, N.ptr(ids),
-               N.ptr(cache.seq), N.ptr(cache.out_tokens), cache.cap, NSLAB, N.ptr(b3["pend"]), None, st)
+        N.call("hsd_spec_accept", b3["keys"], b3["keys"].stride(0), self.slots, 2, ids,
+               cache.seq, cache.out_tokens, cache.cap, NSLAB, b3["pend"], None, st)
 
     def generate_mtp(self, prompt, mtp=None, n_draft=2, max_tokens=128, script=None, accepts=None, graph=True):
         """Greedy speculative decoding with the MTP head (model.py:366-443). Per step: the
@@ -872,7 +877,7 @@ class Session:
             b3 = model._bufs[3]
             b3["x"][0].copy_(x_last[0])
             b3["pend"][0:1].copy_(cache.seq[N.SEQ_TOK:N.SEQ_TOK + 1])
-            N.call("hsd_seq_add", N.ptr(cache.seq), N.SEQ_R, 1, N.stream(dev))
+            N.call("hsd_seq_add", cache.seq, N.SEQ_R, 1, N.stream(dev))
         torch.cuda.synchronize(dev)
         self.prompt_s = time.perf_counter() - t0
         cache.check_status("prefill")

@@ -144,10 +144,10 @@ def up_relu2(x, inds, w1, s1, b1, sw1, ss1, sb1, *, topk, live_masks=None, statu
                                    or live_masks.numel() < B * (NR // 64)):
         raise N.HSDError("live_masks must be a contiguous int64 tensor of B*(topk*F + FS)/64 entries")
     inds = inds if inds.dtype == torch.int32 and inds.is_contiguous() else N.contig(inds.to(torch.int32))
-    N.call("hsd_moe_up_relu2", N.ptr(x), N.dtype_tag(x.dtype), N.ptr(inds),
-           N.ptr(N.as_words(N.contig(w1))), N.ptr(N.contig(s1)), N.ptr(N.contig(b1)),
-           N.ptr(N.as_words(N.contig(sw1))), N.ptr(N.contig(ss1)), N.ptr(N.contig(sb1)), N.ptr(hcat),
-           B, D, F, FS, topk, E, N.ptr(live_masks), N.ptr(status), N.stream(x.device))
+    N.call("hsd_moe_up_relu2", x, N.dtype_tag(x.dtype), inds,
+           N.as_words(N.contig(w1)), N.contig(s1), N.contig(b1),
+           N.as_words(N.contig(sw1)), N.contig(ss1), N.contig(sb1), hcat,
+           B, D, F, FS, topk, E, live_masks, status, N.stream(x.device))
     return hcat
 
 
@@ -169,10 +169,10 @@ def route_up_relu2(x, logits, e_bias, w1, s1, b1, sw1, ss1, sb1, *, topk, routed
     hcat = out if out is not None else torch.empty((B, NR), dtype=torch.bfloat16, device=x.device)
     sel = sel if sel is not None else torch.empty((B, topk), dtype=torch.int32, device=x.device)
     gains = gains if gains is not None else torch.empty((B, topk + 1), dtype=torch.float32, device=x.device)
-    N.call("hsd_moe_route_up_relu2", N.ptr(x), N.DT_BF16, N.ptr(logits), N.ptr(e_bias), float(routed_scale),
-           1 if norm_topk else 0, N.ptr(sel), N.ptr(gains), N.ptr(N.as_words(N.contig(w1))), N.ptr(N.contig(s1)),
-           N.ptr(N.contig(b1)), N.ptr(N.as_words(N.contig(sw1))), N.ptr(N.contig(ss1)), N.ptr(N.contig(sb1)),
-           N.ptr(hcat), B, D, F, FS, topk, E, N.ptr(live_masks), N.stream(x.device))
+    N.call("hsd_moe_route_up_relu2", x, N.DT_BF16, logits, e_bias, float(routed_scale),
+           1 if norm_topk else 0, sel, gains, N.as_words(N.contig(w1)), N.contig(s1),
+           N.contig(b1), N.as_words(N.contig(sw1)), N.contig(ss1), N.contig(sb1),
+           hcat, B, D, F, FS, topk, E, live_masks, N.stream(x.device))
     return hcat, sel, gains
 
 
@@ -183,8 +183,8 @@ def router_topk(logits, e_bias, *, topk, routed_scale=1.0, norm_topk=True, sel=N
     B, E = logits.shape
     sel = sel if sel is not None else torch.empty((B, topk), dtype=torch.int32, device=logits.device)
     gains = gains if gains is not None else torch.empty((B, topk + 1), dtype=torch.float32, device=logits.device)
-    N.call("hsd_router_topk", N.ptr(logits), N.ptr(e_bias), float(routed_scale), 1 if norm_topk else 0, N.ptr(sel),
-           N.ptr(gains), B, E, topk, N.stream(logits.device))
+    N.call("hsd_router_topk", logits, e_bias, float(routed_scale), 1 if norm_topk else 0, sel,
+           gains, B, E, topk, N.stream(logits.device))
     return sel, gains
 
 

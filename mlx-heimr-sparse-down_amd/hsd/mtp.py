@@ -34,9 +34,9 @@ def greedy_accept(draft, logits, cur=None, nslab=4):
     draft = N.contig(draft.to(torch.int32)) if k > 0 else torch.zeros(1, dtype=torch.int32, device=dev)
     out = {n: torch.empty(s, dtype=torch.int32, device=dev)
            for n, s in (("tgt", k + 1), ("tokens", k + 1), ("n_accept", 1), ("n_keep", 1))}
-    N.call("hsd_greedy_accept", N.ptr(logits), N.dtype_tag(logits.dtype), k, V, N.ptr(draft),
-           N.ptr(out["tgt"]), N.ptr(out["tokens"]), N.ptr(out["n_accept"]), N.ptr(out["n_keep"]),
-           N.ptr(cur), nslab, N.stream(dev))
+    N.call("hsd_greedy_accept", logits, N.dtype_tag(logits.dtype), k, V, draft,
+           out["tgt"], out["tokens"], out["n_accept"], out["n_keep"],
+           cur, nslab, N.stream(dev))
     return out
 
 
@@ -93,7 +93,7 @@ class MTPHead:
             m.mtp_rows(x, toks[r0:r0 + n], b, self.kv, self._pos, keys=b["keys"][:n])
             nn.argmax(b["keys"][:n], n, out=pred[r0:r0 + n])
             hn[r0:r0 + n].copy_(b["hn"][:n])
-            N.call("hsd_seq_add", N.ptr(self._pos), 0, n, st)
+            N.call("hsd_seq_add", self._pos, 0, n, st)
         self.rows += R
         return pred, hn
 

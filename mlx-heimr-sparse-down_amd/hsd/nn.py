@@ -45,7 +45,7 @@ class QWeight:
 
 
 def argmax_slots(O, q4=True):
-    return int(N.lib().hsd_linear_argmax_slots(O, N.W_Q4 if q4 else N.W_BF16))
+    return int(N.call("hsd_linear_argmax_slots", O, N.W_Q4 if q4 else N.W_BF16))
 
 
 def linear(x, W: QWeight, *, norm=None, eps=1e-5, gate=None, gated_z=False, residual=None, out=None,
@@ -96,10 +96,10 @@ def linear(x, W: QWeight, *, norm=None, eps=1e-5, gate=None, gated_z=False, resi
         y = out if out is not None else torch.empty((B, W.O), dtype=out_dtype, device=x.device)
     if y is not None and (y.stride(1) != 1 or (y.dtype == torch.float32) != (yk == N.Y_F32)):
         raise N.HSDError("linear: out must have unit column stride and the requested dtype")
-    N.call("hsd_linear", N.ptr(x), x.stride(0), xk, N.ptr(gate), 0 if gate is None else gate.stride(0), N.ptr(norm),
-           float(eps), N.ptr(W.w), N.ptr(W.scales), N.ptr(W.biases), W.kind, N.ptr(y),
-           0 if y is None else y.stride(0), yk, N.ptr(residual), 0 if residual is None else residual.stride(0),
-           N.ptr(xn_out), 0 if xn_out is None else xn_out.stride(0), N.ptr(argmax_keys),
+    N.call("hsd_linear", x, x.stride(0), xk, gate, 0 if gate is None else gate.stride(0), norm,
+           float(eps), W.w, W.scales, W.biases, W.kind, y,
+           0 if y is None else y.stride(0), yk, residual, 0 if residual is None else residual.stride(0),
+           xn_out, 0 if xn_out is None else xn_out.stride(0), argmax_keys,
            0 if argmax_keys is None else argmax_keys.stride(0), B, W.O, W.I, N.stream(x.device))
     return y
 
@@ -108,7 +108,7 @@ def argmax(keys, B=None, out=None):
     """tok [B] int32 from the per-workgroup keys of linear(..., argmax_keys=keys)."""
     B = keys.shape[0] if B is None else B
     out = out if out is not None else torch.empty(B, dtype=torch.int32, device=keys.device)
-    N.call("hsd_argmax_keys", N.ptr(keys), keys.stride(0), keys.shape[1], B, N.ptr(out), N.stream(keys.device))
+    N.call("hsd_argmax_keys", keys, keys.stride(0), keys.shape[1], B, out, N.stream(keys.device))
     return out
 
 
@@ -117,8 +117,8 @@ def embed(tok, W: QWeight, out=None, status=None):
     B = tok.shape[0]
     D = W.I
     out = out if out is not None else torch.empty((B, D), dtype=torch.bfloat16, device=tok.device)
-    N.call("hsd_embed_q4", N.ptr(tok), B, N.ptr(W.w), N.ptr(W.scales), N.ptr(W.biases), W.O, D, N.ptr(out),
-           out.stride(0), N.ptr(status), N.stream(tok.device))
+    N.call("hsd_embed_q4", tok, B, W.w, W.scales, W.biases, W.O, D, out,
+           out.stride(0), status, N.stream(tok.device))
     return out
 
 
@@ -127,8 +127,8 @@ def pair_norm(e, h, we, wh, eps=1e-5, out=None):
     mtp.py:81-83)."""
     B, D = e.shape
     out = out if out is not None else torch.empty((B, 2 * D), dtype=torch.bfloat16, device=e.device)
-    N.call("hsd_pair_norm", N.ptr(e), e.stride(0), N.ptr(h), h.stride(0), N.ptr(we), N.ptr(wh), float(eps), B, D,
-           N.ptr(out), out.stride(0), N.stream(e.device))
+    N.call("hsd_pair_norm", e, e.stride(0), h, h.stride(0), we, wh, float(eps), B, D,
+           out, out.stride(0), N.stream(e.device))
     return out
 
 
@@ -141,10 +141,10 @@ def head_input(tok, h, W: QWeight, we, wh, eps=1e-5, out=None, status=None, chai
     B, D = h.shape
     out = out if out is not None else torch.empty((B, 2 * D), dtype=torch.bfloat16, device=h.device)
     keys, seq, d1 = chain if chain is not None else (None, None, None)
-    N.call("hsd_head_input", None if chain is not None else N.ptr(tok), N.ptr(keys),
-           0 if keys is None else keys.shape[-1], N.ptr(W.w), N.ptr(W.scales), N.ptr(W.biases), W.O, N.ptr(h),
-           h.stride(0), N.ptr(we), N.ptr(wh), float(eps), B, D, N.ptr(seq), N.ptr(d1), N.ptr(out), out.stride(0),
-           N.ptr(status), N.stream(h.device))
+    N.call("hsd_head_input", None if chain is not None else tok, keys,
+           0 if keys is None else keys.shape[-1], W.w, W.scales, W.biases, W.O, h,
+           h.stride(0), we, wh, float(eps), B, D, seq, d1, out, out.stride(0),
+           status, N.stream(h.device))
     return out
 
 
@@ -167,10 +167,10 @@ def attention(qkv, cache: KVCache, pos, *, n_heads, n_kv_heads, head_dim=128, sc
     B = qkv.shape[0]
     scale = 1.0 / math.sqrt(head_dim) if scale is None else scale
     out = out if out is not None else torch.empty((B, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
-    nbytes = N.lib().hsd_attn_workspace_bytes(B, n_heads, cache.smax)
+    nbytes = N.call("hsd_attn_workspace_bytes", B, n_heads, cache.smax)
     if workspace is None:
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=qkv.device)
-    N.call("hsd_attn_decode", N.ptr(qkv), qkv.stride(0), B, N.ptr(cache.k), N.ptr(cache.v), cache.smax, N.ptr(pos),
-           N.ptr(out), out.stride(0), n_heads, n_kv_heads, head_dim, float(scale), N.ptr(status), N.ptr(workspace),
+    N.call("hsd_attn_decode", qkv, qkv.stride(0), B, cache.k, cache.v, cache.smax, pos,
+           out, out.stride(0), n_heads, n_kv_heads, head_dim, float(scale), status, workspace,
            workspace.numel() * workspace.element_size(), N.stream(qkv.device))
     return out

@@ -28,9 +28,9 @@ def build_tiles(sel, E, tt, status=None):
     NT = num_tiles(T, K, E, tt)
     tile_e = torch.empty(NT, dtype=torch.int32, device=sel.device)
     tile_slot = torch.empty(NT * tt, dtype=torch.int32, device=sel.device)
-    ws = _workspace(N.lib().hsd_prefill_tiles_workspace_bytes(T, K, E), sel.device, None)
-    N.call("hsd_prefill_tiles", N.ptr(sel), T, K, E, tt, N.ptr(tile_e), N.ptr(tile_slot),
-           N.ptr(status), N.ptr(ws), ws.numel(), N.stream(sel.device))
+    ws = _workspace(N.call("hsd_prefill_tiles_workspace_bytes", T, K, E), sel.device, None)
+    N.call("hsd_prefill_tiles", sel, T, K, E, tt, tile_e, tile_slot,
+           status, ws, ws.numel(), N.stream(sel.device))
     return tile_e, tile_slot
 
 
@@ -45,8 +45,8 @@ def build_union(h, tile_e, tile_slot, *, F, FS, topk, E, tt, kc=32, nth=256):
     umax = (FS + kc - 1) // kc * kc
     ulist = torch.empty((NT, umax), dtype=torch.int32, device=h.device)
     ucount = torch.empty(NT, dtype=torch.int32, device=h.device)
-    N.call("hsd_prefill_union", N.ptr(h), N.dtype_tag(h.dtype), N.ptr(N.contig(tile_e)),
-           N.ptr(N.contig(tile_slot)), N.ptr(ulist), N.ptr(ucount), T, F, FS, topk, E, tt, NT,
+    N.call("hsd_prefill_union", h, N.dtype_tag(h.dtype), N.contig(tile_e),
+           N.contig(tile_slot), ulist, ucount, T, F, FS, topk, E, tt, NT,
            umax, N.stream(h.device))
     return ulist, ucount
 
@@ -75,12 +75,12 @@ def sparse_down_prefill(h, sel, gains, pw, ps, pb, spw, sps, spb, *, F, FS, D, t
     NT = tile_e.shape[0]
     gains = N.contig(gains.to(torch.float32))
     y = torch.empty((T, D), dtype=od, device=h.device)
-    ws = _workspace(N.lib().hsd_prefill_gemm_workspace_bytes(T, D, F, FS, topk, E, tt), h.device,
+    ws = _workspace(N.call("hsd_prefill_gemm_workspace_bytes", T, D, F, FS, topk, E, tt), h.device,
                     workspace)
     sel = N.contig(sel.to(torch.int32))
-    N.call("hsd_prefill_gemm", N.ptr(h), N.ptr(sel), N.ptr(gains), N.ptr(N.contig(tile_e)), N.ptr(N.contig(tile_slot)),
-           N.ptr(N.contig(ulist)), N.ptr(N.contig(ucount)), N.ptr(N.as_words(N.contig(pw))),
-           N.ptr(N.contig(ps)), N.ptr(N.contig(pb)), N.ptr(N.as_words(N.contig(spw))),
-           N.ptr(N.contig(sps)), N.ptr(N.contig(spb)), N.ptr(y), N.dtype_tag(od), T, D, F, FS, topk,
-           E, tt, NT, ulist.shape[1], N.ptr(ws), ws.numel(), N.stream(h.device))
+    N.call("hsd_prefill_gemm", h, sel, gains, N.contig(tile_e), N.contig(tile_slot),
+           N.contig(ulist), N.contig(ucount), N.as_words(N.contig(pw)),
+           N.contig(ps), N.contig(pb), N.as_words(N.contig(spw)),
+           N.contig(sps), N.contig(spb), y, N.dtype_tag(od), T, D, F, FS, topk,
+           E, tt, NT, ulist.shape[1], ws, ws.numel(), N.stream(h.device))
     return y

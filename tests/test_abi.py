@@ -205,3 +205,25 @@ def test_capture_guard_pauses_the_collector():
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+def test_native_entries_cover_the_table():
+    """Every entry point of the signature table (but the two plain readers) is a native function
+    of hsd._hsdcall, which raises what a bad argument or a refused call gives."""
+    import torch
+    for name in N.EXPORTS:
+        if name not in ("hsd_last_error", "hsd_abi_version"):
+            assert callable(N.entry(name)), name
+    f = N.entry("hsd_permute_nibbles")
+    with pytest.raises(N.HSDError, match="null"):
+        f(None, None, 1, 8, 1, None)
+    with pytest.raises(N.HSDError, match="multiple of 8"):
+        f(16, ctypes.c_void_p(16), 1, 12, 1, 0)
+    with pytest.raises(N.HSDError, match="device tensors"):
+        f(torch.zeros(4), 16, 1, 8, 1, None)
+    with pytest.raises(TypeError):
+        f(16, 16)
+    with pytest.raises((TypeError, OverflowError)):
+        f(16, 16, 1 << 80, 8, 1, None)
+    assert N.call("hsd_sparse_down_workspace_bytes", 1, 2688, 1856, 3712, 6) == \
+        N.lib().hsd_sparse_down_workspace_bytes(1, 2688, 1856, 3712, 6)
