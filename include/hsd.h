@@ -72,6 +72,13 @@ int hsd_permute_nibbles(const uint32_t* w, uint32_t* out, int64_t batch, int64_t
 int hsd_transpose_u16(const uint16_t* in, uint16_t* out, int64_t batch, int64_t rows,
                       int64_t cols, void* stream);
 
+/* Both for a weight's three tensors in one launch (hsd/layout.py:53-74): w [batch, rows,
+ * words] as hsd_permute_nibbles, s and b [batch, rows, groups] as hsd_transpose_u16.
+ * groups <= 64, rows % 8 == 0, 16-byte aligned s and b. */
+int hsd_neuron_major(const uint32_t* w, const uint16_t* s, const uint16_t* b, uint32_t* pw,
+                     uint16_t* ps, uint16_t* pb, int64_t batch, int64_t rows, int64_t words,
+                     int64_t groups, void* stream);
+
 /* ------------------------------------------------------------------ decode
  * Replaces hsd/decode.py:164-186 `sparse_down(h, sel, gains, pw, ps, pb, spw, sps,
  * spb, *, F, FS, D, topk, ...)` (kernels decode.py:37-144).

@@ -42,42 +42,48 @@ __device__ __forceinline__ void transpose8x8_nibbles(uint32_t v[8]) {
   }
 }
 
+// Tile (cw0, wo0) of w [R, CW] -> out [8*CW, R/8]. Every load of the tile is issued before the
+// first is used (positions past the edges re-read the last one: a load under a branch would
+// end in a wait per iteration).
+__device__ __forceinline__ void permute_tile(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int64_t R,
+                                             int64_t CW, int64_t cw0, int64_t wo0, uint32_t* tileT, int tid) {
+  const int64_t RW = R / 8;
+  constexpr int kIt = (kTile * kTile) / kThreads;
+  uint32_t v[kIt][8];
+  const int cw_l = tid & (kTile - 1);
+  const int64_t cw = min(cw0 + cw_l, CW - 1);
+#pragma unroll
+  for (int i = 0; i < kIt; ++i) {
+    const int64_t wo = min(wo0 + (tid + kThreads * i) / kTile, RW - 1);
+#pragma unroll
+    for (int n = 0; n < 8; ++n) v[i][n] = src[(8 * wo + n) * CW + cw];
+  }
+#pragma unroll
+  for (int i = 0; i < kIt; ++i) {
+    const int wo_l = (tid + kThreads * i) / kTile;
+    transpose8x8_nibbles(v[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tileT[(8 * cw_l + j) * kTile + (wo_l ^ cw_l)] = v[i][j];
+  }
+  __syncthreads();
+  const int wo_l = tid & (kTile - 1);
+#pragma unroll 4
+  for (int row = tid / kTile; row < 8 * kTile; row += kThreads / kTile) {
+    const int cl = row >> 3;
+    const int64_t orow = 8 * cw0 + row, wo = wo0 + wo_l;
+    if (cw0 + cl < CW && wo < RW) dst[orow * RW + wo] = tileT[row * kTile + (wo_l ^ cl)];
+  }
+}
+
 // w [batch, R, CW] -> out [batch, 8*CW, R/8]
 __global__ __launch_bounds__(kThreads) void k_permute_nibbles(const uint32_t* __restrict__ w,
                                                               uint32_t* __restrict__ out,
                                                               int64_t R, int64_t CW,
                                                               int tiles_cw) {
   __shared__ uint32_t tileT[8 * kTile * kTile];  // [8*cw_l + j][wo_l ^ cw_l]
-  const int64_t RW = R / 8;
-  const int tid = threadIdx.x;
   const int64_t b = blockIdx.y;
-  const int64_t cw0 = (int64_t)(blockIdx.x % tiles_cw) * kTile;
-  const int64_t wo0 = (int64_t)(blockIdx.x / tiles_cw) * kTile;
-  const uint32_t* src = w + b * R * CW;
-  uint32_t* dst = out + b * (8 * CW) * RW;
-
-#pragma unroll
-  for (int i = 0; i < (kTile * kTile) / kThreads; ++i) {
-    const int bi = tid + kThreads * i;
-    const int cw_l = bi & (kTile - 1), wo_l = bi / kTile;
-    const int64_t cw = cw0 + cw_l, wo = wo0 + wo_l;
-    uint32_t v[8];
-    if (cw < CW && wo < RW) {
-#pragma unroll
-      for (int n = 0; n < 8; ++n) v[n] = src[(8 * wo + n) * CW + cw];
-      transpose8x8_nibbles(v);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) tileT[(8 * cw_l + j) * kTile + (wo_l ^ cw_l)] = v[j];
-    }
-  }
-  __syncthreads();
-  const int wo_l = tid & (kTile - 1);
-#pragma unroll 4
-  for (int row = tid / kTile; row < 8 * kTile; row += kThreads / kTile) {
-    const int cw_l = row >> 3;
-    const int64_t orow = 8 * cw0 + row, wo = wo0 + wo_l;
-    if (cw0 + cw_l < CW && wo < RW) dst[orow * RW + wo] = tileT[row * kTile + (wo_l ^ cw_l)];
-  }
+  permute_tile(w + b * R * CW, out + b * R * CW, R, CW, (int64_t)(blockIdx.x % tiles_cw) * kTile,
+               (int64_t)(blockIdx.x / tiles_cw) * kTile, tileT, (int)threadIdx.x);
 }
 
 constexpr int kT16 = 64;
@@ -101,6 +107,57 @@ __global__ __launch_bounds__(kThreads) void k_transpose_u16(const uint16_t* __re
   for (int lr = tid / kT16; lr < kT16; lr += kThreads / kT16) {
     const int64_t c = c0 + lr, r = r0 + lc;  // output row c, column r
     if (r < R && c < C) dst[c * R + r] = (uint16_t)tile[lc][lr];
+  }
+}
+
+// A whole weight in one launch: the nibble tiles of every matrix, then kTR-row pieces of its
+// scales and its biases [batch, R, G] -> [batch, G, R] with G <= 64. A piece's kTR rows are
+// contiguous (16-byte loads) and its columns become G runs of 2 kTR bytes: 128 experts' scales
+// 35 -> 12 us against 64 x 64 tiles of which G = 29 columns fill less than half. Consecutive
+// nibble tiles run on one XCD, whose L2 joins the tiles' shares of a 128-byte line (rows of
+// 928 and 1344 bytes are not multiples of it).
+constexpr int kTR = 128;
+constexpr int kGMaxT = 64;
+__global__ __launch_bounds__(kThreads) void k_neuron_major(
+    const uint32_t* __restrict__ w, const uint16_t* __restrict__ s, const uint16_t* __restrict__ b,
+    uint32_t* __restrict__ pw, uint16_t* __restrict__ ps, uint16_t* __restrict__ pb, int64_t R, int64_t CW, int G,
+    int tiles_cw, int tiles, int nperm, int pieces) {
+  __shared__ __attribute__((aligned(16))) uint32_t lds[8 * kTile * kTile];
+  static_assert(sizeof(uint32_t) * 8 * kTile * kTile >= sizeof(uint16_t) * kGMaxT * (kTR + 2), "the piece fits the tile");
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < nperm) {
+    const int id = xcd_remap((int)blockIdx.x, nperm), m = id / tiles, t = id - m * tiles;
+    permute_tile(w + (int64_t)m * R * CW, pw + (int64_t)m * R * CW, R, CW, (int64_t)(t % tiles_cw) * kTile,
+                 (int64_t)(t / tiles_cw) * kTile, lds, tid);
+    return;
+  }
+  const int id = (int)blockIdx.x - nperm, half = (int)(gridDim.x - nperm) / 2;
+  const bool bias = id >= half;
+  const int u = bias ? id - half : id, m = u / pieces;
+  const int64_t r0 = (int64_t)(u - m * pieces) * kTR;
+  const int rows = (int)min((int64_t)kTR, R - r0);
+  const uint16_t* src = (bias ? b : s) + ((int64_t)m * R + r0) * G;
+  uint16_t* dst = (bias ? pb : ps) + (int64_t)m * R * G;
+  uint16_t* tile = reinterpret_cast<uint16_t*>(lds);   // [G][kTR + 2]
+  const int nv = rows * G / 8;                         // R and so rows are multiples of 8
+  for (int i = tid; i < nv; i += kThreads) {
+    const uint4 v = reinterpret_cast<const uint4*>(src)[i];
+    const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+    int r = 8 * i / G, c = 8 * i - r * G;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      tile[c * (kTR + 2) + r] = (uint16_t)((k & 1) ? x[k >> 1] >> 16 : x[k >> 1]);
+      if (++c == G) {
+        c = 0;
+        ++r;
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < G * (kTR / 2); i += kThreads) {
+    const int c = i / (kTR / 2), r = 2 * (i - c * (kTR / 2));
+    if (r < rows)
+      *reinterpret_cast<uint32_t*>(dst + (int64_t)c * R + r0 + r) = *reinterpret_cast<const uint32_t*>(&tile[c * (kTR + 2) + r]);
   }
 }
 
@@ -137,4 +194,21 @@ extern "C" int hsd_transpose_u16(const uint16_t* in, uint16_t* out, int64_t batc
   hipLaunchKernelGGL(k_transpose_u16, grid, dim3(kThreads), 0, as_stream(stream), in, out, rows,
                      cols, (int)tc);
   return check_launch("hsd_transpose_u16");
+}
+
+extern "C" int hsd_neuron_major(const uint32_t* w, const uint16_t* s, const uint16_t* b, uint32_t* pw, uint16_t* ps,
+                                uint16_t* pb, int64_t batch, int64_t rows, int64_t words, int64_t groups, void* stream) {
+  const char* fn = "hsd_neuron_major";
+  if (!w || !s || !b || !pw || !ps || !pb) return set_error(HSD_ERR_ARG, "%s: null pointer", fn);
+  if (batch < 0 || rows < 0 || rows % 8 || words < 0 || groups < 1 || groups > kGMaxT || batch > 65535)
+    return set_error(HSD_ERR_SHAPE, "%s: need rows %% 8 == 0 and 1 <= groups <= %d", fn, kGMaxT);
+  if (((uintptr_t)s | (uintptr_t)b) & 15u || ((uintptr_t)ps | (uintptr_t)pb) & 3u)
+    return set_error(HSD_ERR_ALIGN, "%s: scales and biases must be 16-byte aligned", fn);
+  if (batch == 0 || rows == 0 || words == 0) return HSD_OK;
+  const int64_t tcw = (words + kTile - 1) / kTile, tiles = tcw * ((rows / 8 + kTile - 1) / kTile);
+  const int64_t pieces = (rows + kTR - 1) / kTR, grid = batch * (tiles + 2 * pieces);
+  if (grid > 0x7FFFFFFF || rows * groups > 0x7FFFFFFF) return set_error(HSD_ERR_SHAPE, "%s: too large", fn);
+  hipLaunchKernelGGL(k_neuron_major, dim3((unsigned)grid), dim3(kThreads), 0, as_stream(stream), w, s, b, pw, ps, pb, rows,
+                     words, (int)groups, (int)tcw, (int)tiles, (int)(batch * tiles), (int)pieces);
+  return check_launch(fn);
 }

@@ -16,6 +16,7 @@ namespace {
 #define HSD_ENTRIES(X) \
   X(hsd_permute_nibbles) \
   X(hsd_transpose_u16) \
+  X(hsd_neuron_major) \
   X(hsd_sparse_down_decode) \
   X(hsd_sparse_down_residual) \
   X(hsd_sparse_down_decode_noalloc) \

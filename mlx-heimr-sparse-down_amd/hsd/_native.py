@@ -54,6 +54,7 @@ _SIGS = {
     "hsd_abi_version": (_c_int, []),
     "hsd_permute_nibbles": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
     "hsd_transpose_u16": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "hsd_neuron_major": (_c_int, [_vp] * 6 + [_c_i64] * 4 + [_vp]),
     "hsd_sparse_down_workspace_bytes": (_c_size, [_c_i64] * 5),
     "hsd_sparse_down_decode": (_c_int, [_vp, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int,
                                         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _vp,

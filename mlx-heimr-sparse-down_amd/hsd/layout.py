@@ -18,6 +18,8 @@ kernel (libhsd `hsd_permute_nibbles`); the scales and biases are moved bit for b
 """
 from __future__ import annotations
 
+import math
+
 import torch
 
 from . import _native as N
@@ -57,4 +59,16 @@ def to_neuron_major(w: torch.Tensor, s: torch.Tensor, b: torch.Tensor, chunk: in
     (pw [.., F, D/8], ps [.., F/64, D], pb [.., F/64, D]). `chunk` is accepted for API
     compatibility: the device permutation needs no transient, so it is not chunked."""
     del chunk
+    w, s, b = N.contig(w), N.contig(N.as_u16(s)), N.contig(N.as_u16(b))
+    *lead, R, CW = w.shape
+    G = s.shape[-1]
+    # one launch for the three, where its kernel takes them: matching shapes, few groups
+    if s.shape == b.shape == (*lead, R, G) and R % 8 == 0 and G <= 64 and (s.data_ptr() | b.data_ptr()) % 16 == 0:
+        batch = math.prod(lead)
+        pw = torch.empty((*lead, CW * 8, R // 8), dtype=torch.int32, device=w.device)
+        ps = torch.empty((*lead, G, R), dtype=s.dtype, device=s.device)
+        pb = torch.empty((*lead, G, R), dtype=b.dtype, device=b.device)
+        if pw.numel() and ps.numel() and batch <= 65535:
+            N.call("hsd_neuron_major", N.as_words(w), s, b, pw, ps, pb, batch, R, CW, G, N.stream(w.device))
+            return pw.view(w.dtype) if w.dtype != torch.int32 else pw, ps, pb
     return nibble_transpose(w), transpose_last2(s), transpose_last2(b)
