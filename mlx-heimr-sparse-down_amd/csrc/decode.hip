@@ -43,7 +43,8 @@ constexpr int kWPC = 16;                 // weight words per D chunk (one lane e
 constexpr int kThreads = kGPW * kWPC * kRS;
 constexpr int kDC = kWPC * 8;            // outputs per D chunk
 constexpr int kL1 = kThreads / kDC;      // first-level sub-sums per output
-constexpr int kRB = 16;                  // rows per team per batch (a phase has 32 rows)
+constexpr int kRowBatch = 16;            // rows per team per batch (a phase has 32 rows), / W
+constexpr int kWideRows = 2;             // token rows from which a lane takes two words
 
 struct Geom {
   int D, F, FS, topk, E, NR, NW;
@@ -80,9 +81,16 @@ template <> __device__ __forceinline__ bool live_bits<HSD_DT_BF16>(uint16_t v) {
 template <> __device__ __forceinline__ bool live_bits<HSD_DT_F16>(uint16_t v) { return (v & 0x7FFFu) != 0; }
 template <> __device__ __forceinline__ bool live_bits<HSD_DT_F32>(float v) { return !(v == 0.0f); }
 
-template <int HDT>
+// W: weight words per lane (a D chunk is 128 W outputs). The kernel is bound by its vector
+// instructions (two per weight, and about as many again per row and word for the list entry,
+// the activation, the address and the load's select), which two words per lane share between 16
+// outputs. The sums' order is the same. One call, one word -> two words (2688 outputs, 10 % of
+// 14848 inputs live), us: 1 row 6.7 -> 6.9, 2 rows 8.7 -> 8.4, 3 rows 10.2 -> 9.2, 8 rows
+// 18.2 -> 15.1, 32 rows 53.3 -> 41.3, 64 rows 101 -> 77: one row, where half the workgroups
+// leave the chip short, keeps one word.
+template <int HDT, int W>
 __global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 ? 7 : 8))) void k_sparse_down_part(
+__attribute__((amdgpu_waves_per_eu(W > 1 ? 5 : HDT == HSD_DT_F32 ? 7 : 8, W > 1 ? 8 : HDT == HSD_DT_F32 ? 7 : 8))) void k_sparse_down_part(
     const typename Elem<HDT>::T* __restrict__ h, const int32_t* __restrict__ sel,
     const float* __restrict__ gains, int nwg_, int nchunk_, int topk_, int ppr_, int gpr_, int gsh_, int nblk_,
     int F_, const uint32_t* __restrict__ pw, const uint16_t* __restrict__ ps, const uint16_t* __restrict__ pb,
@@ -107,7 +115,8 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
   // Per-team rows padded by 64 bytes, so that the team strides are 16 banks mod 32 and
   // the four teams of a wavefront (16 lanes each) write different LDS banks.
   constexpr int kHP = 64 + 64 / (int)sizeof(HT);
-  constexpr int kRedP = 8 * kWPC + 16;
+  constexpr int kRedP = 8 * kWPC * W + 16;
+  constexpr int kRB = kRowBatch / W;
   // 16-bit activations: each list entry carries the row's activation bits beside its index
   // ((bits << 16) | row), so one LDS read per row gives both and a lane holds one register
   // per row instead of two (64 VGPRs: 8 wavefronts per SIMD); fp32: index list + table
@@ -116,7 +125,7 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
   __shared__ uint8_t lst[kPack ? 1 : kGPW * kRS][64];  // per team: the group's live rows, ascending
   __shared__ uint32_t lsp[kPack ? kGPW * kRS : 1][64];  // the same with the activation bits
   __shared__ float red[kGPW * kRS][kRedP];          // per team: group terms [t][word]
-  __shared__ float sum2[kDC][kL1 + 1];
+  __shared__ float sum2[kDC * W][kL1 + 1];
 
   // grid (chunk, part, token row): the coordinates need no division (a one-dimensional
   // grid placed on the XCDs by part took 3 divisions ahead of the first loads: one call
@@ -150,13 +159,18 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
   const bool ok = !routed || (unsigned)e < (unsigned)g.E;
   // the group's scale and bias vectors depend on the expert id alone: issued as soon as
   // the id is in, while the activations are still on their way
-  const int w = c * kWPC + l;
+  // (W > 1: lanes of the last chunk past D re-read its last words and are not written)
+  const int w = W > 1 ? min((c * kWPC + l) * W, g.NW - W) : c * kWPC + l;
   const size_t es = ok ? (size_t)e : 0;
   const uint16_t* sb = routed ? ps + es * (size_t)g.gpr * g.D : sps;
   const uint16_t* bb = routed ? pb + es * (size_t)g.gpr * g.D : spb;
   const size_t soff = ((size_t)grc * g.D + 8u * (uint32_t)w) * 2u;
-  const uint4 sv = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(sb) + soff);
-  const uint4 bv = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(bb) + soff);
+  uint4 sv[W], bv[W];
+#pragma unroll
+  for (int u = 0; u < W; ++u) {
+    sv[u] = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(sb) + soff)[u];
+    bv[u] = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(bb) + soff)[u];
+  }
   __builtin_amdgcn_sched_barrier(0);
   HT hv[4];
 #pragma unroll
@@ -194,9 +208,11 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
   // ---- round trip 2: live rows of this phase
   const uint32_t* wb = routed ? pw + es * (size_t)g.F * g.NW : spw;
   const uint32_t row0 = (uint32_t)grp * 64u * (uint32_t)g.NW + (uint32_t)w;
-  float acc[8];
+  float acc[W][8];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = 0.0f;
+  for (int u = 0; u < W; ++u)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[u][t] = 0.0f;
   float hsum = 0.0f;
   const int nmine = cnt;                              // this team's rows
   // most rows of any team of the wave: a team is one 16-lane row, so lanes 0, 16, 32
@@ -213,13 +229,21 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
       else
         ent[r] = r0 + r < nmine ? (uint32_t)lst[team][r0 + r] : 0u;
     }
-    uint32_t q[kRB];
+    uint32_t q[kRB][W];
 #pragma unroll
     for (int r = 0; r < kRB; ++r) {
-      q[r] = 0u;
-      if (r0 + r < nmine)
-        q[r] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(wb) +
-                                                  (size_t)(row0 + (ent[r] & 63u) * (uint32_t)g.NW) * 4u);
+#pragma unroll
+      for (int u = 0; u < W; ++u) q[r][u] = 0u;
+      if (r0 + r < nmine) {
+        const char* src = reinterpret_cast<const char*>(wb) + (size_t)(row0 + (ent[r] & 63u) * (uint32_t)g.NW) * 4u;
+        if constexpr (W == 2) {
+          const uint2 v = *reinterpret_cast<const uint2*>(src);
+          q[r][0] = v.x;
+          q[r][1] = v.y;
+        } else {
+          q[r][0] = *reinterpret_cast<const uint32_t*>(src);
+        }
+      }
     }
     float hx[kPack ? 1 : kRB];
     if constexpr (!kPack) {
@@ -239,23 +263,29 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
         }
         x = r0 + r < nmine ? x : 0.0f;
         hsum += x;
-        const uint32_t lo = q[r] & 0x0F0F0F0Fu, hi = (q[r] >> 4) & 0x0F0F0F0Fu;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[2 * i] = fmaf(x, (float)((lo >> (8 * i)) & 0xFFu), acc[2 * i]);
-          acc[2 * i + 1] = fmaf(x, (float)((hi >> (8 * i)) & 0xFFu), acc[2 * i + 1]);
+        for (int u = 0; u < W; ++u) {
+          const uint32_t lo = q[r][u] & 0x0F0F0F0Fu, hi = (q[r][u] >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            acc[u][2 * i] = fmaf(x, (float)((lo >> (8 * i)) & 0xFFu), acc[u][2 * i]);
+            acc[u][2 * i + 1] = fmaf(x, (float)((hi >> (8 * i)) & 0xFFu), acc[u][2 * i + 1]);
+          }
         }
       }
     }
   }
 
   // ---- group terms, then the ordered sum over (group, phase), two levels
-  const uint32_t s32[4] = {sv.x, sv.y, sv.z, sv.w};
-  const uint32_t b32[4] = {bv.x, bv.y, bv.z, bv.w};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    red[team][(2 * i) * kWPC + l] = fmaf(lo_bf16(s32[i]), acc[2 * i], lo_bf16(b32[i]) * hsum);
-    red[team][(2 * i + 1) * kWPC + l] = fmaf(hi_bf16(s32[i]), acc[2 * i + 1], hi_bf16(b32[i]) * hsum);
+  for (int u = 0; u < W; ++u) {
+    const uint32_t s32[4] = {sv[u].x, sv[u].y, sv[u].z, sv[u].w};
+    const uint32_t b32[4] = {bv[u].x, bv[u].y, bv[u].z, bv[u].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      red[team][(8 * u + 2 * i) * kWPC + l] = fmaf(lo_bf16(s32[i]), acc[u][2 * i], lo_bf16(b32[i]) * hsum);
+      red[team][(8 * u + 2 * i + 1) * kWPC + l] = fmaf(hi_bf16(s32[i]), acc[u][2 * i + 1], hi_bf16(b32[i]) * hsum);
+    }
   }
   __syncthreads();
   // level 1: kThreads/kDC threads per output, each over a contiguous run of groups. A
@@ -264,29 +294,33 @@ __attribute__((amdgpu_waves_per_eu(HDT == HSD_DT_F32 ? 7 : 8, HDT == HSD_DT_F32 
   constexpr int kGPS = kGPW / kL1;                    // groups per sub-sum
   {
     const int o = tid % kDC, s = tid / kDC;
-    const int lw = o % kWPC, t = o / kWPC, col = 8 * lw + t;
-    float acc2 = 0.0f;
-    bool first = true;
+    const int lw = o % kWPC, t = o / kWPC;
 #pragma unroll
-    for (int i = 0; i < kGPS; ++i) {
-      const int jj = s * kGPS + i;
-      if (jj < ng) {
+    for (int u = 0; u < W; ++u) {
+      float acc2 = 0.0f;
+      bool first = true;
 #pragma unroll
-        for (int ph = 0; ph < kRS; ++ph) {
-          const float v = red[ph * kGPW + jj][t * kWPC + lw];
-          acc2 = first ? v : acc2 + v;
-          first = false;
+      for (int i = 0; i < kGPS; ++i) {
+        const int jj = s * kGPS + i;
+        if (jj < ng) {
+#pragma unroll
+          for (int ph = 0; ph < kRS; ++ph) {
+            const float v = red[ph * kGPW + jj][(8 * u + t) * kWPC + lw];
+            acc2 = first ? v : acc2 + v;
+            first = false;
+          }
         }
       }
+      sum2[8 * (W * lw + u) + t][s] = acc2;
     }
-    sum2[col][s] = acc2;
   }
   __syncthreads();
-  if (tid < kDC) {
-    float v = sum2[tid][0];
+  for (int i = tid; i < kDC * W; i += kThreads) {
+    float v = sum2[i][0];
 #pragma unroll
-    for (int s = 1; s < kL1; ++s) v += sum2[tid][s];
-    part[((size_t)b * g.nparts + p) * g.D + (size_t)c * kDC + tid] = gain * v;
+    for (int s = 1; s < kL1; ++s) v += sum2[i][s];
+    const size_t col = (size_t)c * (kDC * W) + i;
+    if (W == 1 || col < (size_t)g.D) part[((size_t)b * g.nparts + p) * g.D + col] = gain * v;
   }
   if (!ok && tid == 0 && c == 0 && status) atomicOr(status, (int32_t)HSD_STATUS_BAD_EXPERT);
 }
@@ -625,18 +659,22 @@ int launch_sparse_down(const char* fn, const void* h, int h_dtype, const int32_t
   // the grid is (chunks, parts, token rows): at most 65535 token rows per call
   if (B > 65535 || g.nparts > 65535) return set_error(HSD_ERR_SHAPE, "%s: too many token rows or parts", fn);
   const int64_t nblk = B * (int64_t)g.nwg;
-#define HSD_PART(DT)                                                                          \
-  hipLaunchKernelGGL(k_sparse_down_part<DT>, dim3((unsigned)g.nchunk, (unsigned)g.nparts, (unsigned)B),      \
-                     dim3(kThreads), 0, st,                                                               \
+  const bool wide = B >= kWideRows && !(((uintptr_t)pw | (uintptr_t)spw) & 7u);
+#define HSD_PART_W(DT, W)                                                                     \
+  hipLaunchKernelGGL((k_sparse_down_part<DT, W>), dim3((unsigned)((D + kDC * W - 1) / (kDC * W)), (unsigned)g.nparts, \
+                     (unsigned)B), dim3(kThreads), 0, st,                                                 \
                      reinterpret_cast<const typename Elem<DT>::T*>(h), sel, gains, g.nwg, g.nchunk,   \
                      g.topk, g.ppr, g.gpr, g.gsh, (int)nblk, g.F, pw, ps, pb, spw, sps, spb, part,    \
                      live_masks, dev_status, g, dense)
+#define HSD_PART(DT) \
+  if (wide) HSD_PART_W(DT, 2); else HSD_PART_W(DT, 1)
   switch (h_dtype) {
     case HSD_DT_BF16: HSD_PART(HSD_DT_BF16); break;
     case HSD_DT_F16: HSD_PART(HSD_DT_F16); break;
     case HSD_DT_F32: HSD_PART(HSD_DT_F32); break;
     default: return set_error(HSD_ERR_DTYPE, "%s: h_dtype %d", fn, h_dtype);
   }
+#undef HSD_PART_W
 #undef HSD_PART
   int rc = check_launch(fn);
   if (rc) return rc;
