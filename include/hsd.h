@@ -352,14 +352,15 @@ int hsd_seq_add(int32_t* seq, int64_t idx, int64_t delta, void* stream);
  * the matrix cores').
  * hsd_rows_prep: the prologue of hsd_linear (x_kind HSD_X_BF16, HSD_X_RMS or HSD_X_GATED_Z,
  * the same bits) for T rows -> xp [T, I] bf16. hs non-null: xp's inputs in the order
- * 0 4 1 5 2 6 3 7 of every 8 and hs [T, 2 GP] bf16, GP = ceil(I/64/8)*8: every 64-input
- * group's sum as hi + lo (zero past I/64); hs null: the natural order.
+ * 0 4 1 5 2 6 3 7 of every 8 and hs [T, 3 GP] bf16, GP = ceil(I/64/8)*8: every 64-input
+ * group's sum as the sum of three bf16 values (zero past I/64); hs null: the natural order.
  * I a multiple of 64 (8 without hs; 512 for the gated norm), at most 6144. */
 int hsd_rows_prep(const void* x, int64_t x_ld, int x_kind, const uint16_t* norm_w, float eps,
                   uint16_t* xp, uint16_t* hs, int64_t T, int64_t I, void* stream);
 
 /* y [T, O] = xn W^T in bf16, W 4-bit (stock layout), from hsd_rows_prep's xp and hs; res
- * non-null: y = bf16(res + bf16(xn W^T)) (y may be res). I a multiple of 128. */
+ * non-null: y = bf16(res + bf16(xn W^T)) (y may be res). I a multiple of 128; y, res and the
+ * buffers of the two calls below less than 1 GiB each. */
 int hsd_gemm_q4(const uint16_t* xp, const uint16_t* hs, const uint32_t* w, const uint16_t* s,
                 const uint16_t* b, uint16_t* y, int64_t y_ld, const uint16_t* res, int64_t res_ld,
                 int64_t T, int64_t O, int64_t I, void* stream);
@@ -375,8 +376,8 @@ int hsd_moe_tiles(const int32_t* sel, int64_t T, int64_t topk, int64_t E, int64_
 
 /* hsd_moe_up_relu2 for a chunk: hcat [T, topk*F + FS] from hsd_rows_prep's xp and hs and
  * hsd_moe_tiles' lists (tt 32 or 64); the slots of experts outside [0, E) are not written.
- * hsum (nullable, [T, topk + 1, 2 GPH] bf16, GPH = ceil(max(F, FS)/64/8)*8): the sum of every
- * 64 neurons of a slot's h as hi + lo, for hsd_moe_down_gemm (entries past a slot's groups
+ * hsum (nullable, [T, topk + 1, 3 GPH] bf16, GPH = ceil(max(F, FS)/64/8)*8): the sum of every
+ * 64 neurons of a slot's h as three bf16 values, for hsd_moe_down_gemm (entries past a slot's groups
  * are not written). D a multiple of 128. */
 int hsd_moe_up_gemm(const uint16_t* xp, const uint16_t* hs, const int32_t* tile_e,
                     const int32_t* tile_slot, const int32_t* ntiles, const uint32_t* w1,

@@ -4,13 +4,15 @@
 //                 the Mamba-2 gated norm of the SSM kernel's z) normalised and rounded as
 //                 hsd_linear's prologue does it (the same instruction sequence, so the same
 //                 bits), stored with every 8 inputs in the order of a weight word's nibble
-//                 pairs (0 4 1 5 2 6 3 7), and the sum of every 64-input group as two bf16
-//                 values (hi + lo: 16 bits of the fp32 sum).
+//                 pairs (0 4 1 5 2 6 3 7), and the sum of every 64-input group as three bf16
+//                 values (all 24 bits of the fp32 sum).
 //   k_gemm_q4     y = x W^T, W affine 4-bit group 64 in the stock layout [O, I/8], and, with
 //                 tiles of (token, slot) pairs sorted by expert, every expert's up projection
 //                 with ReLU^2 (a grouped product over gathered rows).
 //   k_gemm_bf16   y = x W^T with a bf16 weight (the router gate, the MTP head's eh_proj).
 #include "hsd_common.h"
+
+#include "gemm.h"
 
 namespace hsd {
 namespace {
@@ -18,6 +20,9 @@ namespace {
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 constexpr uint32_t kBfOne2 = 0x3F803F80u;   // bf16 pair (1, 1)
@@ -34,9 +39,26 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ float lo_f(uint32_t v) { return __uint_as_float(v << 16); }
 __device__ __forceinline__ float hi_f(uint32_t v) { return __uint_as_float(v & 0xFFFF0000u); }
 
+// Offsets past any buffer of the epilogues (the host bounds those to 1 GiB), also added up
+constexpr uint32_t kNoRow = 0x80000000u, kNoCol = 0x40000000u;
+
 // -16 times both values of a bf16 pair (exact: a power of two)
 __device__ __forceinline__ uint32_t neg16(uint32_t v) {
   return __builtin_amdgcn_perm(__float_as_uint(hi_f(v) * -16.0f), __float_as_uint(lo_f(v) * -16.0f), 0x07060302u);
+}
+
+// 16 bytes at a multiple of 4
+struct __attribute__((packed, aligned(4))) Piece {
+  u32x4 v;
+};
+
+// v as the sum of three bf16 values: all 24 bits
+__device__ __forceinline__ void split3(float v, uint16_t (&p)[3]) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    p[k] = f32_to_bf16_bits(v);
+    v -= bf16_bits_to_f32(p[k]);
+  }
 }
 
 // ------------------------------------------------------------------ rows
@@ -147,9 +169,10 @@ __global__ __launch_bounds__(kPT) void k_rows_prep(const void* __restrict__ x_, 
       const int g = t >> 3;
       if ((t & 7) == 0 && g < GP) {
         const float v = t < NW ? s8 : 0.0f;   // groups past the row (up to GP) are zero
-        const uint16_t hi = f32_to_bf16_bits(v);
-        hs[row * 2 * GP + g] = hi;
-        hs[row * 2 * GP + GP + g] = f32_to_bf16_bits(v - bf16_bits_to_f32(hi));
+        uint16_t p[3];
+        split3(v, p);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) hs[(row * 3 + k) * GP + g] = p[k];
       }
     }
   }
@@ -166,45 +189,19 @@ __global__ __launch_bounds__(kPT) void k_rows_prep(const void* __restrict__ x_, 
 // A weight word is one lane's B operand of one MFMA: 8 consecutive inputs as bf16 16 + q (a
 // shift and an and-or per pair), so lane half h takes words 4h .. 4h+3 of a group and the
 // rows' pieces in the same order. Per group acc = sum x (16 + q) starts from zero and
-// y += s acc in fp32; sum_g (b - 16 s) sum(x) starts y: the group sums (hi and lo in the two
-// lane halves) times b and times -16 s, 8 groups per MFMA pair.
+// y += s acc in fp32; sum_g (b - 16 s) sum(x) starts y: the group sums' first and second parts
+// (in the two lane halves) times b and times -16 s and their third parts times both, 8 groups
+// per three MFMAs, so that no bit of the fp32 sums is lost (a third part costs 3 % of the kernel).
 // The matrix cores need 8 instructions per group and 32 x 64 outputs, the vector unit about
 // 100 for the nibbles, the scales' products and the addresses: a wavefront of 64 rows shares
 // the nibbles' part between two row blocks.
-struct GemmArgs {
-  const uint16_t* xp;      // [T, I] prepared rows
-  const uint16_t* hs;      // [T, 2 GP] group sums: hi, lo
-  const uint32_t* w;       // [O, I/8] (expert products: [E, F, I/8])
-  const uint16_t* s;       // [O, I/64]
-  const uint16_t* b;
-  uint16_t* y;
-  int64_t y_ld;
-  const uint16_t* res;
-  int64_t res_ld;
-  // expert products
-  const uint32_t* sw;
-  const uint16_t* ss;
-  const uint16_t* sb;
-  const int32_t* tile_e;
-  const int32_t* tile_slot;
-  const int32_t* ntiles;   // [0]: routed tiles in use
-  uint16_t* hsum;          // nullable, [T * (topk + 1), 2 GPH]: the outputs' group sums, hi | lo
-  int GPH;
-  int nt_routed;           // first shared tile
-  int nt_shared;
-  int T, O, I, GP;
-  int F, FS, topk, E;
-};
-
-enum GemmMode : int { kStore = 0, kResid = 1, kUpRelu2 = 2 };
-
 template <int MT, int MODE>
 __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
   constexpr int MI = MT / 32;
   constexpr int kA = MT * 256, kB = 256 * 64, kS = 256 * 4, kStage = kA + kB + kS;
   __shared__ __attribute__((aligned(1024))) char lds[2 * kStage];
-  __shared__ int drow[MT];         // a tile row's output row (expert products: its offset in y), -1: none
-  __shared__ int srow[MODE == kUpRelu2 ? MT : 1];   // expert products: its (token, slot) index
+  // a tile row's byte offset in y (and in res; expert products: in hsum); kNoRow: none
+  __shared__ __attribute__((aligned(16))) uint32_t drow[MT], erow[MODE == kStore ? 1 : MT];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, kh = lane >> 5;
   const int I = a.I, G = I / 64, NS = I / 128;
@@ -245,9 +242,9 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
       arow[i] = token(ts[8 * (MI * wave + i) + (lane >> 3)]);
     }
     if (tid < MT) {
-      const int s = ts[tid], NR = a.topk * a.F + a.FS;
-      drow[tid] = s < 0 ? -1 : sh ? s * NR + a.topk * a.F : (s / a.topk) * NR + (s % a.topk) * a.F;
-      srow[tid] = s < 0 ? 0 : sh ? s * (a.topk + 1) + a.topk : (s / a.topk) * (a.topk + 1) + s % a.topk;
+      const int s = ts[tid], NR = a.topk * a.F + a.FS, k = sh ? a.topk : max(s, 0) % a.topk, tok = token(s);
+      drow[tid] = s < 0 ? kNoRow : 2u * (uint32_t)(tok * NR + k * a.F);
+      erow[tid] = s < 0 ? kNoRow : 6u * (uint32_t)((tok * (a.topk + 1) + k) * a.GPH);
     }
   } else {
     const int nbm = (a.T + MT - 1) / MT, nbn = (a.O + 255) / 256;
@@ -260,7 +257,11 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
       trow[i] = min(m0 + 32 * i + j, a.T - 1);
       arow[i] = min(m0 + 8 * (MI * wave + i) + (lane >> 3), a.T - 1);
     }
-    if (tid < MT) drow[tid] = m0 + tid < a.T ? m0 + tid : -1;
+    if (tid < MT) {
+      const bool in = m0 + tid < a.T;
+      drow[tid] = in ? (uint32_t)(m0 + tid) * (uint32_t)a.y_ld * 2u : kNoRow;
+      if constexpr (MODE == kResid) erow[tid] = in ? (uint32_t)(m0 + tid) * (uint32_t)a.res_ld * 2u : kNoRow;
+    }
   }
 
   // ---- the ring's loads of one stage by this wavefront: 2 MI KB of rows, 4 KB of nibbles,
@@ -305,7 +306,12 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
   };
   issue(0);
 
-  // ---- y = sum_g (b - 16 s) sum(x), while the first stage is on its way
+  // ---- y = sum_g (b - 16 s) sum(x), while the first stage is on its way: 8 groups at a time,
+  // the next ones' loads in flight. The last 8 end at the row's last group, with zero for the
+  // sums that the 8 before have covered, so that every load is 16 bytes and none leaves the
+  // row (with 4-byte loads clamped to the row 2048 rows of 4096 inputs took 107 us against 89);
+  // rows of fewer than 8 groups take 4 bytes each, pairs past the row its last pair, where
+  // the sums are zero.
   f32x16 y[MI][2];
   {
 #pragma unroll
@@ -314,41 +320,70 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
       for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) y[mi][nt][v] = 0.0f;
-    const uint32_t* brow[2];
-    const uint32_t* srow[2];
+    uint32_t coff[2];
+    const char* hrow[MI];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const size_t col = (size_t)min(n0 + 64 * wave + 32 * nt + j, O - 1);
-      brow[nt] = reinterpret_cast<const uint32_t*>(bp + col * G);
-      srow[nt] = reinterpret_cast<const uint32_t*>(sp + col * G);
-    }
-    for (int c = 0; 8 * c < G; ++c) {
-      uint4 hv[MI], bv[2], sv[2];
+    for (int nt = 0; nt < 2; ++nt) coff[nt] = (uint32_t)min(n0 + 64 * wave + 32 * nt + j, O - 1) * (uint32_t)(2 * G);
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-        hv[mi] = *reinterpret_cast<const uint4*>(a.hs + (size_t)trow[mi] * 2 * a.GP + kh * a.GP + 8 * c);
+    for (int mi = 0; mi < MI; ++mi)
+      hrow[mi] = reinterpret_cast<const char*>(a.hs + (size_t)trow[mi] * 3 * a.GP);
+    const int nc = (G + 7) / 8, o1 = kh * 2 * a.GP, o2 = 4 * a.GP;   // first or second parts by half; third parts
+    u32x4 hv[2][MI], h3[2][MI], bv[2][2], sv[2][2];
+    auto load = [&](int c, int u) {
+      c = min(c, nc - 1);
+      const int g = max(min(8 * c, G - 8), 0), over = (8 * c - g) / 2;   // uniform; pairs already covered
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        uint32_t bw[4], sw[4];
+      for (int mi = 0; mi < MI; ++mi) {
+        hv[u][mi] = reinterpret_cast<const Piece*>(hrow[mi] + o1 + 2 * g)->v;
+        h3[u][mi] = reinterpret_cast<const Piece*>(hrow[mi] + o2 + 2 * g)->v;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {   // pairs past the row re-read its last pair and are zeroed
-          const int p = 4 * c + q, pc = min(p, G / 2 - 1);
-          bw[q] = brow[nt][pc];
-          sw[q] = srow[nt][pc];
-          bw[q] = p < G / 2 ? bw[q] : 0u;
-          sw[q] = p < G / 2 ? neg16(sw[q]) : 0u;
+        for (int q = 0; q < 3; ++q) {
+          hv[u][mi][q] = q < over ? 0u : hv[u][mi][q];
+          h3[u][mi][q] = q < over ? 0u : h3[u][mi][q];
         }
-        bv[nt] = make_uint4(bw[0], bw[1], bw[2], bw[3]);
-        sv[nt] = make_uint4(sw[0], sw[1], sw[2], sw[3]);
       }
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
+      if (G >= 8) {
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
-          const bf16x8 h8 = __builtin_bit_cast(bf16x8, hv[mi]);
-          y[mi][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, __builtin_bit_cast(bf16x8, bv[nt]), y[mi][nt], 0, 0, 0);
-          y[mi][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, __builtin_bit_cast(bf16x8, sv[nt]), y[mi][nt], 0, 0, 0);
+          bv[u][nt] = reinterpret_cast<const Piece*>(reinterpret_cast<const char*>(bp) + 2 * g + coff[nt])->v;
+          sv[u][nt] = reinterpret_cast<const Piece*>(reinterpret_cast<const char*>(sp) + 2 * g + coff[nt])->v;
         }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int o = 4 * min(q, G / 2 - 1);       // uniform
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt) {
+            bv[u][nt][q] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(bp) + o + coff[nt]);
+            sv[u][nt][q] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(sp) + o + coff[nt]);
+          }
+        }
+      }
+    };
+    auto apply = [&](int u) {
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        u32x4 sw;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sw[q] = neg16(sv[u][nt][q]);
+        // the third parts: b in lane half 0, -16 s in half 1
+        const u32x4 bs = kh ? sw : bv[u][nt];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+          const bf16x8 h8 = __builtin_bit_cast(bf16x8, hv[u][mi]);
+          y[mi][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, h3[u][mi]), __builtin_bit_cast(bf16x8, bs), y[mi][nt], 0, 0, 0);
+          y[mi][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, __builtin_bit_cast(bf16x8, bv[u][nt]), y[mi][nt], 0, 0, 0);
+          y[mi][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, __builtin_bit_cast(bf16x8, sw), y[mi][nt], 0, 0, 0);
+        }
+      }
+    };
+    load(0, 0);
+    for (int c = 0; c < nc; c += 2) {
+      load(c + 1, 1);
+      apply(0);
+      if (c + 1 >= nc) break;
+      load(c + 2, 0);
+      apply(1);
     }
   }
 
@@ -401,28 +436,57 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
     }
   }
 
-  // ---- outputs: lane column n, rows 32 mi + 8 (v / 4) + 4 kh + v % 4
-  if constexpr (MODE == kUpRelu2) {
-    // F and FS are multiples of 64, so a wavefront's 64 outputs are one group (or past the
-    // end): h, and its group sum for the down projection, summed over the half-wavefront's
-    // lanes (a fixed order) and written by lanes 0 and 32
-    const int g = n0 / 64 + wave;
-    if (64 * g >= O) return;
+  // ---- outputs: lane column n, rows 32 mi + 8 (v / 4) + 4 kh + v % 4. Buffer stores at 32-bit
+  // offsets, which drop what lies past the buffer: rows and columns that are none have offsets
+  // there, so there is no branch and no 64-bit address per row.
+  const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(a.y, (short)0, (int)a.y_bytes, 0x00020000);
+  uint32_t col[2];
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+  for (int nt = 0; nt < 2; ++nt) {
+    const int n = n0 + 64 * wave + 32 * nt + j;
+    col[nt] = n < O ? 2u * (uint32_t)n : kNoCol;
+  }
+  auto put = [&](uint32_t row, const uint32_t (&u)[2]) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = 32 * mi + 8 * (v >> 2) + 4 * kh + (v & 3), d = drow[row];
-        float hv[2];
+    for (int nt = 0; nt < 2; ++nt) __builtin_amdgcn_raw_buffer_store_b16((short)u[nt], yr, row + col[nt], 0, 0);
+  };
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          const float ub = bf16_bits_to_f32(f32_to_bf16_bits(y[mi][nt][v])), r = ub != ub ? ub : fmaxf(ub, 0.0f);
-          const uint16_t h = f32_to_bf16_bits(r * r);
-          hv[nt] = bf16_bits_to_f32(h);
-          if (d >= 0) a.y[(size_t)d + n0 + 64 * wave + 32 * nt + j] = h;
-        }
+  for (int mi = 0; mi < MI; ++mi) {
+    u32x4 ro[4], eo[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      ro[q] = *reinterpret_cast<const u32x4*>(&drow[32 * mi + 8 * q + 4 * kh]);
+      if constexpr (MODE != kStore) eo[q] = *reinterpret_cast<const u32x4*>(&erow[32 * mi + 8 * q + 4 * kh]);
+    }
+    uint32_t rv[MODE == kResid ? 16 : 1][2];
+    if constexpr (MODE == kResid) {
+      const __amdgpu_buffer_rsrc_t rr =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.res), (short)0, (int)a.res_bytes, 0x00020000);
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          rv[v][nt] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rr, eo[v >> 2][v & 3] + col[nt], 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t p = pack_bf16x2(y[mi][0][v], y[mi][1][v]);
+      if constexpr (MODE == kStore) {
+        put(ro[v >> 2][v & 3], {p & 0xFFFFu, p >> 16});
+      } else if constexpr (MODE == kResid) {
+        const uint32_t r = pack_bf16x2(lo_f(rv[v][0]) + lo_f(p), lo_f(rv[v][1]) + hi_f(p));
+        put(ro[v >> 2][v & 3], {r & 0xFFFFu, r >> 16});
+      } else {
+        // h = square(relu(bf16(u))), NaN kept. F and FS are multiples of 64, so a wavefront's 64
+        // outputs are one group (or past the end): its sum over the half-wavefront's lanes in
+        // a fixed order, written by lanes 0 and 32 for the down projection
+        float r0 = lo_f(p), r1 = hi_f(p);
+        r0 = r0 < 0.0f ? 0.0f : r0;
+        r1 = r1 < 0.0f ? 0.0f : r1;
+        const uint32_t h = pack_bf16x2(r0 * r0, r1 * r1);
+        put(ro[v >> 2][v & 3], {h & 0xFFFFu, h >> 16});
         if (a.hsum) {   // uniform
-          float t = hv[0] + hv[1];
+          float t = lo_f(h) + hi_f(h);
           t += dpp_f32<0xB1>(t);
           t += dpp_f32<0x4E>(t);
           t += dpp_f32<0x141>(t);
@@ -430,34 +494,16 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
           const uint32_t tb = __float_as_uint(t);
           const auto pt = __builtin_amdgcn_permlane16_swap(tb, tb, false, false);
           t = __uint_as_float(pt[0]) + __uint_as_float(pt[1]);
-          if (j == 0 && d >= 0) {
-            uint16_t* hp = a.hsum + (size_t)srow[row] * 2 * a.GPH + g;
-            const uint16_t hi = f32_to_bf16_bits(t);
-            hp[0] = hi;
-            hp[a.GPH] = f32_to_bf16_bits(t - bf16_bits_to_f32(hi));
-          }
+          const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(a.hsum, (short)0, (int)a.hsum_bytes, 0x00020000);
+          uint16_t p3[3];
+          split3(t, p3);
+          const uint32_t off = eo[v >> 2][v & 3] + (j == 0 && col[0] != kNoCol ? 2u * (uint32_t)(n0 / 64 + wave) : kNoCol);
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            __builtin_amdgcn_raw_buffer_store_b16((short)p3[k], hr, off + 2u * (uint32_t)(k * a.GPH), 0, 0);
         }
       }
-    return;
-  }
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    const int n = n0 + 64 * wave + 32 * nt + j;
-    if (n >= O) continue;
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int d = drow[32 * mi + 8 * (v >> 2) + 4 * kh + (v & 3)];
-        if (d < 0) continue;
-        const uint16_t u = f32_to_bf16_bits(y[mi][nt][v]);
-        if constexpr (MODE == kStore) {
-          a.y[(size_t)d * a.y_ld + n] = u;
-        } else {
-          a.y[(size_t)d * a.y_ld + n] =
-              f32_to_bf16_bits(bf16_bits_to_f32(a.res[(size_t)d * a.res_ld + n]) + bf16_bits_to_f32(u));
-        }
-      }
+    }
   }
 }
 
@@ -476,7 +522,7 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
 // union lists (k_gemm in prefill.hip) save nothing for their passes over h.
 struct DownArgs {
   const uint16_t* h;       // [T, topk*F + FS]
-  const uint16_t* hsum;    // [T * (topk + 1), 2 GPH]
+  const uint16_t* hsum;    // [T * (topk + 1), 3 GPH]
   const float* gains;      // [T, topk + 1]
   const uint32_t* w;       // [E, F, D/8]
   const uint16_t* s;       // [E, F/64, D]
@@ -488,6 +534,7 @@ struct DownArgs {
   const int32_t* tile_slot;
   const int32_t* ntiles;
   float* part;             // [T * (topk + 1), D]
+  uint32_t part_bytes;     // below 1 GiB
   int nt_routed, nt_shared, T, D, F, FS, topk, E, GPH;
 };
 
@@ -496,8 +543,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_down(DownArgs a) {
   constexpr int MI = MT / 32, kRing = 3;
   constexpr int kA = MT * 128, kB = 64 * 256, kS = 1024, kStage = kA + kB + kS;
   __shared__ __attribute__((aligned(1024))) char lds[kRing * kStage];
-  __shared__ int srow[MT];
-  __shared__ float grow[MT];
+  __shared__ __attribute__((aligned(16))) uint32_t srow[MT];   // a slot's byte offset in part
+  __shared__ __attribute__((aligned(16))) float grow[MT];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, kh = lane >> 5, D = a.D;
   const int nb = (D + 511) / 512;
@@ -529,7 +576,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_down(DownArgs a) {
   }
   if (tid < MT) {
     const int s = ts[tid];
-    srow[tid] = s < 0 ? -1 : sidx(s);
+    srow[tid] = s < 0 ? kNoRow : 4u * (uint32_t)sidx(s) * (uint32_t)D;
     grow[tid] = a.gains[sidx(s)];
   }
   // weight rows: 4 per load, 16 lanes each; wavefront w loads rows 16 w .. 16 w + 15 of a
@@ -567,7 +614,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_down(DownArgs a) {
   issue(0, 0);
   issue(min(1, G - 1), 1);
 
-  // ---- y = sum_g (b - 16 s) sum(h): the group sums (hi, lo in the lane halves) times b and s
+  // ---- y = sum_g (b - 16 s) sum(h): the group sums (in three parts, as above) times b and
+  // -16 s, 8 groups at a time with the next ones' loads in flight; groups past the last are
+  // zeroed on both sides (their sums are not written)
   f32x16 y[MI][4];
   {
 #pragma unroll
@@ -576,41 +625,67 @@ __global__ __launch_bounds__(256, 2) void k_gemm_down(DownArgs a) {
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) y[mi][i][v] = 0.0f;
-    const int col = min(n0 + 4 * j, D - 4);
-    for (int c = 0; 8 * c < G; ++c) {
-      bf16x8 hv[MI];
+    const int col = min(n0 + 4 * j, D - 4), nc = (G + 7) / 8;
+    const char* hr[MI];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+      hr[mi] = reinterpret_cast<const char*>(a.hsum + (size_t)hrow[mi] * 3 * a.GPH);
+    const int o1 = kh * 2 * a.GPH, o2 = 4 * a.GPH;   // first or second parts by half; third parts
+    u32x4 hv[2][MI], h3[2][MI];
+    u32x2 r[2][2][8];
+    auto load = [&](int c, int u) {
+      c = min(c, nc - 1);
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
-        uint4 u = *reinterpret_cast<const uint4*>(a.hsum + (size_t)hrow[mi] * 2 * a.GPH + kh * a.GPH + 8 * c);
-        const int live = G - 8 * c;   // groups of this chunk (the entries past them are not written)
-        auto keep = [&](uint32_t v, int p) { return 2 * p + 1 < live ? v : 2 * p < live ? v & 0xFFFFu : 0u; };
-        u = make_uint4(keep(u.x, 0), keep(u.y, 1), keep(u.z, 2), keep(u.w, 3));
-        hv[mi] = __builtin_bit_cast(bf16x8, u);
+        hv[u][mi] = *reinterpret_cast<const u32x4*>(hr[mi] + o1 + 16 * c);
+        h3[u][mi] = *reinterpret_cast<const u32x4*>(hr[mi] + o2 + 16 * c);
       }
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {   // b, then -16 s; groups past the last are zeroed on both sides
-        const uint16_t* src = u ? sp : bp;
-        uint2 r[8];
+      for (int q = 0; q < 8; ++q) {
+        const size_t o = (size_t)min(8 * c + q, G - 1) * D + col;
+        r[u][0][q] = *reinterpret_cast<const u32x2*>(bp + o);
+        r[u][1][q] = *reinterpret_cast<const u32x2*>(sp + o);
+      }
+    };
+    auto apply = [&](int c, int u) {
+      const int live = G - 8 * c;                    // groups of this chunk
+      auto keep = [&](uint32_t x, int p) { return 2 * p + 1 < live ? x : 2 * p < live ? x & 0xFFFFu : 0u; };
+      bf16x8 h8[MI], hx[MI];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          r[q] = *reinterpret_cast<const uint2*>(src + (size_t)min(8 * c + q, G - 1) * D + col);
-          if (u) r[q] = make_uint2(neg16(r[q].x), neg16(r[q].y));
-          r[q].x = 8 * c + q < G ? r[q].x : 0u;
-          r[q].y = 8 * c + q < G ? r[q].y : 0u;
-        }
+      for (int mi = 0; mi < MI; ++mi) {
+        h8[mi] = __builtin_bit_cast(
+            bf16x8, u32x4{keep(hv[u][mi][0], 0), keep(hv[u][mi][1], 1), keep(hv[u][mi][2], 2), keep(hv[u][mi][3], 3)});
+        hx[mi] = __builtin_bit_cast(
+            bf16x8, u32x4{keep(h3[u][mi][0], 0), keep(h3[u][mi][1], 1), keep(h3[u][mi][2], 2), keep(h3[u][mi][3], 3)});
+      }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          uint32_t f[4];
+      for (int i = 0; i < 4; ++i) {
+        u32x4 f[3];                                  // b, -16 s, and by lane half for the third parts
 #pragma unroll
-          for (int p = 0; p < 4; ++p) {
-            const uint32_t lo = i < 2 ? r[2 * p].x : r[2 * p].y, hi = i < 2 ? r[2 * p + 1].x : r[2 * p + 1].y;
-            f[p] = (i & 1) ? (lo >> 16) | (hi & 0xFFFF0000u) : (lo & 0xFFFFu) | (hi << 16);
+        for (int p = 0; p < 4; ++p) {
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            uint32_t w = __builtin_amdgcn_perm(r[u][k][2 * p + 1][i >> 1], r[u][k][2 * p][i >> 1],
+                                               (i & 1) ? 0x07060302u : 0x05040100u);
+            if (k) w = neg16(w);
+            f[k][p] = keep(w, p);
           }
-          const bf16x8 bv = __builtin_bit_cast(bf16x8, make_uint4(f[0], f[1], f[2], f[3]));
-#pragma unroll
-          for (int mi = 0; mi < MI; ++mi) y[mi][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hv[mi], bv, y[mi][i], 0, 0, 0);
+          f[2][p] = kh ? f[1][p] : f[0][p];
         }
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            y[mi][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k == 2 ? hx[mi] : h8[mi], __builtin_bit_cast(bf16x8, f[k]), y[mi][i], 0, 0, 0);
       }
+    };
+    load(0, 0);
+    for (int c = 0; c < nc; c += 2) {
+      load(c + 1, 1);
+      apply(c, 0);
+      if (c + 1 >= nc) break;
+      load(c + 2, 0);
+      apply(c + 1, 1);
     }
   }
 
@@ -677,15 +752,21 @@ __global__ __launch_bounds__(256, 2) void k_gemm_down(DownArgs a) {
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // no ring load outlives the workgroup
   if (!active) return;
+  // 16-byte buffer stores at 32-bit offsets (a pad slot's lies past the buffer: dropped)
+  const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(a.part, (short)0, (int)a.part_bytes, 0x00020000);
+  const uint32_t cb = 4u * (uint32_t)(n0 + 4 * j);
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int row = 32 * mi + 8 * (v >> 2) + 4 * kh + (v & 3), si = srow[row];
-      if (si < 0) continue;
-      const float gn = grow[row];
-      *reinterpret_cast<float4*>(a.part + (size_t)si * D + n0 + 4 * j) =
-          make_float4(gn * y[mi][0][v], gn * y[mi][1][v], gn * y[mi][2][v], gn * y[mi][3][v]);
+    for (int q = 0; q < 4; ++q) {
+      const u32x4 ro = *reinterpret_cast<const u32x4*>(&srow[32 * mi + 8 * q + 4 * kh]);
+      const f32x4 gn = *reinterpret_cast<const f32x4*>(&grow[32 * mi + 8 * q + 4 * kh]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int v = 4 * q + i;
+        const f32x4 o = {gn[i] * y[mi][0][v], gn[i] * y[mi][1][v], gn[i] * y[mi][2][v], gn[i] * y[mi][3][v]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), pr, ro[i] + cb, 0, 0);
+      }
     }
 }
 
@@ -888,8 +969,16 @@ extern "C" int hsd_gemm_q4(const uint16_t* xp, const uint16_t* hs, const uint32_
   GemmArgs a{};
   a.xp = xp; a.hs = hs; a.w = w; a.s = s; a.b = b; a.y = y; a.y_ld = y_ld; a.res = res; a.res_ld = res_ld;
   a.T = (int)T; a.O = (int)O; a.I = (int)I; a.GP = (int)group_pitch(I);
+  const int64_t yb = ((T - 1) * y_ld + O) * 2, rb = res ? ((T - 1) * res_ld + O) * 2 : 0;
+  if (yb >= kNoCol || rb >= kNoCol) return set_error(HSD_ERR_SHAPE, "%s: y and res must be below 1 GiB", fn);
+  a.y_bytes = (uint32_t)yb;
+  a.res_bytes = (uint32_t)rb;
   const int64_t nbn = (O + 255) / 256;
   hipStream_t st = as_stream(stream);
+  {
+    const int rr = launch_gemm_rows(fn, a, res ? kResid : kStore, st);   // few rows
+    if (rr != 1) return rr;
+  }
   const bool wide = nbn * ((T + 63) / 64) >= 256;
 #define HSD_GEMM(MT, MODE) \
   hipLaunchKernelGGL((k_gemm_q4<MT, MODE>), dim3((unsigned)(nbn * ((T + MT - 1) / MT))), dim3(256), 0, st, a)
@@ -919,6 +1008,10 @@ extern "C" int hsd_moe_up_gemm(const uint16_t* xp, const uint16_t* hs, const int
   GemmArgs a{};
   a.hsum = hsum;
   a.GPH = (int)group_pitch(F > FS ? F : FS);
+  const int64_t yb = T * (topk * F + FS) * 2, hb = T * (topk + 1) * 6 * a.GPH;
+  if (yb >= kNoCol || hb >= kNoCol) return set_error(HSD_ERR_SHAPE, "%s: hcat and hsum must be below 1 GiB", fn);
+  a.y_bytes = (uint32_t)yb;
+  a.hsum_bytes = hsum ? (uint32_t)hb : 0;
   a.xp = xp; a.hs = hs; a.w = w1; a.s = s1; a.b = b1; a.y = hcat;
   a.sw = sw1; a.ss = ss1; a.sb = sb1; a.tile_e = tile_e; a.tile_slot = tile_slot; a.ntiles = ntiles;
   a.nt_routed = (int)(T * topk / tt + E);
@@ -929,6 +1022,10 @@ extern "C" int hsd_moe_up_gemm(const uint16_t* xp, const uint16_t* hs, const int
   const int64_t most = T * topk / tt + (E < T * topk ? E : T * topk);
   const int64_t grid = most * ((F + 255) / 256) + a.nt_shared * ((FS + 255) / 256);
   if (grid > 0x7FFFFFFF) return set_error(HSD_ERR_SHAPE, "%s: sizes too large", fn);
+  if (tt == 32) {
+    const int rr = launch_gemm_rows(fn, a, kUpRelu2, as_stream(stream));
+    if (rr != 1) return rr;
+  }
   if (tt == 32)
     hipLaunchKernelGGL((k_gemm_q4<32, kUpRelu2>), dim3((unsigned)grid), dim3(256), 0, as_stream(stream), a);
   else
@@ -985,7 +1082,9 @@ extern "C" int hsd_moe_down_gemm(const uint16_t* hcat, const uint16_t* hsum, con
   if (T == 0) return HSD_OK;
   if (!workspace || workspace_bytes < hsd_moe_down_workspace_bytes(T, D, topk))
     return set_error(HSD_ERR_WORKSPACE, "%s: workspace too small", fn);
+  if (T * (topk + 1) * D * 4 >= kNoCol) return set_error(HSD_ERR_SHAPE, "%s: the workspace must be below 1 GiB", fn);
   DownArgs a{};
+  a.part_bytes = (uint32_t)(T * (topk + 1) * D * 4);
   a.h = hcat; a.hsum = hsum; a.gains = gains; a.w = pw; a.s = ps; a.b = pb; a.sw = spw; a.ss = sps; a.sb = spb;
   a.tile_e = tile_e; a.tile_slot = tile_slot; a.ntiles = ntiles; a.part = reinterpret_cast<float*>(workspace);
   a.nt_routed = (int)(T * topk / tt + E);

@@ -27,7 +27,7 @@ constexpr int kTT = 256;  // threads of the tile-order kernel
 // expert its stable rank (ballots below it, in slot order). The unused tiles, the shared
 // tiles and the pads are spread over the workgroups. Counting per workgroup instead of
 // once costs n LDS atomics each, in parallel, against a chain of passes with barriers in
-// one workgroup: 512 tokens 10.9 -> 5.3 us, 2048 tokens 28 -> 8.6 us (128 experts, top-6).
+// one workgroup: 512 tokens 10.9 -> 5.8 us (128 experts, top-6).
 __global__ __launch_bounds__(kTT) void k_tiles(const int32_t* __restrict__ sel, int T, int topk,
                                                int E, int tt, int32_t* __restrict__ tile_e,
                                                int32_t* __restrict__ tile_slot,

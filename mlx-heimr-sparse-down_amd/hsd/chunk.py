@@ -20,12 +20,19 @@ from .prefill import num_tiles
 
 
 def group_pitch(I):
-    """Group sums per row and half: I/64 rounded up to 8."""
+    """Group sums per row and part: I/64 rounded up to 8."""
     return (I // 64 + 7) // 8 * 8
 
 
+def moe_rows(D, F, FS, topk):
+    """The most rows of one moe_up or moe_down call: each of its buffers (h, the group sums, the
+    slots' partial sums) stays below 1 GiB."""
+    row = max(2 * (topk * F + FS), 6 * (topk + 1) * group_pitch(max(F, FS)), 4 * (topk + 1) * D)
+    return max(((1 << 30) - 1) // row, 1)
+
+
 class Rows:
-    """Prepared rows: xp [T, I] bf16 and, for 4-bit weights, the group sums hs [T, 2 GP]."""
+    """Prepared rows: xp [T, I] bf16 and, for 4-bit weights, the group sums hs [T, 3 GP]."""
 
     def __init__(self, xp, hs):
         self.xp, self.hs = xp, hs
@@ -37,7 +44,7 @@ def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
     T, I = x.shape
     kind = N.X_GATED_Z if gated_z else N.X_RMS if norm is not None else N.X_BF16
     xp = torch.empty((T, I), dtype=torch.bfloat16, device=x.device)
-    hs = torch.empty((T, 2 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
+    hs = torch.empty((T, 3 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
     N.call("hsd_rows_prep", x, x.stride(0), kind, norm, float(eps), xp, hs, T, I,
            N.stream(x.device))
     return Rows(xp, hs)
@@ -74,7 +81,7 @@ def moe_up(rows: Rows, tiles, w1, s1, b1, sw1, ss1, sb1, *, topk, tt):
     T, D = rows.xp.shape
     E, F, FS = w1.shape[0], w1.shape[1], sw1.shape[0]
     hcat = torch.empty((T, topk * F + FS), dtype=torch.bfloat16, device=rows.xp.device)
-    hsum = torch.empty((T, topk + 1, 2 * group_pitch(max(F, FS))), dtype=torch.bfloat16, device=rows.xp.device)
+    hsum = torch.empty((T, topk + 1, 3 * group_pitch(max(F, FS))), dtype=torch.bfloat16, device=rows.xp.device)
     N.call("hsd_moe_up_gemm", rows.xp, rows.hs, tiles[0], tiles[1], tiles[2],
            N.as_words(w1), s1, b1, N.as_words(sw1), ss1, sb1, hcat,
            hsum, T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
