@@ -304,8 +304,7 @@ __global__ __launch_bounds__(256) void k_kv_append(const uint16_t* __restrict__ 
 // 64-key tile of K and V is staged in LDS once for four heads. S^T = K Q^T (a lane then holds
 // 32 keys of one query, so the softmax is per lane plus one half-wavefront exchange, and the
 // probabilities are already a B operand), O^T = V^T P^T. The probabilities enter the second
-// product as two bf16 parts (hi + lo: 16 bits of the fp32 value), two MFMAs per fragment, so
-// they lose nothing the bf16 output would show. K rows are stored with their 16-byte pieces
+// product as three bf16 parts (all 24 bits of the fp32 value), three MFMAs per fragment. K rows are stored with their 16-byte pieces
 // swapped by (key % 16), V transposed with 8-byte pieces swapped by (dim / 2 % 16): no bank
 // conflicts. The last query tiles have the most keys and are launched first.
 __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restrict__ qkv, int64_t ld,
@@ -417,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
     for (int d = 0; d < 4; ++d)
 #pragma unroll
       for (int v = 0; v < 16; ++v) o[d][v] *= corr;
-    bf16x8 ph[4], pl[4];                             // 16-key steps: registers 8 (st % 2) .. of block st / 2
+    bf16x8 ph[4], pm[4], pl[4];                      // 16-key steps: registers 8 (st % 2) .. of block st / 2
 #pragma unroll
     for (int st = 0; st < 4; ++st)
 #pragma unroll
@@ -426,7 +425,10 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
         l += pv;
         const __bf16 hi = (__bf16)pv;
         ph[st][v] = hi;
-        pl[st][v] = (__bf16)(pv - (float)hi);
+        const float rest = pv - (float)hi;
+        const __bf16 mid = (__bf16)rest;
+        pm[st][v] = mid;
+        pl[st][v] = (__bf16)(rest - (float)mid);
       }
 #pragma unroll
     for (int st = 0; st < 4; ++st)
@@ -466,6 +468,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
 // dst[i] = prompt[clamp(POS + offset + i)]
 __global__ void k_prompt_tokens(const int32_t* __restrict__ src, int n, const int32_t* __restrict__ seq, int offset,
                                 int count, int32_t* __restrict__ dst) {
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pm[st], o[d], 0, 0, 0);
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < count) dst[i] = src[min(max(seq[HSD_SEQ_POS] + offset + i, 0), n - 1)];
 }
