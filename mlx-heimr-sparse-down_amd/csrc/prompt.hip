@@ -10,6 +10,8 @@
 //   k_prompt_*    token gather and state advance.
 // The prompt has Ttot tokens, of which rows P .. Ttot-1 are new: a row past them (P > 0) is
 // computed but leaves nothing behind.
+#include <type_traits>
+
 #include "hsd_common.h"
 
 namespace hsd {
@@ -19,6 +21,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 // staging registers that go from global memory to LDS unread (an array of the HIP vector
 // structs copied like that stays in scratch memory)
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -92,33 +95,50 @@ __global__ __launch_bounds__(256) void k_conv_rows(const uint16_t* __restrict__ 
 }
 
 // ------------------------------------------------------------------ scan
-// The arithmetic of a row is k_mamba_ssm's (the same fma, product and lane order), so the
-// states and z equal a row-by-row run's. Workgroup = (head, 16 state rows); wavefront w owns
-// state rows 4w .. 4w+3, 16 lanes per row with 8 state elements each, for all rows of the
-// chunk. kTS rows' inputs are staged in LDS at a time, the next ones in registers meanwhile.
-// Bound by the vector unit's issue (about 30 instructions per row and wavefront, one
-// wavefront per SIMD): rows are a serial chain of one fma.
+// The state after every row is k_mamba_ssm's, bit for bit (the same product and fma per
+// element); y = sum_n S C adds in another order. Workgroup = (head, 16 state rows), 8
+// wavefronts; wavefront w owns state rows 2w and 2w + 1, lane l their elements 2l and 2l + 1,
+// for all rows of the chunk: a row's B and C are read from LDS once for both state rows, and
+// two wavefronts per SIMD issue twice as fast as one (an instruction per 2.5 cycles against 5).
+// kTS rows' inputs are staged in LDS at a time, the next ones' in registers meanwhile; after
+// them the 2 x kTS lane sums are added over the lanes by halving: v_permlane32_swap and
+// v_permlane16_swap bring two values' lane halves together, then DPP steps between lanes that
+// keep one value each (70 instructions for 32 sums over 64 lanes).
+// Bound by the serial chain over the rows: vector instructions (a stage is about 500 per
+// wavefront) and LDS reads alternate with one barrier per stage. 2048 rows, 64 heads of 64 x
+// 128: 323 us with 4 wavefronts of 8 elements per lane, one per SIMD; 279 with 8; 221 with the
+// inputs read two stages ahead, a stage's outputs written under the next one's rows and B and C
+// in one LDS read.
 constexpr int kTS = 16;
-__global__ __launch_bounds__(256, 1) void k_scan(
+constexpr int kSW = 8;      // wavefronts
+
+// a + b of two values summed over one lane bit: lanes with the bit clear keep a's sum, the
+// others b's (CTRL: a DPP control that pairs the lanes)
+template <int CTRL>
+__device__ __forceinline__ float halve(float a, float b, bool bit) {
+  const float keep = bit ? b : a, give = bit ? a : b;
+  return keep + dpp_f32<CTRL>(give);
+}
+
+__global__ __launch_bounds__(64 * kSW, 2) void k_scan(
     const float* __restrict__ co, const float* __restrict__ dtA, const uint16_t* __restrict__ cin, int64_t cin_ld,
     const uint16_t* __restrict__ gate, int64_t gate_ld, const float* __restrict__ Dp, float* __restrict__ ssm,
     uint16_t* __restrict__ convs, const int32_t* __restrict__ cur_ptr, const int32_t* __restrict__ pos, int nslab,
     float* __restrict__ z, int64_t z_ld, int T, int Ttot, int H, int P, int G, int32_t* __restrict__ status) {
-  // a lane's 8 B (C) elements as two float4, the 16 lanes' first ones, then their second
-  // ones: consecutive lanes read consecutive 16 bytes (no bank conflicts)
-  __shared__ __attribute__((aligned(16))) f32x4 Bs[2][kTS][2][kN / 8], Cs[2][kTS][2][kN / 8];
-  __shared__ __attribute__((aligned(16))) float xs[2][kTS][kPB];
-  __shared__ float ds[2][kTS][2];
-  __shared__ float ys[kTS][kPB + 1];
+  constexpr int kT = 64 * kSW;
+  __shared__ __attribute__((aligned(16))) f32x4 bc[2][kTS][kN / 2];                  // B and C of elements 2 l, 2 l + 1
+  __shared__ __attribute__((aligned(16))) float xs[2][kTS][kPB], xd[2][kPB / 2][kTS][2];   // x; x dt by state row pair
+  __shared__ __attribute__((aligned(16))) float ds[2][kTS];                          // exp(A dt)
+  __shared__ float ys[2][kTS][kPB + 1];
   const int npb = P / kPB, lb = xcd_remap((int)blockIdx.x, H * npb);
   const int hh = lb / npb, pblk = lb - hh * npb, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int DI = H * P, GN = G * kN, CD = DI + 2 * GN, hpg = H / G, g = hh / hpg;
   const int cur = *cur_ptr, V = valid_rows(*pos, Ttot, T);
   const float Dh = bf16_bits_to_f32(f32_to_bf16_bits(Dp[hh]));
   if ((unsigned)cur >= (unsigned)nslab) {
-    for (int i = tid; i < T * kPB; i += 256)
+    for (int i = tid; i < T * kPB; i += kT)
       z[(size_t)(i / kPB) * z_ld + (size_t)hh * P + pblk * kPB + i % kPB] = __int_as_float(0x7FC00000);
-    for (int i = tid; i < T; i += 256) z[(size_t)i * z_ld + DI + (size_t)hh * npb + pblk] = __int_as_float(0x7FC00000);
+    for (int i = tid; i < T; i += kT) z[(size_t)i * z_ld + DI + (size_t)hh * npb + pblk] = __int_as_float(0x7FC00000);
     if (tid == 0 && status) atomicOr(status, (int32_t)HSD_STATUS_BAD_STATE);
     return;
   }
@@ -127,152 +147,161 @@ __global__ __launch_bounds__(256, 1) void k_scan(
   // channels in one workgroup per group; every read of the old window precedes the writes
   const bool owner = (hh % hpg == 0) && pblk == 0;
   if (V > 0) {
-    const int nch = owner ? kPB + 2 * kN : kPB;
-    uint16_t wv[2][kK - 1];
+    const int nch = owner ? kPB + 2 * kN : kPB, t = min(tid, nch - 1);
+    static_assert(kPB + 2 * kN <= kT, "a channel per thread");
+    const int ch = t < kPB ? hh * P + pblk * kPB + t
+                           : t < kPB + kN ? DI + g * kN + (t - kPB) : DI + GN + g * kN + (t - kPB - kN);
+    uint16_t wv[kK - 1];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int t = min(tid + 256 * u, nch - 1);
-      const int ch = t < kPB ? hh * P + pblk * kPB + t
-                             : t < kPB + kN ? DI + g * kN + (t - kPB) : DI + GN + g * kN + (t - kPB - kN);
-#pragma unroll
-      for (int i = 0; i < kK - 1; ++i) {
-        const int r = V - (kK - 1) + i;
-        wv[u][i] = r < 0 ? convs[((size_t)cur * (kK - 1) + r + kK - 1) * CD + ch] : cin[(size_t)r * cin_ld + ch];
-      }
+    for (int i = 0; i < kK - 1; ++i) {
+      const int r = V - (kK - 1) + i;
+      wv[i] = r < 0 ? convs[((size_t)cur * (kK - 1) + r + kK - 1) * CD + ch] : cin[(size_t)r * cin_ld + ch];
     }
     __syncthreads();
+    if (tid < nch) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int t = tid + 256 * u;
-      if (t < nch) {
-        const int ch = t < kPB ? hh * P + pblk * kPB + t
-                               : t < kPB + kN ? DI + g * kN + (t - kPB) : DI + GN + g * kN + (t - kPB - kN);
-#pragma unroll
-        for (int i = 0; i < kK - 1; ++i) convs[((size_t)dst_slab * (kK - 1) + i) * CD + ch] = wv[u][i];
-      }
+      for (int i = 0; i < kK - 1; ++i) convs[((size_t)dst_slab * (kK - 1) + i) * CD + ch] = wv[i];
     }
   }
-  const int ri = lane >> 4, c8 = lane & 15, pl = 4 * wave + ri, p = pblk * kPB + pl;
-  const size_t slab = (size_t)H * P * kN, soff = ((size_t)hh * P + p) * kN + 8 * c8;
-  float4 S0 = *reinterpret_cast<const float4*>(ssm + (size_t)cur * slab + soff);
-  float4 S1 = *reinterpret_cast<const float4*>(ssm + (size_t)cur * slab + soff + 4);
+  const int pl = 2 * wave;                             // this wavefront's first state row of the 16
+  const size_t slab = (size_t)H * P * kN, soff = ((size_t)hh * P + pblk * kPB + pl) * kN + 2 * lane;
+  f32x2 S[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) S[i] = *reinterpret_cast<const f32x2*>(ssm + (size_t)cur * slab + soff + i * kN);
 
-  // staging: 16 rows x (32 + 32 float4 of B and C, 4 of x) and (dt, exp(A dt))
-  f32x4 rb[4], rx;
-  float rd;
-  uint16_t gv;
-  auto load = [&](int t0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = tid + 256 * i, r = min(t0 + (idx >> 6), T - 1), q = idx & 63;
-      rb[i] = *reinterpret_cast<const f32x4*>(co + (size_t)r * CD + DI + (q < 32 ? 0 : GN) + g * kN + 4 * (q & 31));
-    }
-    rx = *reinterpret_cast<const f32x4*>(co + (size_t)min(t0 + (tid >> 2 & 15), T - 1) * CD + (size_t)hh * P + pblk * kPB +
-                                          4 * (tid & 3));
-    rd = dtA[(size_t)min(t0 + (tid >> 1 & 15), T - 1) * 2 * H + (tid & 1) * H + hh];
-    gv = gate[(size_t)min(t0 + (tid >> 4), T - 1) * gate_ld + (size_t)hh * P + pblk * kPB + (tid & 15)];
+  // staging, two stages ahead: 16 rows x (32 + 32 float4 of B and C, 16 of x) and (dt, exp(A dt))
+  struct Regs {
+    f32x4 rb[2];
+    float rx, rdt, rda;
+    uint16_t gv;
   };
-  auto store = [&](int b) {
+  auto load = [&](Regs& u, int t0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = tid + 256 * i, r = idx >> 6, q = idx & 63;
-      (q < 32 ? Bs[b][r][q & 1] : Cs[b][r][q & 1])[(q & 31) >> 1] = rb[i];
+    for (int i = 0; i < 2; ++i) {
+      const int idx = tid + kT * i, r = min(t0 + (idx >> 6), T - 1), q = idx & 63;
+      u.rb[i] = *reinterpret_cast<const f32x4*>(co + (size_t)r * CD + DI + (q < 32 ? 0 : GN) + g * kN + 4 * (q & 31));
     }
-    if (tid < 64) *reinterpret_cast<f32x4*>(&xs[b][tid >> 2][4 * (tid & 3)]) = rx;
-    if (tid < 32) ds[b][tid >> 1][tid & 1] = rd;
+    const int r = min(t0 + (tid >> 4 & 15), T - 1);
+    u.rx = co[(size_t)r * CD + (size_t)hh * P + pblk * kPB + (tid & 15)];
+    u.rdt = dtA[(size_t)r * 2 * H + hh];
+    u.rda = dtA[(size_t)r * 2 * H + H + hh];
+    u.gv = gate[(size_t)r * gate_ld + (size_t)hh * P + pblk * kPB + (tid & 15)];
   };
-  load(0);
-  store(0);
-  int b = 0;
-  for (int t0 = 0; t0 < T; t0 += kTS, b ^= 1) {
-    const uint16_t gcur = gv;
-    __syncthreads();                               // stage b in LDS, ys read
-    load(t0 + kTS);                                // past the chunk: its last row again, unused
+  auto store = [&](const Regs& u, int b) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = tid + kT * i, r = idx >> 6, q = idx & 63;
+      f32x2* dst = reinterpret_cast<f32x2*>(&bc[b][r][2 * (q & 31)]) + (q >> 5);
+      dst[0] = f32x2{u.rb[i].x, u.rb[i].y};
+      dst[2] = f32x2{u.rb[i].z, u.rb[i].w};
+    }
+    if (tid < 256) {
+      const int r = tid >> 4, c = tid & 15;
+      xs[b][r][c] = u.rx;
+      xd[b][c >> 1][r][c & 1] = u.rx * u.rdt;
+      if (c == 0) ds[b][r] = u.rda;
+    }
+  };
+  // z and the 16 channels' sums of z^2 of the stage at t0, from ys[b] (whole wavefronts)
+  auto finish = [&](int t0, int b, uint16_t gv) {
+    if (tid < 256) {
+      const int r = tid >> 4, c = tid & 15;
+      float o = ys[b][r][c] * silu_f32(bf16_bits_to_f32(gv));
+      if (t0 + r < T) z[(size_t)(t0 + r) * z_ld + (size_t)hh * P + pblk * kPB + c] = o;
+      o = o * o;
+      o += dpp_f32<0xB1>(o);
+      o += dpp_f32<0x4E>(o);
+      o += dpp_f32<0x141>(o);
+      o += dpp_f32<0x140>(o);
+      if (c == 0 && t0 + r < T) z[(size_t)(t0 + r) * z_ld + DI + (size_t)hh * npb + pblk] = o;
+    }
+  };
+  // the stage at t0, in buffer kB: its gate values gv[kB], the next stage's inputs in nx (to
+  // the other buffer at the end), the one's after that on their way to fill
+  uint16_t gv[2];
+  auto stage = [&](int t0, auto B, const Regs& nx, Regs& fill) {
+    constexpr int b = decltype(B)::value;
+    __syncthreads();                               // stage t0 in LDS; the last one's ys complete, its buffer read
+    load(fill, t0 + 2 * kTS);                      // past the chunk: its last row again, unused
+    if (t0) finish(t0 - kTS, b ^ 1, gv[b ^ 1]);
     const int n = min(kTS, T - t0);
-    float yk = 0.0f;
-    // a row's inputs; the next kPF rows' are read while kPF rows are computed (one wavefront
-    // per SIMD: nothing else hides the LDS latency)
-    struct In {
-      f32x4 B0, B1, C0, C1;
-      float x, dt, a;
-    };
-    auto fetch = [&](In& v, int r) {
-      v.B0 = Bs[b][r][0][c8];
-      v.B1 = Bs[b][r][1][c8];
-      v.C0 = Cs[b][r][0][c8];
-      v.C1 = Cs[b][r][1][c8];
-      v.x = xs[b][r][pl];
-      v.dt = ds[b][r][0];
-      v.a = ds[b][r][1];
-    };
-    auto row = [&](const In& v, int r) {
-      const f32x4 B0 = v.B0, B1 = v.B1, C0 = v.C0, C1 = v.C1;
-      const float xdt = v.x * v.dt, a = v.a;
-      S0.x = fmaf(a, S0.x, xdt * B0.x);
-      S0.y = fmaf(a, S0.y, xdt * B0.y);
-      S0.z = fmaf(a, S0.z, xdt * B0.z);
-      S0.w = fmaf(a, S0.w, xdt * B0.w);
-      S1.x = fmaf(a, S1.x, xdt * B1.x);
-      S1.y = fmaf(a, S1.y, xdt * B1.y);
-      S1.z = fmaf(a, S1.z, xdt * B1.z);
-      S1.w = fmaf(a, S1.w, xdt * B1.w);
-      float y = S0.x * C0.x;
-      y = fmaf(S0.y, C0.y, y);
-      y = fmaf(S0.z, C0.z, y);
-      y = fmaf(S0.w, C0.w, y);
-      y = fmaf(S1.x, C1.x, y);
-      y = fmaf(S1.y, C1.y, y);
-      y = fmaf(S1.z, C1.z, y);
-      y = fmaf(S1.w, C1.w, y);
-      y += dpp_f32<0xB1>(y);
-      y += dpp_f32<0x4E>(y);
-      y += dpp_f32<0x141>(y);
-      y += dpp_f32<0x140>(y);
-      yk = c8 == r ? y : yk;                       // lane c8 keeps row c8's (a select, no branch per row)
+    float y[2][kTS];
+    auto row = [&](int r) {
+      const f32x4 v = bc[b][r][lane];
+      const f32x2 x = *reinterpret_cast<const f32x2*>(&xd[b][wave][r][0]);
+      const float a = ds[b][r];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        S[i].x = fmaf(a, S[i].x, x[i] * v.x);
+        S[i].y = fmaf(a, S[i].y, x[i] * v.y);
+        y[i][r] = fmaf(S[i].y, v.w, S[i].x * v.z);
+      }
     };
     auto save = [&]() {
-      float* dst = ssm + (size_t)dst_slab * slab + soff;
-      *reinterpret_cast<float4*>(dst) = S0;
-      *reinterpret_cast<float4*>(dst + 4) = S1;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x2*>(ssm + (size_t)dst_slab * slab + soff + i * kN) = S[i];
     };
     if (n == kTS && (V - 1 < t0 || V - 1 >= t0 + kTS - 1)) {
-      constexpr int kPF = 4;
-      In in[2][kPF];
 #pragma unroll
-      for (int u = 0; u < kPF; ++u) fetch(in[0][u], u);
-#pragma unroll
-      for (int r0 = 0; r0 < kTS; r0 += kPF) {
-#pragma unroll
-        for (int u = 0; u < kPF; ++u)
-          if (r0 + kPF < kTS) fetch(in[(r0 / kPF + 1) & 1][u], r0 + kPF + u);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < kPF; ++u) row(in[(r0 / kPF) & 1][u], r0 + u);
-      }
+      for (int r = 0; r < kTS; ++r) row(r);
       if (V - 1 == t0 + kTS - 1) save();
     } else {
-      for (int r = 0; r < n; ++r) {
-        In v;
-        fetch(v, r);
-        row(v, r);
-        if (t0 + r == V - 1) save();
+#pragma unroll
+      for (int r = 0; r < kTS; ++r) {
+        y[0][r] = y[1][r] = 0.0f;
+        if (r < n) {                               // uniform
+          row(r);
+          if (t0 + r == V - 1) save();
+        }
       }
     }
-    ys[c8][pl] = yk + xs[b][c8][pl] * Dh;
-    __syncthreads();                               // ys complete
-    {
-      const int r = tid >> 4, c = tid & 15;
-      float v = ys[r][c] * silu_f32(bf16_bits_to_f32(gcur));
-      if (r < n) z[(size_t)(t0 + r) * z_ld + (size_t)hh * P + pblk * kPB + c] = v;
-      // the 16 channels' sum of z^2 in channel order, lane 15 of each row
-      v = v * v;
-      float s = __shfl(v, lane & 48, 64);
+    // lane sums: after the swaps lanes 32 .. 63 hold state row 1's values and lane bit 4 the
+    // upper 8 rows of the stage, then lane bits 3, 2, 1 a row each of what is left; lane bit 0
+    // holds both halves of one sum
+    float v[kTS], w[8], u[4], q2[2];
 #pragma unroll
-      for (int i = 1; i < kPB; ++i) s += __shfl(v, (lane & 48) + i, 64);
-      if (c == 0 && r < n) z[(size_t)(t0 + r) * z_ld + DI + (size_t)hh * npb + pblk] = s;
+    for (int r = 0; r < kTS; ++r) {
+      const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[0][r]), __float_as_uint(y[1][r]), false, false);
+      v[r] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
     }
-    store(b ^ 1);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + 8]), false, false);
+      w[r] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = halve<0x140>(w[r], w[r + 4], lane & 8);    // row_mirror
+#pragma unroll
+    for (int r = 0; r < 2; ++r) q2[r] = halve<0x141>(u[r], u[r + 2], lane & 4);   // row_half_mirror
+    float s1 = halve<0x4E>(q2[0], q2[1], lane & 2);                                // quad_perm [2, 3, 0, 1]
+    s1 += dpp_f32<0xB1>(s1);                                                       // quad_perm [1, 0, 3, 2]
+    {
+      const int r = 8 * (lane >> 4 & 1) + 4 * (lane >> 3 & 1) + 2 * (lane >> 2 & 1) + (lane >> 1 & 1);
+      const int c = pl + (lane >> 5);
+      ys[b][r][c] = s1 + xs[b][r][c] * Dh;         // (two lanes write one value)
+    }
+    store(nx, b ^ 1);
+    gv[b ^ 1] = nx.gv;
+  };
+  Regs r0, r1;
+  load(r0, 0);
+  load(r1, kTS);
+  store(r0, 0);
+  gv[0] = r0.gv;
+  int t0 = 0;
+  for (;;) {
+    stage(t0, std::integral_constant<int, 0>{}, r1, r0);
+    if (t0 + kTS >= T) break;
+    t0 += kTS;
+    stage(t0, std::integral_constant<int, 1>{}, r0, r1);
+    if (t0 + kTS >= T) break;
+    t0 += kTS;
   }
+  __syncthreads();
+  if ((t0 / kTS) & 1)
+    finish(t0, 1, gv[1]);
+  else
+    finish(t0, 0, gv[0]);
 }
 
 // ------------------------------------------------------------------ attention
@@ -439,6 +468,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
         const uint2 v1 = *reinterpret_cast<const uint2*>(vt + 128 * dim + 8 * ((4 * st + 2 + kh) ^ sw));
         const bf16x8 vf = __builtin_bit_cast(bf16x8, make_uint4(v0.x, v0.y, v1.x, v1.y));
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph[st], o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pm[st], o[d], 0, 0, 0);
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl[st], o[d], 0, 0, 0);
       }
   }
@@ -468,7 +498,6 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
 // dst[i] = prompt[clamp(POS + offset + i)]
 __global__ void k_prompt_tokens(const int32_t* __restrict__ src, int n, const int32_t* __restrict__ seq, int offset,
                                 int count, int32_t* __restrict__ dst) {
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pm[st], o[d], 0, 0, 0);
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < count) dst[i] = src[min(max(seq[HSD_SEQ_POS] + offset + i, 0), n - 1)];
 }
@@ -523,7 +552,7 @@ extern "C" int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const
                      (int)H, dt_lo, dt_hi);
   int rc = check_launch(fn);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_scan, dim3((unsigned)(H * (P / kPB))), dim3(256), 0, st, co, dtA, conv_in, conv_in_ld, gate, gate_ld,
+  hipLaunchKernelGGL(k_scan, dim3((unsigned)(H * (P / kPB))), dim3(64 * kSW), 0, st, co, dtA, conv_in, conv_in_ld, gate, gate_ld,
                      Dp, ssm_slabs, conv_slabs, cur, pos, (int)nslab, z, z_ld, (int)T, (int)Ttot, (int)H, (int)P, (int)G,
                      dev_status);
   return check_launch(fn);

@@ -1,11 +1,13 @@
 """GPU: the mixers of a prompt chunk (hsd.chunk.scan, hsd.chunk.attention) and the chunked
 prompt against the decode kernels' row-by-row runs.
 
-* scan: bit-identical to mamba.ssm_rows in steps of up to 3 rows (the same arithmetic per row):
-  z, the 16-channel sums, the state and the conv window;
+* scan: the state and the conv window bit-identical to mamba.ssm_rows in steps of up to 3 rows
+  (the same arithmetic per element); z, whose sum over the 128 state elements has another
+  order, within 2^-24 of the terms' sizes per addition (7 + 7 levels against 8 + 4: 2^-20 of
+  sum |S C| covers both), and the 16-channel sums of z^2 accordingly;
 * attention: the cache rows bit-exact, the outputs against float64 attention. The kernel sums
-  exact bf16 products in fp32, keeps 16 bits of each probability and rounds once to bf16:
-  half a bf16 ulp (2^-9) plus 2^-16 of the values' scale, doubled for the fp32 exponentials;
+  exact bf16 products in fp32 and rounds once to bf16: half a bf16 ulp (2^-9) plus 2^-16 of
+  the values' scale, doubled for the fp32 exponentials;
 * prefill: both modes equal bits, and the caches near a run in 3-row steps. Two correct runs
   differ by bf16 roundings (a few 1e-3 after these layers) and, where a token's sixth and
   seventh experts are nearly tied, by one of six gains of that block's update of that row:
@@ -57,7 +59,9 @@ def test_scan_equals_rows(dev, T, cur0, pos0, total):
         zr = M.ssm_rows(m, proj[r:r + n], cb, gated=True)
         full = torch.as_strided(zr, (n, DI + DI // 16), (DI + DI // 16, 1))
         got = torch.as_strided(z, (T, DI + DI // 16), (DI + DI // 16, 1))[r:r + n]
-        assert torch.equal(got.view(torch.int32), full.view(torch.int32)), r
+        scale = full[:, :DI].abs().amax()        # sum |S C| is at most 16 times the largest |z| here
+        assert float((got - full)[:, :DI].abs().max()) <= 2.0 ** -16 * float(scale), r
+        assert float(((got - full)[:, DI:] / full[:, DI:]).abs().max()) <= 2.0 ** -12, r
         N.call("hsd_mamba_select_row", N.ptr(cb.cur), None, n, n, 4, None, N.stream(dev))
     d = (cur0 + V) % 4
     assert int(cb.cur.item()) == d and int(ca.cur.item()) == cur0
