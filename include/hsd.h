@@ -412,9 +412,14 @@ int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const uint16_t* 
                    int64_t P, int64_t N, int64_t G, float dt_lo, float dt_hi, int32_t* dev_status,
                    void* workspace, size_t workspace_bytes, void* stream);
 
-/* hsd_attn_decode for a chunk: the keys and values of rows 0 .. V-1 (qkv's k | v columns) go
- * to the cache at P .., then out [T, HQ*HD] (null: the cache only) = causal attention of
- * every row over keys 0 .. P+r. HD = 128, HQ/HKV a multiple of 4. P < 0 or P + V > smax:
+/* The keys and values of rows 0 .. V-1 (kv [T, 2*HKV*HD]: k | v) to the cache at P .. . P < 0 or
+ * P + V > smax: HSD_STATUS_BAD_STATE and nothing written. */
+int hsd_kv_append(const uint16_t* kv, int64_t kv_ld, int64_t T, int64_t Ttot, uint16_t* k_cache,
+                  uint16_t* v_cache, int64_t smax, const int32_t* pos, int64_t HKV, int64_t HD,
+                  int32_t* dev_status, void* stream);
+
+/* hsd_attn_decode for a chunk: hsd_kv_append of qkv's k | v columns, then out [T, HQ*HD] =
+ * causal attention of every row over keys 0 .. P+r. HD = 128, HQ/HKV a multiple of 4. P < 0 or P + V > smax:
  * HSD_STATUS_BAD_STATE, nothing written to the cache, out 0. */
 int hsd_attn_prompt(const uint16_t* qkv, int64_t qkv_ld, int64_t T, int64_t Ttot, uint16_t* k_cache,
                     uint16_t* v_cache, int64_t smax, const int32_t* pos, uint16_t* out,

@@ -558,24 +558,37 @@ extern "C" int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const
   return check_launch(fn);
 }
 
+extern "C" int hsd_kv_append(const uint16_t* kv, int64_t kv_ld, int64_t T, int64_t Ttot, uint16_t* k_cache,
+                             uint16_t* v_cache, int64_t smax, const int32_t* pos, int64_t HKV, int64_t HD,
+                             int32_t* dev_status, void* stream) {
+  const char* fn = "hsd_kv_append";
+  if (!kv || !k_cache || !v_cache || !pos) return set_error(HSD_ERR_ARG, "%s: null pointer", fn);
+  if (T < 1 || T > (1 << 20) || Ttot < 0 || Ttot > 0x7FFFFFFF || HD != kHD || HKV <= 0 || HKV > 4096 || smax < 1 ||
+      smax > (1 << 24) || kv_ld < 2 * HKV * HD || kv_ld % 8)
+    return set_error(HSD_ERR_SHAPE, "%s: bad sizes", fn);
+  if (((uintptr_t)kv | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15u)
+    return set_error(HSD_ERR_ALIGN, "%s: 16-byte aligned pointers", fn);
+  const int64_t pieces = T * 2 * HKV * 16;
+  hipLaunchKernelGGL(k_kv_append, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, as_stream(stream), kv, kv_ld, k_cache,
+                     v_cache, smax, pos, (int)T, (int)Ttot, (int)HKV, dev_status);
+  return check_launch(fn);
+}
+
 extern "C" int hsd_attn_prompt(const uint16_t* qkv, int64_t qkv_ld, int64_t T, int64_t Ttot, uint16_t* k_cache,
                                uint16_t* v_cache, int64_t smax, const int32_t* pos, uint16_t* out, int64_t out_ld,
                                int64_t HQ, int64_t HKV, int64_t HD, float scale, int32_t* dev_status, void* stream) {
   const char* fn = "hsd_attn_prompt";
-  if (!qkv || !k_cache || !v_cache || !pos) return set_error(HSD_ERR_ARG, "%s: null pointer", fn);
+  if (!qkv || !k_cache || !v_cache || !pos || !out) return set_error(HSD_ERR_ARG, "%s: null pointer", fn);
   if (T < 1 || T > (1 << 20) || Ttot < 0 || Ttot > 0x7FFFFFFF || HD != kHD || HKV <= 0 || HQ <= 0 || HQ % HKV ||
       (HQ / HKV) % 4 || smax < 1 || smax > (1 << 24))
     return set_error(HSD_ERR_SHAPE, "%s: need head dim %d and a multiple of 4 query heads per kv head", fn, kHD);
-  if (qkv_ld < (HQ + 2 * HKV) * HD || qkv_ld % 8 || (out && (out_ld < HQ * HD || out_ld % 8)))
+  if (qkv_ld < (HQ + 2 * HKV) * HD || qkv_ld % 8 || out_ld < HQ * HD || out_ld % 8)
     return set_error(HSD_ERR_SHAPE, "%s: bad row strides", fn);
   if (((uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15u)
     return set_error(HSD_ERR_ALIGN, "%s: 16-byte aligned pointers", fn);
   hipStream_t st = as_stream(stream);
-  const int64_t pieces = T * 2 * HKV * 16;
-  hipLaunchKernelGGL(k_kv_append, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, qkv + HQ * HD, qkv_ld, k_cache,
-                     v_cache, smax, pos, (int)T, (int)Ttot, (int)HKV, dev_status);
-  const int rc = check_launch(fn);
-  if (rc || !out) return rc;
+  const int rc = hsd_kv_append(qkv + HQ * HD, qkv_ld, T, Ttot, k_cache, v_cache, smax, pos, HKV, HD, dev_status, stream);
+  if (rc) return rc;
   hipLaunchKernelGGL(k_attn_prompt, dim3((unsigned)((T + 31) / 32 * (HQ / 4))), dim3(256), 0, st, qkv, qkv_ld, k_cache,
                      v_cache, smax, pos, out, out_ld, (int)T, (int)Ttot, (int)HQ, (int)HKV, scale);
   return check_launch(fn);

@@ -48,6 +48,7 @@ namespace {
   X(hsd_moe_down_gemm) \
   X(hsd_mamba_scan) \
   X(hsd_attn_prompt) \
+  X(hsd_kv_append) \
   X(hsd_prompt_tokens) \
   X(hsd_prompt_advance) \
   X(hsd_prefill_tiles) \

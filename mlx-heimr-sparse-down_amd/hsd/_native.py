@@ -116,6 +116,7 @@ _SIGS = {
                        + [_c_i64] * 6 + [_c_float] * 2 + [_vp, _vp, _c_size, _vp]),
     "hsd_attn_prompt": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _c_i64, _vp, _vp] + [_c_i64] * 4
                         + [_c_float, _vp, _vp]),
+    "hsd_kv_append": (_c_int, [_vp] + [_c_i64] * 3 + [_vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _vp]),
     "hsd_prompt_tokens": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _vp]),
     "hsd_prompt_advance": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp]),
     "hsd_moe_up_gemm": (_c_int, [_vp] * 13 + [_c_i64] * 7 + [_vp]),

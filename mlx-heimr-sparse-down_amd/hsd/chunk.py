@@ -122,12 +122,18 @@ def scan(mixer, proj, cache, pos, total, status=None):
     return z[:, :DI]
 
 
-def attention(qkv, kv, pos, total, *, n_heads, n_kv_heads, head_dim=128, cache_only=False, status=None):
+def attention(qkv, kv, pos, total, *, n_heads, n_kv_heads, head_dim=128, status=None):
     """nn.attention of a chunk: the rows' keys and values into the cache, then causal attention
-    -> [T, HQ*HD] bf16 (None with cache_only)."""
+    -> [T, HQ*HD] bf16."""
     T = qkv.shape[0]
-    out = None if cache_only else torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
+    out = torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
     N.call("hsd_attn_prompt", qkv, qkv.stride(0), T, total, kv.k, kv.v, kv.smax, pos,
-           out, 0 if out is None else out.stride(0), n_heads, n_kv_heads, head_dim, 1.0 / math.sqrt(head_dim),
+           out, out.stride(0), n_heads, n_kv_heads, head_dim, 1.0 / math.sqrt(head_dim),
            status, N.stream(qkv.device))
     return out
+
+
+def kv_append(kvrows, kv, pos, total, *, n_kv_heads, head_dim=128, status=None):
+    """The keys and values of a chunk's rows (kvrows [T, 2*HKV*HD]: k | v) into the cache."""
+    N.call("hsd_kv_append", kvrows, kvrows.stride(0), kvrows.shape[0], total, kv.k, kv.v, kv.smax, pos, n_kv_heads,
+           head_dim, status, N.stream(kvrows.device))

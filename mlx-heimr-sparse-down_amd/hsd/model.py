@@ -199,6 +199,13 @@ class AttnBlock:
         chunk.gemm(chunk.prep(o), self.o_proj, residual=x, out=x)
         return x
 
+    def chunk_cache(self, x, kv: nn.KVCache, pos, total, status=None):
+        """Only the cache rows of chunk: the k and v outputs of the projection."""
+        c, QD = self.cfg, self.cfg.attn_heads * self.cfg.head_dim
+        kvw = nn.QWeight(self.qkv.w[QD:], self.qkv.scales[QD:], self.qkv.biases[QD:])
+        rows = chunk.gemm(chunk.prep(x, norm=self.norm_w, eps=c.eps), kvw)
+        chunk.kv_append(rows, kv, pos, total, n_kv_heads=c.kv_heads, head_dim=c.head_dim, status=status)
+
     def nbytes(self):
         return self.qkv.nbytes() + self.o_proj.nbytes()
 
@@ -348,6 +355,12 @@ class MoEBlock:
         tile nearly every row has a live one). No row's result depends on the zeros of another,
         so both modes are the same bits."""
         c = self.cfg
+        most = chunk.moe_rows(c.hidden, c.moe_inter, c.shared_inter, c.topk)
+        if x.shape[0] > most:
+            out = torch.empty_like(x) if out is None else out
+            for r in range(0, x.shape[0], most):
+                self._chunk(x[r:r + most], tt, out=out[r:r + most])
+            return out
         rows = chunk.prep(x, norm=self.norm_w, eps=c.eps)
         logits = chunk.gemm(rows, self.gate)
         sel, gains = router_topk(logits, self.e_bias, topk=c.topk, routed_scale=c.routed_scale, norm_topk=c.norm_topk)
@@ -355,12 +368,6 @@ class MoEBlock:
         hcat, hsum = chunk.moe_up(rows, tiles, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, topk=c.topk, tt=tt)
         if self.trace is not None:                       # calibration / statistics only
             self.trace.append(float((hcat == 0).float().mean().item()))
-        most = chunk.moe_rows(c.hidden, c.moe_inter, c.shared_inter, c.topk)
-        if x.shape[0] > most:
-            out = torch.empty_like(x) if out is None else out
-            for r in range(0, x.shape[0], most):
-                self._chunk(x[r:r + most], tt, out=out[r:r + most])
-            return out
         return chunk.moe_down(x, hcat, hsum, sel, gains, tiles, self.pw, self.ps, self.pb, self.spw, self.sps, self.spb,
                               topk=c.topk, tt=tt, out=out)
 
@@ -662,8 +669,13 @@ class NemotronModel:
             hd = self.mtp
             pair = nn.head_input(ids, x, self.embedding, hd.enorm, hd.hnorm, eps=c.eps, status=cache.status)
             hx = chunk.gemm(chunk.prep(pair, sums=False), hd.eh_proj)
-            hd.attn.chunk(hx, cache.head_kv, cache.head_pos, T - 1, status=cache.status)
-            hd.moe.chunk(hx)
+            # the head's cache rows are all that a prompt leaves of it: its attention output and
+            # its MoE block feed nothing (they run when their statistics are asked for)
+            if hd.moe.trace is None:
+                hd.attn.chunk_cache(hx, cache.head_kv, cache.head_pos, T - 1, status=cache.status)
+            else:
+                hd.attn.chunk(hx, cache.head_kv, cache.head_pos, T - 1, status=cache.status)
+                hd.moe.chunk(hx)
         N.call("hsd_prompt_advance", seq, T, B, NSLAB, st)
         return x
 
