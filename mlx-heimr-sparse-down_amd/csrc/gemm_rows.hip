@@ -433,12 +433,12 @@ __global__ __launch_bounds__(64 * kWv, 2) void k_gemm_rows_4096(GemmArgs a) {
 // The rules: the expert products in 32-row tiles always; a dense product with rows of up to 3072
 // inputs for up to 64 token rows (10304 outputs: 16 rows 20.5 -> 13.3 us, 32 rows 19.9 -> 16.9,
 // 64 rows 20.7 -> 20.5; 96 rows 21.3 in the ring kernel against 32.2 here: its 64-row tiles
-// share the unpacking); with rows of 4096 inputs always (2688 outputs: 64 rows 31 -> 14 us, 512
-// rows 34.8 -> 33.3, 1024 rows 58.2 -> 50.8, 2048 rows 86.6 -> 85.3).
+// share the unpacking); with rows of 4096 inputs for up to 256 (2688 outputs and a residual:
+// 64 rows 31 -> 14 us, 256 rows 32.4 -> 23.9; 384 rows 33.2 there against 35.7 here).
 int launch_gemm_rows(const char* fn, GemmArgs a, int mode, hipStream_t st) {
   const bool wide = a.I == 4096 && mode != kUpRelu2;
   if (!wide && a.I > 64 * kNG * kWv) return 1;
-  if (mode != kUpRelu2 && (a.O < 32 || a.O % 8 || (!wide && a.T > 64))) return 1;
+  if (mode != kUpRelu2 && (a.O < 32 || a.O % 8 || a.T > (wide ? 256 : 64))) return 1;
   const uintptr_t al = (uintptr_t)a.s | (uintptr_t)a.b | (uintptr_t)a.ss | (uintptr_t)a.sb;
   if (al & 15u) return 1;           // scales and biases are read in 16-byte pieces
 #define HSD_ROWS(K)                                                                                  \
