@@ -806,46 +806,35 @@ __global__ __launch_bounds__(256) void k_sum_resid(const float* __restrict__ par
 }
 
 // ------------------------------------------------------------------ bf16 product
-// A workgroup of KS wavefronts: 32 MI token rows x 32 NI outputs, the inputs split over the
+// A workgroup of 8 wavefronts: 32 token rows x 32 outputs, the inputs split over the
 // wavefronts in contiguous runs of 16 and the partial sums added in wavefront order through
 // LDS. Fragments come straight from global memory (16 bytes per lane; the rows and the
 // weight stay in L2). PERM: the rows are in k_rows_prep's order (the weight's pairs are
-// brought to it with v_perm). The router gate (128 outputs) has few tiles: one 32 x 32 tile
-// per workgroup and the inputs over 8 wavefronts keep its chain of loads short.
-template <int MI, int NI, int KS, bool PERM>
-__global__ __launch_bounds__(64 * KS) void k_gemm_bf16(const uint16_t* __restrict__ x, int64_t x_ld,
-                                                       const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
-                                                       int64_t y_ld, int T, int O, int I) {
-  __shared__ float red[KS > 1 ? KS - 1 : 1][MI * NI * 16][64];
+// brought to it with v_perm). The router gate (128 outputs) has few tiles: small ones and the
+// inputs over 8 wavefronts keep its chain of loads short.
+constexpr int kGW = 8;
+template <bool PERM>
+__global__ __launch_bounds__(64 * kGW) void k_gemm_bf16(const uint16_t* __restrict__ x, int64_t x_ld,
+                                                        const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                                                        int64_t y_ld, int T, int O, int I) {
+  __shared__ float red[kGW - 1][16][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 31, kh = lane >> 5;
-  const int nbm = (T + 32 * MI - 1) / (32 * MI), nbn = (O + 32 * NI - 1) / (32 * NI);
+  const int nbm = (T + 31) / 32, nbn = (O + 31) / 32;
   const int id = xcd_remap((int)blockIdx.x, nbm * nbn);
-  const int nb = id / nbm, m0 = (id - nb * nbm) * 32 * MI, n0 = nb * 32 * NI;
-  const int nk = (I + 15) / 16, per = (nk + KS - 1) / KS, k0 = wave * per, k1 = min(k0 + per, nk);
-  const uint16_t* xr[MI];
-  const uint16_t* wr[NI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) xr[i] = x + (size_t)min(m0 + 32 * i + j, T - 1) * x_ld + 8 * kh;
-#pragma unroll
-  for (int i = 0; i < NI; ++i) wr[i] = w + (size_t)min(n0 + 32 * i + j, O - 1) * I + 8 * kh;
-  f32x16 acc[MI][NI];
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0.0f;
+  const int nb = id / nbm, m0 = (id - nb * nbm) * 32, n0 = nb * 32;
+  const int nk = (I + 15) / 16, per = (nk + kGW - 1) / kGW, k0 = wave * per, k1 = min(k0 + per, nk);
+  const uint16_t* xr = x + (size_t)min(m0 + j, T - 1) * x_ld;
+  const uint16_t* wr = w + (size_t)min(n0 + j, O - 1) * I;
+  f32x16 acc = {};
   // steps in flight; the loop has no branch around a load or its use (the compiler would
   // wait for every load in flight where the paths merge): a step past the run re-reads the
   // last one and is multiplied as zeros
-  constexpr int U = MI * NI == 1 ? 8 : 4;
-  uint4 av[U][MI], bv[U][NI];
+  constexpr int U = 8;
+  uint4 av[U], bv[U];
   auto load = [&](int u, int k) {
-    const size_t o = 16 * (size_t)min(k, nk - 1);
-#pragma unroll
-    for (int i = 0; i < MI; ++i) av[u][i] = *reinterpret_cast<const uint4*>(xr[i] + o);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) bv[u][i] = *reinterpret_cast<const uint4*>(wr[i] + o);
+    const int o = min(16 * k + 8 * kh, I - 8);
+    av[u] = *reinterpret_cast<const uint4*>(xr + o);
+    bv[u] = *reinterpret_cast<const uint4*>(wr + o);
   };
 #pragma unroll
   for (int u = 0; u < U; ++u) load(u, k0 + u);
@@ -854,54 +843,114 @@ __global__ __launch_bounds__(64 * KS) void k_gemm_bf16(const uint16_t* __restric
     for (int u = 0; u < U; ++u) {
       // I % 16 == 8: the upper half of the last step is past the row
       const bool live = k + u < k1 && 16 * (k + u) + 8 * kh < I;
-      bf16x8 ax[MI];
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-        ax[mi] = __builtin_bit_cast(bf16x8, make_uint4(live ? av[u][mi].x : 0u, live ? av[u][mi].y : 0u,
-                                                       live ? av[u][mi].z : 0u, live ? av[u][mi].w : 0u));
-#pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
-        uint4 b = bv[u][ni];
-        if constexpr (PERM)
-          b = make_uint4((b.x & 0xFFFFu) | (b.z << 16), (b.x >> 16) | (b.z & 0xFFFF0000u),
-                         (b.y & 0xFFFFu) | (b.w << 16), (b.y >> 16) | (b.w & 0xFFFF0000u));
-        b = make_uint4(live ? b.x : 0u, live ? b.y : 0u, live ? b.z : 0u, live ? b.w : 0u);
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax[mi], __builtin_bit_cast(bf16x8, b), acc[mi][ni], 0, 0, 0);
-      }
+      const uint4 a = make_uint4(live ? av[u].x : 0u, live ? av[u].y : 0u, live ? av[u].z : 0u, live ? av[u].w : 0u);
+      uint4 b = bv[u];
+      if constexpr (PERM)
+        b = make_uint4((b.x & 0xFFFFu) | (b.z << 16), (b.x >> 16) | (b.z & 0xFFFF0000u),
+                       (b.y & 0xFFFFu) | (b.w << 16), (b.y >> 16) | (b.w & 0xFFFF0000u));
+      b = make_uint4(live ? b.x : 0u, live ? b.y : 0u, live ? b.z : 0u, live ? b.w : 0u);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
       load(u, k + U + u);
     }
   }
-  if constexpr (KS > 1) {
-    if (wave > 0) {
+  if (wave > 0) {
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
+    for (int v = 0; v < 16; ++v) red[wave - 1][v][lane] = acc[v];
+  }
+  __syncthreads();
+  if (wave > 0) return;
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
+  for (int s = 0; s < kGW - 1; ++s)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) red[wave - 1][(mi * NI + ni) * 16 + v][lane] = acc[mi][ni][v];
+    for (int v = 0; v < 16; ++v) acc[v] += red[s][v][lane];
+  const int n = n0 + j;
+  if (n >= O) return;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int r = m0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+    if (r < T) y[(size_t)r * y_ld + n] = f32_to_bf16_bits(acc[v]);
+  }
+}
+
+// Many rows of many outputs (the MTP head's eh_proj on a long prompt): 128 token rows x 128
+// outputs per workgroup, 64 x 64 per wavefront. 64 inputs of both sides are brought to LDS by
+// direct loads into a ring of two stages, the rows' 16-byte pieces swapped by (row % 8) in the
+// source address: half of what 64 x 64 tiles took from L2, and no wavefront waits on fragments
+// of its own. 2048 rows, 5376 -> 2688: 237 -> 79 us (750 TFLOP/s); the rest is a last wave of 80
+// workgroups beside 256 CUs and the loop's serial stages (54 us however few the tiles).
+constexpr int kTileM = 128;
+template <bool PERM>
+__global__ __launch_bounds__(256, 2) void k_gemm_bf16_tiles(const uint16_t* __restrict__ x, int64_t x_ld,
+                                                            const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                                                            int64_t y_ld, int T, int O, int I) {
+  constexpr int kA = kTileM * 128, kStage = 2 * kA;   // 64 inputs of the rows, then of the outputs
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kStage];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, kh = lane >> 5, NS = I / 64;
+  const int nbm = (T + kTileM - 1) / kTileM, nbn = (O + kTileM - 1) / kTileM;
+  const int id = xcd_remap((int)blockIdx.x, nbm * nbn);
+  const int nb = id / nbm, m0 = (id - nb * nbm) * kTileM, n0 = nb * kTileM;
+  // this wavefront's loads: 4 of 8 rows and 4 of 8 outputs (past the end: the last one again)
+  const char *asrc[4], *bsrc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 8 * (4 * wave + i) + (lane >> 3), pc = 16 * ((lane & 7) ^ (lane >> 3));
+    asrc[i] = reinterpret_cast<const char*>(x + (size_t)min(m0 + r, T - 1) * x_ld) + pc;
+    bsrc[i] = reinterpret_cast<const char*>(w + (size_t)min(n0 + r, O - 1) * I) + pc;
+  }
+  const uint32_t lbase = (uint32_t)(uintptr_t)(lds_void_t*)lds;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  auto load16 = [&](uint32_t dst, const char* src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
+                 : "memory", "m0");
+  };
+#pragma clang diagnostic pop
+  auto issue = [&](int st) {
+    const uint32_t base = lbase + (uint32_t)(st & 1) * kStage + 4096u * (uint32_t)wave;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      load16(base + 1024u * i, asrc[i] + 128 * (size_t)st);
+      load16(base + kA + 1024u * i, bsrc[i] + 128 * (size_t)st);
     }
-    __syncthreads();
-    if (wave > 0) return;
+  };
+  issue(0);
+  const int wm = 64 * (wave & 1), wn = 64 * (wave >> 1);
+  f32x16 acc[2][2] = {};
+  for (int st = 0; st < NS; ++st) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wavefront's part of stage st is in
+    lds_barrier();                        // everyone's, and the other slot has been read
+    if (st + 1 < NS) issue(st + 1);
+    const char* base = lds + (st & 1) * kStage;
 #pragma unroll
-    for (int s = 0; s < KS - 1; ++s)
+    for (int s = 0; s < 4; ++s) {
+      bf16x8 av[2], bv[2];
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
+      for (int i = 0; i < 2; ++i) {
+        const int off = 128 * (32 * i + j) + 16 * ((2 * s + kh) ^ (j & 7));
+        av[i] = *reinterpret_cast<const bf16x8*>(base + 128 * wm + off);
+        u32x4 b = *reinterpret_cast<const u32x4*>(base + kA + 128 * wn + off);
+        if constexpr (PERM)
+          b = u32x4{(b.x & 0xFFFFu) | (b.z << 16), (b.x >> 16) | (b.z & 0xFFFF0000u),
+                    (b.y & 0xFFFFu) | (b.w << 16), (b.y >> 16) | (b.w & 0xFFFF0000u)};
+        bv[i] = __builtin_bit_cast(bf16x8, b);
+      }
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
+      for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) acc[mi][ni][v] += red[s][(mi * NI + ni) * 16 + v][lane];
+        for (int ni = 0; ni < 2; ++ni)
+          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi], bv[ni], acc[mi][ni], 0, 0, 0);
+    }
   }
 #pragma unroll
-  for (int ni = 0; ni < NI; ++ni) {
-    const int n = n0 + 32 * ni + j;
+  for (int ni = 0; ni < 2; ++ni) {
+    const int n = n0 + wn + 32 * ni + j;
     if (n >= O) continue;
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int r = m0 + 32 * mi + 8 * (v >> 2) + 4 * kh + (v & 3);
+        const int r = m0 + wm + 32 * mi + 8 * (v >> 2) + 4 * kh + (v & 3);
         if (r < T) y[(size_t)r * y_ld + n] = f32_to_bf16_bits(acc[mi][ni][v]);
       }
   }
@@ -1042,15 +1091,16 @@ extern "C" int hsd_gemm_bf16(const uint16_t* x, int64_t x_ld, int permuted, cons
   if (((uintptr_t)x | (uintptr_t)w) & 15u) return set_error(HSD_ERR_ALIGN, "%s: x and w must be 16-byte aligned", fn);
   if (T == 0) return HSD_OK;
   hipStream_t st = as_stream(stream);
-#define HSD_GB(MI, NI, KS, P)                                                                                     \
-  hipLaunchKernelGGL((k_gemm_bf16<MI, NI, KS, P>),                                                                \
-                     dim3((unsigned)(((T + 32 * MI - 1) / (32 * MI)) * ((O + 32 * NI - 1) / (32 * NI)))), dim3(64 * KS), \
-                     0, st, x, x_ld, w, y, y_ld, (int)T, (int)O, (int)I)
-  const int64_t big = ((T + 63) / 64) * ((O + 63) / 64);
-  if (big >= 512) {
-    if (permuted) HSD_GB(2, 2, 1, true); else HSD_GB(2, 2, 1, false);
+#define HSD_GB(K, GRID, BLOCK)                                                                               \
+  hipLaunchKernelGGL((K), dim3((unsigned)(GRID)), dim3(BLOCK), 0, st, x, x_ld, w, y, y_ld, (int)T, (int)O, (int)I)
+  // the tiled kernel from 32 tiles on (5376 -> 2688: 128 rows, 21 tiles, 54 us against 48; 256
+  // rows, 42 tiles, 54 against 69; 512 rows 54 against 133); it steps by 64 inputs
+  const int64_t tiles = ((T + kTileM - 1) / kTileM) * ((O + kTileM - 1) / kTileM);
+  if (tiles >= 32 && I % 64 == 0) {
+    if (permuted) HSD_GB(k_gemm_bf16_tiles<true>, tiles, 256); else HSD_GB(k_gemm_bf16_tiles<false>, tiles, 256);
   } else {
-    if (permuted) HSD_GB(1, 1, 8, true); else HSD_GB(1, 1, 8, false);
+    const int64_t small = ((T + 31) / 32) * ((O + 31) / 32);
+    if (permuted) HSD_GB(k_gemm_bf16<true>, small, 512); else HSD_GB(k_gemm_bf16<false>, small, 512);
   }
 #undef HSD_GB
   return check_launch(fn);

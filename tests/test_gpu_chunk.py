@@ -60,6 +60,18 @@ def test_gemm_q4(dev, T, O, I):
     assert close(chunk.gemm(chunk.prep(x, norm=nw, sums=False), Wb), refb)
 
 
+@pytest.mark.parametrize("T", [1, 33, 129, 400])
+@pytest.mark.parametrize("O,I,sums", [(40, 24, False), (128, 640, True), (1312, 192, True), (1312, 192, False),
+                                      (4100, 64, False)])
+def test_gemm_bf16(dev, T, O, I, sums):
+    """Both bf16 kernels (few and many tiles, the last one of each side cut), rows in either order."""
+    W = nn.QWeight(rand(dev, O, O, I).to(torch.bfloat16))
+    x = rand(dev, T, T, I).to(torch.bfloat16)
+    y = chunk.gemm(chunk.prep(x, sums=sums), W).double()
+    ref = x.double() @ W.w.double().t()
+    assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.abs().max()).all())
+
+
 @pytest.mark.parametrize("T,tt", [(1, 32), (5, 32), (33, 64), (150, 32), (150, 64), (700, 64)])
 def test_moe_up(dev, T, tt):
     E, D, F, FS, K = 16, 256, 192, 320, 3
