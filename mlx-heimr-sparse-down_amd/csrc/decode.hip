@@ -44,7 +44,7 @@ constexpr int kThreads = kGPW * kWPC * kRS;
 constexpr int kDC = kWPC * 8;            // outputs per D chunk
 constexpr int kL1 = kThreads / kDC;      // first-level sub-sums per output
 constexpr int kRowBatch = 16;            // rows per team per batch (a phase has 32 rows), / W
-constexpr int kWideRows = 2;             // token rows from which a lane takes two words
+constexpr int kWideRows = 4;             // token rows from which a lane takes two words
 
 struct Geom {
   int D, F, FS, topk, E, NR, NW;
@@ -84,10 +84,11 @@ template <> __device__ __forceinline__ bool live_bits<HSD_DT_F32>(float v) { ret
 // W: weight words per lane (a D chunk is 128 W outputs). The kernel is bound by its vector
 // instructions (two per weight, and about as many again per row and word for the list entry,
 // the activation, the address and the load's select), which two words per lane share between 16
-// outputs. The sums' order is the same. One call, one word -> two words (2688 outputs, 10 % of
-// 14848 inputs live), us: 1 row 6.7 -> 6.9, 2 rows 8.7 -> 8.4, 3 rows 10.2 -> 9.2, 8 rows
-// 18.2 -> 15.1, 32 rows 53.3 -> 41.3, 64 rows 101 -> 77: one row, where half the workgroups
-// leave the chip short, keeps one word.
+// outputs. The sums' order is the same. One call of 23 layers' (2688 outputs, 10 % of 14848
+// inputs live), one word -> two words, us: 4 rows 12.5 -> 11.8; one layer's again and again: 1
+// row 6.7 -> 6.9, 8 rows 18.2 -> 15.1, 32 rows 53.3 -> 41.3, 64 rows 101 -> 77. Three rows: 10.5
+// -> 10.4, but a speculative step around them 1.649 -> 1.657 ms (half the workgroups leave the
+// chip short while other kernels' tails run), so they keep one word.
 template <int HDT, int W>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(W > 1 ? 5 : HDT == HSD_DT_F32 ? 7 : 8, W > 1 ? 8 : HDT == HSD_DT_F32 ? 7 : 8))) void k_sparse_down_part(

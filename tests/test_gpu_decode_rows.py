@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 F, FS, TOPK, E = 128, 192, 3, 5
 
 
-@pytest.mark.parametrize("B", [2, 3, 9])
+@pytest.mark.parametrize("B", [3, 4, 9])
 @pytest.mark.parametrize("D", [128, 256, 384, 640])
 @pytest.mark.parametrize("off", [0, 1])
 def test_rows_equal_single_rows(dev, B, D, off):
