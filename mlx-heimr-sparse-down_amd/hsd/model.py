@@ -337,7 +337,11 @@ class MoEBlock:
         union of live rows (tiles, unions and the GEMM on the device)."""
         from . import prefill as P
         c = self.cfg
-        if c.hidden % 128 == 0 and x.shape[0] > CHUNK_MIN:
+        if c.hidden % 128 == 0 and c.hidden <= 3072 and x.shape[0] > CHUNK_MIN:
+            if x.dim() != 2 or x.shape[1] != c.hidden or x.dtype != torch.bfloat16:
+                raise N.HSDError(f"prefill takes bf16 rows of {c.hidden} values")
+            if tt not in (32, 64):
+                raise N.HSDError(f"tt is {tt}: tiles have 32 or 64 slots")
             return self._chunk(N.contig(x), tt)
         hcat, sel, gains = self._front_packed(x)
         tiles = P.build_tiles(sel, c.n_experts, tt)
