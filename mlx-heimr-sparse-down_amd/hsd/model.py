@@ -35,7 +35,13 @@ from . import chunk, layout, mamba as M, nn
 from .moe import route_up_relu2, router_topk, up_relu2
 
 NSLAB = 4          # Mamba checkpoint ring: a verify of up to 3 rows
-CHUNK_MIN = 4      # more token rows than this run as a chunk on the matrix cores
+# MoEBlock.prefill_sparse runs more token rows than this on the matrix cores with every down row
+# read (_chunk); up to it an expert has about one token, so its tile's union of live rows is short
+# and the decode front end reads no expert twice. One block of 128 experts, top-6, 90 % zeros,
+# union lists against _chunk, us: 5 rows 102 / 114, 8 rows 119 / 121, 10 rows 131 / 133, 12 rows
+# 141 / 142, 16 rows 161 / 150, 24 rows 201 / 180, 64 rows 370 / 206 (six blocks in turn: 5 rows
+# 105 / 118, 10 rows 134 / 137, 12 rows 144 / 142, 16 rows 166 / 151).
+CHUNK_MIN = 12
 CHUNK_ROWS = 2048  # prompt rows per chunk (the reference's chunk, model.py:259)
 ROWS = (1, 3)      # row counts with preallocated buffers: decode, verify / prefill steps
 
@@ -337,11 +343,11 @@ class MoEBlock:
         union of live rows (tiles, unions and the GEMM on the device)."""
         from . import prefill as P
         c = self.cfg
-        if c.hidden % 128 == 0 and c.hidden <= 3072 and x.shape[0] > CHUNK_MIN:
-            if x.dim() != 2 or x.shape[1] != c.hidden or x.dtype != torch.bfloat16:
-                raise N.HSDError(f"prefill takes bf16 rows of {c.hidden} values")
-            if tt not in (32, 64):
-                raise N.HSDError(f"tt is {tt}: tiles have 32 or 64 slots")
+        if x.dim() != 2 or x.shape[1] != c.hidden or x.dtype != torch.bfloat16:
+            raise N.HSDError(f"prefill takes bf16 rows of {c.hidden} values")
+        if tt not in (32, 64):
+            raise N.HSDError(f"tt is {tt}: tiles have 32 or 64 slots")
+        if x.shape[0] > CHUNK_MIN and c.hidden % 128 == 0 and c.hidden <= 3072:
             return self._chunk(N.contig(x), tt)
         hcat, sel, gains = self._front_packed(x)
         tiles = P.build_tiles(sel, c.n_experts, tt)

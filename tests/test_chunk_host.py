@@ -9,12 +9,13 @@ from hsd import model as Mdl
 
 @pytest.mark.parametrize("rows,shape,dtype,tt", [
     (5, (5, 2688), torch.float16, 32), (64, (64, 2688), torch.float32, 32), (5, (5, 2560), torch.bfloat16, 32),
-    (5, (5, 1, 2688), torch.bfloat16, 32), (5, (5, 2688), torch.bfloat16, 16), (5, (5, 2688), torch.bfloat16, 0)])
+    (5, (5, 1, 2688), torch.bfloat16, 32), (5, (5, 2688), torch.bfloat16, 16), (5, (5, 2688), torch.bfloat16, 0),
+    (2, (2, 2688), torch.float16, 32), (64, (64, 2688), torch.bfloat16, 48)])
 def test_prefill_refuses(rows, shape, dtype, tt):
     blk = Mdl.MoEBlock.__new__(Mdl.MoEBlock)
     blk.cfg = Mdl.ModelConfig()
     assert blk.cfg.hidden == 2688
-    with pytest.raises(N.HSDError):
+    with pytest.raises(N.HSDError, match="bf16 rows of 2688|slots"):
         blk.prefill_sparse(torch.zeros(shape, dtype=dtype), tt)
 
 

@@ -1,0 +1,43 @@
+"""GPU: MoEBlock.prefill_sparse on both sides of its rule. Up to CHUNK_MIN rows its bits are those
+of the front end and the down projection over each tile's union of live rows; above, the two
+paths differ by fp32 summation orders: a bf16 rounding of h (2^-9 relative, squared) in some of
+a row's neurons and one of the projection, far below 2^-6 of the update."""
+import pytest
+import torch
+
+from hsd import model as Mdl
+from hsd import prefill as P
+
+pytestmark = pytest.mark.gpu
+CFG = Mdl.ModelConfig(hidden=512, n_experts=16, topk=3, moe_inter=256, shared_inter=512)
+
+
+def block(dev):
+    return Mdl.MoEBlock(CFG, Mdl._Init(3, dev))
+
+
+def rows(dev, T):
+    g = torch.Generator(device=dev)
+    g.manual_seed(T)
+    return torch.randn((T, CFG.hidden), device=dev, generator=g).to(torch.bfloat16)
+
+
+def by_union(blk, x, tt):
+    h, sel, gains = blk._front_packed(x)
+    tiles = P.build_tiles(sel, CFG.n_experts, tt)
+    kw = dict(F=CFG.moe_inter, FS=CFG.shared_inter, topk=CFG.topk, E=CFG.n_experts, tt=tt)
+    union = P.build_union(h, *tiles, **kw)
+    y = P.sparse_down_prefill(h, sel, gains, blk.pw, blk.ps, blk.pb, blk.spw, blk.sps, blk.spb, D=CFG.hidden,
+                              tiles=tiles, union=union, **kw)
+    return x + y.to(x.dtype)
+
+
+@pytest.mark.parametrize("tt", [32, 64])
+@pytest.mark.parametrize("T", [1, 4, 5, 12, 13, 40])
+def test_rule(dev, T, tt):
+    blk, x = block(dev), rows(dev, T)
+    y, ref = blk.prefill_sparse(x, tt), by_union(blk, x, tt)
+    if T <= 12:
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+    else:
+        assert float((y.double() - ref.double()).norm()) <= 2.0 ** -6 * float((ref.double() - x.double()).norm())
