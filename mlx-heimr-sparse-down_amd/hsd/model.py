@@ -358,7 +358,7 @@ class MoEBlock:
                                   tiles=tiles, union=union)
         return x + y.to(x.dtype)
 
-    def _chunk(self, x, tt, out=None):
+    def _chunk(self, x, tt, out=None, trace=None):
         """A prompt chunk's rows on the matrix cores (hsd.chunk): the projections run over the
         tiles of (token, slot) pairs sorted by expert, so an expert's weights are read once
         per tile and not once per token, and every down row of a tile (with the tokens of a
@@ -369,15 +369,15 @@ class MoEBlock:
         if x.shape[0] > most:
             out = torch.empty_like(x) if out is None else out
             for r in range(0, x.shape[0], most):
-                self._chunk(x[r:r + most], tt, out=out[r:r + most])
+                self._chunk(x[r:r + most], tt, out=out[r:r + most], trace=trace)
             return out
         rows = chunk.prep(x, norm=self.norm_w, eps=c.eps)
         logits = chunk.gemm(rows, self.gate)
         sel, gains = router_topk(logits, self.e_bias, topk=c.topk, routed_scale=c.routed_scale, norm_topk=c.norm_topk)
         tiles = chunk.moe_tiles(sel, c.n_experts, tt)
         hcat, hsum = chunk.moe_up(rows, tiles, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, topk=c.topk, tt=tt)
-        if self.trace is not None:                       # calibration / statistics only
-            self.trace.append(float((hcat == 0).float().mean().item()))
+        if trace is not None:                            # calibration / statistics only
+            trace.append(float((hcat == 0).float().mean().item()))
         return chunk.moe_down(x, hcat, hsum, sel, gains, tiles, self.pw, self.ps, self.pb, self.spw, self.sps, self.spb,
                               topk=c.topk, tt=tt, out=out)
 
@@ -387,7 +387,7 @@ class MoEBlock:
         products of 128 experts, top-6, 32- against 64-slot tiles: 512 rows 273 against 332 us,
         768 rows 390 against 333)."""
         c = self.cfg
-        return self._chunk(x, 64 if x.shape[0] * c.topk >= 32 * c.n_experts else 32, out=x)
+        return self._chunk(x, 64 if x.shape[0] * c.topk >= 32 * c.n_experts else 32, out=x, trace=self.trace)
 
     def nbytes(self):
         t = [self.gate.w, self.w1, self.s1, self.b1, self.sw1, self.ss1, self.sb1, self.pw, self.ps, self.pb,

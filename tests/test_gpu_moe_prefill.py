@@ -41,3 +41,15 @@ def test_rule(dev, T, tt):
         assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
     else:
         assert float((y.double() - ref.double()).norm()) <= 2.0 ** -6 * float((ref.double() - x.double()).norm())
+
+
+@pytest.mark.parametrize("T", [12, 13])
+def test_leaves_no_statistics(dev, T):
+    """The zero fractions of a layer's `trace` are those of the model's own rows: a call of the
+    block by itself adds none (and reads nothing back to the host)."""
+    blk = block(dev)
+    blk.trace = []
+    blk.prefill_sparse(rows(dev, T))
+    assert blk.trace == []
+    blk.chunk(rows(dev, T))
+    assert len(blk.trace) == 1
