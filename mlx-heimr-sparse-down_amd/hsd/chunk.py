@@ -83,8 +83,8 @@ def moe_up(rows: Rows, tiles, w1, s1, b1, sw1, ss1, sb1, *, topk, tt):
     hcat = torch.empty((T, topk * F + FS), dtype=torch.bfloat16, device=rows.xp.device)
     hsum = torch.empty((T, topk + 1, 3 * group_pitch(max(F, FS))), dtype=torch.bfloat16, device=rows.xp.device)
     N.call("hsd_moe_up_gemm", rows.xp, rows.hs, tiles[0], tiles[1], tiles[2],
-           N.as_words(w1), s1, b1, N.as_words(sw1), ss1, sb1, hcat,
-           hsum, T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
+           N.as_words(N.contig(w1)), N.contig(s1), N.contig(b1), N.as_words(N.contig(sw1)), N.contig(ss1),
+           N.contig(sb1), hcat, hsum, T, D, F, FS, topk, E, tt, N.stream(rows.xp.device))
     return hcat, hsum
 
 
@@ -97,7 +97,8 @@ def moe_down(x, hcat, hsum, sel, gains, tiles, pw, ps, pb, spw, sps, spb, *, top
     nb = N.call("hsd_moe_down_workspace_bytes", T, D, topk)
     ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
     N.call("hsd_moe_down_gemm", hcat, hsum, sel, gains, tiles[0], tiles[1],
-           tiles[2], N.as_words(pw), ps, pb, N.as_words(spw), sps, spb,
+           tiles[2], N.as_words(N.contig(pw)), N.contig(ps), N.contig(pb), N.as_words(N.contig(spw)), N.contig(sps),
+           N.contig(spb),
            x, x.stride(0), y, y.stride(0), T, D, F, FS, topk, E, tt, ws, nb, N.stream(x.device))
     return y
 

@@ -53,3 +53,21 @@ def test_leaves_no_statistics(dev, T):
     assert blk.trace == []
     blk.chunk(rows(dev, T))
     assert len(blk.trace) == 1
+
+
+WEIGHTS = ("w1", "s1", "b1", "sw1", "ss1", "sb1", "pw", "ps", "pb", "spw", "sps", "spb")
+
+
+@pytest.mark.parametrize("T", [12, 40])
+def test_strided_weights(dev, T):
+    """Weights that are views of wider tensors (a checkpoint's fused ones) count like their
+    contiguous copies."""
+    blk, x = block(dev), rows(dev, T)
+    want = blk.prefill_sparse(x)
+    for n in WEIGHTS:
+        t = getattr(blk, n)
+        wide = torch.zeros((*t.shape[:-1], 2 * t.shape[-1]), dtype=t.dtype, device=dev)
+        wide[..., :t.shape[-1]] = t
+        setattr(blk, n, wide[..., :t.shape[-1]])
+        assert not getattr(blk, n).is_contiguous()
+        assert torch.equal(blk.prefill_sparse(x).view(torch.int16), want.view(torch.int16)), n
