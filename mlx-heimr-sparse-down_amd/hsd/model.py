@@ -216,6 +216,11 @@ class AttnBlock:
         return self.qkv.nbytes() + self.o_proj.nbytes()
 
 
+def _aligned(*tensors):
+    """Every tensor's kernel input at a multiple of 16 bytes (a strided one is copied first)."""
+    return all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in tensors)
+
+
 class MoEBlock:
     """hsd/model.py:53-175 MoEBlock: router (bf16 gate, sigmoid scores + selection bias,
     top-k, normalised and scaled gains), the routed and shared 4-bit up projections with
@@ -347,7 +352,7 @@ class MoEBlock:
             raise N.HSDError(f"prefill takes bf16 rows of {c.hidden} values")
         if tt not in (32, 64):
             raise N.HSDError(f"tt is {tt}: tiles have 32 or 64 slots")
-        if x.shape[0] > CHUNK_MIN and c.hidden % 128 == 0 and c.hidden <= 3072:
+        if x.shape[0] > CHUNK_MIN and self.chunkable():
             return self._chunk(N.contig(x), tt)
         hcat, sel, gains = self._front_packed(x)
         tiles = P.build_tiles(sel, c.n_experts, tt)
@@ -357,6 +362,13 @@ class MoEBlock:
                                   F=c.moe_inter, FS=c.shared_inter, D=c.hidden, topk=c.topk, E=c.n_experts, tt=tt,
                                   tiles=tiles, union=union)
         return x + y.to(x.dtype)
+
+    def chunkable(self):
+        """Whether the chunk kernels take this block: whole 128-input stages of the hidden rows,
+        and down weights whose rows they can load 16 bytes at a time (the union and decode
+        kernels load single words; every other tensor has the same rule there as here)."""
+        c = self.cfg
+        return c.hidden % 128 == 0 and c.hidden <= 3072 and _aligned(self.pw, self.spw)
 
     def _chunk(self, x, tt, out=None, trace=None):
         """A prompt chunk's rows on the matrix cores (hsd.chunk): the projections run over the
@@ -657,11 +669,24 @@ class NemotronModel:
     # ---- prefill (model.py:259-279): chunks of CHUNK_ROWS rows on the matrix cores, or (few
     # tokens, shapes those kernels do not take) steps of 3 rows through the decode kernels
     def _chunkable(self):
+        """Whether the chunk kernels take this model: their widths, 4-bit mixer projections (a
+        residual is added by that product only), tensors at the alignment of their loads where
+        the decode kernels ask for less, and blocks of these very classes (another one has its
+        own rows())."""
         c = self.cfg
-        return (c.hidden % 128 == 0 and c.hidden <= 3072 and c.moe_inter % 64 == 0 and c.shared_inter % 64 == 0
+        if not (c.hidden % 128 == 0 and c.hidden <= 3072 and c.moe_inter % 64 == 0 and c.shared_inter % 64 == 0
                 and c.mamba_inner % 512 == 0 and c.mamba_inner <= 6144 and c.mamba_head_dim % 16 == 0
                 and c.ssm_state == 128 and c.head_dim == 128 and c.attn_heads % (4 * c.kv_heads) == 0
-                and c.attn_heads * c.head_dim <= 6144 and c.topk <= 8 and c.n_experts <= 256)
+                and c.attn_heads * c.head_dim <= 6144 and c.topk <= 8 and c.n_experts <= 256):
+            return False
+        heads = [] if self.mtp is None else [self.mtp.attn, self.mtp.moe]
+        for b in [*self.blocks, *heads]:
+            kind = type(b)
+            if not (kind is MoEBlock and b.chunkable() or kind is AttnBlock and b.qkv.q4 and b.o_proj.q4
+                    or kind is MambaBlock and b.in_proj.q4 and b.out_proj.q4
+                    and _aligned(b.mixer.conv_w, b.mixer.conv_b)):
+                return False
+        return True
 
     def _prefill_chunk(self, prompt_dev, T, B, cache, with_head):
         """B rows from the cache's position on -> their residual stream [B, D]."""
@@ -678,7 +703,7 @@ class NemotronModel:
             N.call("hsd_prompt_tokens", prompt_dev, T, seq, 1, B, ids, st)
             hd = self.mtp
             pair = nn.head_input(ids, x, self.embedding, hd.enorm, hd.hnorm, eps=c.eps, status=cache.status)
-            hx = chunk.gemm(chunk.prep(pair, sums=False), hd.eh_proj)
+            hx = chunk.gemm(chunk.prep(pair, sums=hd.eh_proj.q4), hd.eh_proj)
             # the head's cache rows are all that a prompt leaves of it: its attention output and
             # its MoE block feed nothing (they run when their statistics are asked for)
             if hd.moe.trace is None:

@@ -71,3 +71,15 @@ def test_strided_weights(dev, T):
         setattr(blk, n, wide[..., :t.shape[-1]])
         assert not getattr(blk, n).is_contiguous()
         assert torch.equal(blk.prefill_sparse(x).view(torch.int16), want.view(torch.int16)), n
+
+
+@pytest.mark.parametrize("name", ["pw", "spw"])
+def test_words_at_any_address(dev, name):
+    """Down weights at a multiple of 4 bytes only, which the chunk's 16-byte loads do not take,
+    go through the union lists."""
+    blk, x = block(dev), rows(dev, 40)
+    assert blk.chunkable()
+    t = getattr(blk, name)
+    setattr(blk, name, torch.zeros(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape).copy_(t))
+    assert not blk.chunkable()
+    assert torch.equal(blk.prefill_sparse(x).view(torch.int16), by_union(blk, x, 32).view(torch.int16))

@@ -136,3 +136,46 @@ def test_chunked_prefill(dev, T):
         u, w = u.double(), w.double()
         assert float((u - w).norm() / w.norm()) < 0.12 / math.sqrt(T) + 2e-2
     assert float((xs[0].double() - xs[2].double()).norm() / xs[2].double().norm()) < 0.24 + 2e-2   # one row
+
+
+def off_by_one(t):
+    """t at an address that is no multiple of 16 bytes."""
+    return torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+
+class OwnRows(Mdl.MambaBlock):
+    pass
+
+
+@pytest.mark.parametrize("change", ["none", "pw", "head spw", "conv_w", "conv_b", "class", "eh_proj"])
+def test_which_models_run_in_chunks(dev, change):
+    """The unpatched rule takes this configuration; weights that the chunk kernels' loads or
+    products do not take, and blocks of other classes, run in steps of 3 rows; a 4-bit eh_proj
+    (1024 inputs) runs in chunks."""
+    m = Mdl.NemotronModel(CFG, seed=5, device=dev, calibrate=False)
+    prompt = np.random.default_rng(7).integers(0, CFG.vocab, 20).astype(np.int32)
+    mamba, moe = m.blocks[0], m.blocks[1]
+    if change == "pw":
+        moe.pw = off_by_one(moe.pw)
+    elif change == "head spw":
+        m.mtp.moe.spw = off_by_one(m.mtp.moe.spw)
+    elif change in ("conv_w", "conv_b"):
+        setattr(mamba.mixer, change, off_by_one(getattr(mamba.mixer, change)))
+    elif change == "class":
+        mamba.__class__ = OwnRows
+    elif change == "eh_proj":
+        w = m.mtp.eh_proj
+        m.mtp.eh_proj = nn.QWeight(*Mdl._Init(3, dev).q4(w.O, w.I, 1.0 / math.sqrt(w.I)))
+    chunks = change in ("none", "eh_proj")
+    assert m._chunkable() is chunks
+    a, b = m.make_cache(cap=8), m.make_cache(cap=8)
+    xa = m.prefill(prompt, a, graph=False).clone()
+    m._chunkable = lambda: False
+    xb = m.prefill(prompt, b, graph=False).clone()
+    assert int(a.status.item()) == 0 and torch.equal(a.seq, b.seq)
+    n = prompt.size - 1
+    for u, v in ((a.head_kv.k[:, :n], b.head_kv.k[:, :n]), (a.head_kv.v[:, :n], b.head_kv.v[:, :n]), (xa, xb)):
+        if chunks:
+            assert float((u.double() - v.double()).norm() / v.double().norm()) < 0.26      # as test_chunked_prefill
+        else:
+            assert torch.equal(u.contiguous().view(torch.int16), v.contiguous().view(torch.int16))
