@@ -401,7 +401,8 @@ int hsd_moe_down_gemm(const uint16_t* hcat, const uint16_t* hsum, const int32_t*
 /* The mixers of a prompt chunk: T consecutive rows at positions P = *pos .. of a prompt of
  * Ttot tokens; the rows past it (V = clamp(Ttot - P, 0, T) are inside) leave nothing behind.
  * hsd_mamba_scan: T rows of hsd_mamba_ssm_gated (the states bit for bit; z's sum over the
- * state in another order) without the per-row checkpoints: the state after row V - 1 goes to slab (cur + V) % nslab (V == 0: nothing).
+ * state in another order) without the per-row checkpoints: the state after row V - 1 goes to
+ * slab (cur + V) % nslab (V == 0: nothing). T <= 524280.
  * workspace: hsd_mamba_scan_workspace_bytes. */
 size_t hsd_mamba_scan_workspace_bytes(int64_t T, int64_t H, int64_t P, int64_t N, int64_t G);
 int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const uint16_t* dt_raw, int64_t dt_ld,

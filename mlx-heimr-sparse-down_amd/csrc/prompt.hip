@@ -533,9 +533,10 @@ extern "C" int hsd_mamba_scan(const uint16_t* conv_in, int64_t conv_in_ld, const
       !cur || !pos || !z)
     return set_error(HSD_ERR_ARG, "%s: null pointer", fn);
   const int64_t DI = H * P, CD = DI + 2 * G * N;
-  if (T < 1 || T > (1 << 20) || Ttot < 0 || Ttot > 0x7FFFFFFF || H <= 0 || G <= 0 || H % G || H > 65535 || P <= 0 ||
+  // k_conv_rows has T / kCR in grid.y
+  if (T < 1 || T > 65535 * kCR || Ttot < 0 || Ttot > 0x7FFFFFFF || H <= 0 || G <= 0 || H % G || H > 65535 || P <= 0 ||
       P % kPB || N != kN || nslab < 1 || nslab > 64 || CD % 8)
-    return set_error(HSD_ERR_SHAPE, "%s: need N == %d, P %% %d == 0, H %% G == 0", fn, kN, kPB);
+    return set_error(HSD_ERR_SHAPE, "%s: need T <= %d, N == %d, P %% %d == 0, H %% G == 0", fn, 65535 * kCR, kN, kPB);
   if (conv_in_ld < CD || dt_ld < H || gate_ld < DI || z_ld < DI + DI / 16)
     return set_error(HSD_ERR_SHAPE, "%s: bad row strides", fn);
   if (((uintptr_t)conv_in | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)conv_slabs | (uintptr_t)ssm_slabs |

@@ -227,3 +227,22 @@ def test_native_entries_cover_the_table():
         f(16, 16, 1 << 80, 8, 1, None)
     assert N.call("hsd_sparse_down_workspace_bytes", 1, 2688, 1856, 3712, 6) == \
         N.lib().hsd_sparse_down_workspace_bytes(1, 2688, 1856, 3712, 6)
+
+
+def scan_args(**kw):
+    """hsd_mamba_scan's arguments, 64 heads of 64 with 16 rows, each replaceable by name."""
+    a = dict(conv_in=4096, conv_in_ld=10304, dt=4096, dt_ld=10304, gate=4096, gate_ld=10304, conv_w=4096, conv_b=4096,
+             A_log=4096, dt_bias=4096, D=4096, ssm=4096, conv=4096, cur=4096, nslab=4, pos=4096, z=4096, z_ld=4352,
+             T=16, total=16, H=64, P=64, N=128, G=8, lo=0.0, hi=1e30, status=None, ws=4096, ws_bytes=1 << 40, stream=None)
+    assert not set(kw) - set(a)
+    return list({**a, **kw}.values())
+
+
+def test_scan_refuses():
+    """Before any launch: addresses that its 16-byte loads do not take, and more rows than the
+    conv kernel's grid."""
+    for name in ("conv_in", "conv_w", "conv_b", "conv", "ssm", "ws"):
+        with pytest.raises(N.HSDError, match="aligned"):
+            N.call("hsd_mamba_scan", *scan_args(**{name: 4104}))
+    with pytest.raises(N.HSDError, match="T <= 524280"):
+        N.call("hsd_mamba_scan", *scan_args(T=524281))
