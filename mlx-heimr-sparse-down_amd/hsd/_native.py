@@ -192,8 +192,10 @@ def ptr(t):
 
 def stream(device=None):
     """The current torch stream of `device` as a hipStream_t."""
-    index = None if device is None else device.index if isinstance(device, torch.device) else torch.device(device).index
-    return _raw_stream(torch.cuda.current_device() if index is None else index)
+    d = device if device is None or isinstance(device, torch.device) else torch.device(device)
+    if d is not None and d.type != "cuda":
+        raise HSDError(f"libhsd takes device tensors only (got a {d.type.upper()} tensor)")
+    return _raw_stream(torch.cuda.current_device() if d is None or d.index is None else d.index)
 
 
 _DT = {torch.bfloat16: DT_BF16, torch.float16: DT_F16, torch.float32: DT_F32}

@@ -246,3 +246,27 @@ def test_scan_refuses():
             N.call("hsd_mamba_scan", *scan_args(**{name: 4104}))
     with pytest.raises(N.HSDError, match="T <= 524280"):
         N.call("hsd_mamba_scan", *scan_args(T=524281))
+
+
+def test_every_call_refuses_cpu_tensors():
+    """The layer above the binding too: HSDError, with and without a GPU."""
+    import torch
+    from hsd import chunk, decode, layout, moe, nn, prefill
+
+    def z(*s, dt=torch.bfloat16):
+        return torch.zeros(s, dtype=dt)
+    i32, f32 = torch.int32, torch.float32
+    nm = (z(8, 128, 16, dt=i32), z(8, 2, 128), z(8, 2, 128), z(128, 16, dt=i32), z(2, 128), z(2, 128))
+    calls = [
+        lambda: decode.sparse_down(z(1, 896), z(1, 6, dt=i32), z(1, 7, dt=f32), *nm, F=128, FS=128, D=128, topk=6),
+        lambda: layout.nibble_transpose(z(8, 4, dt=i32)),
+        lambda: layout.to_neuron_major(z(8, 8, dt=i32), z(8, 1), z(8, 1)),
+        lambda: prefill.build_tiles(z(1, 6, dt=i32), 8, 32),
+        lambda: nn.linear(z(1, 128), nn.QWeight(z(8, 128))),
+        lambda: nn.argmax(z(1, 8, dt=torch.int64)),
+        lambda: nn.pair_norm(z(1, 128), z(1, 128), z(128), z(128)),
+        lambda: moe.router_topk(z(1, 8), z(8, dt=f32), topk=2),
+        lambda: chunk.prep(z(5, 128))]
+    for f in calls:
+        with pytest.raises(N.HSDError, match="device tensors only"):
+            f()
