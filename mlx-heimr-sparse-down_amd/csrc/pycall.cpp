@@ -100,7 +100,11 @@ bool convert(PyObject* o, T& out) {
         PyErr_SetString(g_error, "libhsd takes device tensors only (got a CPU tensor)");
         return false;
       }
-      out = reinterpret_cast<T>(const_cast<void*>(t.const_data_ptr()));
+      // a buffer that the entry point writes: a copy-on-write tensor gets memory of its own first
+      if constexpr (std::is_const_v<std::remove_pointer_t<T>>)
+        out = static_cast<T>(t.const_data_ptr());
+      else
+        out = static_cast<T>(t.mutable_data_ptr());
       return true;
     }
     if (PyLong_Check(o)) {
