@@ -105,6 +105,10 @@ bool convert(PyObject* o, T& out) {
         out = static_cast<T>(t.const_data_ptr());
       else
         out = static_cast<T>(t.mutable_data_ptr());
+      if (!out && t.numel()) {   // a fake tensor: its null would read as "absent"
+        PyErr_SetString(g_error, "libhsd takes device tensors only (got a tensor without memory)");
+        return false;
+      }
       return true;
     }
     if (PyLong_Check(o)) {

@@ -270,3 +270,18 @@ def test_every_call_refuses_cpu_tensors():
     for f in calls:
         with pytest.raises(N.HSDError, match="device tensors only"):
             f()
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+def test_tensors_without_memory_are_refused():
+    """A fake tensor's null pointer must not stand for an argument left out, read or written."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        t = torch.empty(64, dtype=torch.int32, device="cuda")
+    f = N.entry("hsd_permute_nibbles")
+    for args in ((t, 16), (16, t)):
+        with pytest.raises(N.HSDError, match="without memory"):
+            f(*args, 1, 8, 1, 0)
+    with pytest.raises(N.HSDError, match="without memory"):     # status, an optional argument
+        N.call("hsd_mamba_scan", *scan_args(status=t))
