@@ -116,10 +116,16 @@ bool convert(PyObject* o, T& out) {
       return !PyErr_Occurred();
     }
     PyObject* v = PyObject_GetAttrString(o, "value");   // ctypes.c_void_p
-    if (!v) return false;
-    out = v == Py_None ? nullptr : reinterpret_cast<T>(PyLong_AsVoidPtr(v));
-    Py_DECREF(v);
-    return !PyErr_Occurred();
+    if (v && (v == Py_None || PyLong_Check(v))) {
+      out = v == Py_None ? nullptr : reinterpret_cast<T>(PyLong_AsVoidPtr(v));
+      Py_DECREF(v);
+      return !PyErr_Occurred();
+    }
+    Py_XDECREF(v);
+    PyErr_Clear();
+    PyErr_Format(PyExc_TypeError, "a pointer argument takes None, a device tensor, an int or a ctypes pointer, not %s",
+                 Py_TYPE(o)->tp_name);
+    return false;
   } else if constexpr (std::is_floating_point_v<T>) {
     out = static_cast<T>(PyFloat_AsDouble(o));
     return !PyErr_Occurred();

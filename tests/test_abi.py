@@ -285,3 +285,12 @@ def test_tensors_without_memory_are_refused():
             f(*args, 1, 8, 1, 0)
     with pytest.raises(N.HSDError, match="without memory"):     # status, an optional argument
         N.call("hsd_mamba_scan", *scan_args(status=t))
+
+
+def test_pointer_arguments_of_other_types():
+    """What is no pointer is a TypeError that says so (a ctypes string's value is none either)."""
+    for bad in ("words", 1.5, [16], ctypes.c_char_p(b"words"), ctypes.c_float(1.0)):
+        with pytest.raises(TypeError, match="pointer argument"):
+            N.call("hsd_permute_nibbles", bad, 16, 1, 8, 1, 0)
+    with pytest.raises(N.HSDError, match="null"):
+        N.call("hsd_permute_nibbles", ctypes.c_void_p(None), 16, 1, 8, 1, 0)
