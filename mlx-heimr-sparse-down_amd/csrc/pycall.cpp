@@ -141,6 +141,12 @@ bool convert(PyObject* o, T& out) {
   }
 }
 
+// The interpreter's lock given back for a call, and taken again also when it throws.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // An int is a status (0, or an error that is raised); a size is returned.
 template <typename R, typename... A, size_t... I>
 PyObject* invoke(R (*fn)(A...), const char* name, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
@@ -151,11 +157,12 @@ PyObject* invoke(R (*fn)(A...), const char* name, PyObject* const* args, Py_ssiz
     if (!(convert(args[I], std::get<I>(a)) && ...)) return nullptr;
     if constexpr (!std::is_same_v<R, int>) return PyLong_FromLongLong(static_cast<long long>(fn(std::get<I>(a)...)));
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = static_cast<int>(fn(std::get<I>(a)...));
-    Py_END_ALLOW_THREADS
+    {
+      NoGil released;
+      rc = static_cast<int>(fn(std::get<I>(a)...));
+    }
     if (rc != 0) return PyErr_Format(g_error, "%s -> %d: %s", name, rc, g_last_error());
-  } catch (const std::exception& e) {   // a tensor without storage
+  } catch (const std::exception& e) {   // a tensor without storage; an entry point out of host memory
     PyErr_SetString(PyExc_RuntimeError, e.what());
     return nullptr;
   }

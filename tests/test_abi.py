@@ -294,3 +294,43 @@ def test_pointer_arguments_of_other_types():
             N.call("hsd_permute_nibbles", bad, 16, 1, 8, 1, 0)
     with pytest.raises(N.HSDError, match="null"):
         N.call("hsd_permute_nibbles", ctypes.c_void_p(None), 16, 1, 8, 1, 0)
+
+
+def test_an_exception_of_an_entry_point_is_raised(tmp_path):
+    """A C++ exception out of an entry point (bad_alloc) comes back with the interpreter's lock
+    held, as a Python exception. In a process of its own: the binding is pointed at a function
+    that throws."""
+    import shutil
+    import subprocess
+    import sys
+    if not shutil.which("g++"):
+        pytest.skip("no g++")
+    src, so = tmp_path / "t.cpp", tmp_path / "t.so"
+    src.write_text('#include <new>\nextern "C" int thrower(int*, long, long, void*) { throw std::bad_alloc(); }\n')
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    prog = f"""
+import sys, threading, ctypes
+sys.path.insert(0, {os.path.join(ROOT, "mlx-heimr-sparse-down_amd")!r})
+from hsd import _native as N
+N.entry("hsd_seq_add")
+from hsd import _hsdcall
+L = N.lib()
+addr = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+names = {{n: addr(getattr(L, n)) for n in N.EXPORTS if hasattr(_hsdcall, n)}}
+names["hsd_seq_add"] = addr(ctypes.CDLL({str(so)!r}).thrower)
+_hsdcall.bind(N.HSDError, addr(L.hsd_last_error), names)
+stop = threading.Event()
+spin = threading.Thread(target=lambda: [None for _ in iter(stop.is_set, True)])
+spin.start()
+n = 0
+for _ in range(100):
+    try:
+        N.call("hsd_seq_add", 16, 0, 1, 0)
+    except RuntimeError as e:
+        n += "bad_alloc" in str(e)
+stop.set()
+spin.join()
+print("raised", n)
+"""
+    r = subprocess.run([sys.executable, "-c", prog], capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and "raised 100" in r.stdout, (r.returncode, r.stdout[-500:], r.stderr[-500:])
