@@ -62,8 +62,10 @@ def to_neuron_major(w: torch.Tensor, s: torch.Tensor, b: torch.Tensor, chunk: in
     w, s, b = N.contig(w), N.contig(N.as_u16(s)), N.contig(N.as_u16(b))
     *lead, R, CW = w.shape
     G = s.shape[-1]
-    # one launch for the three, where its kernel takes them: matching shapes, few groups
-    if s.shape == b.shape == (*lead, R, G) and R % 8 == 0 and G <= 64 and (s.data_ptr() | b.data_ptr()) % 16 == 0:
+    # one launch for the three, where its kernel takes them: matching shapes, few groups, a
+    # matrix's scales in 31 bits
+    if (s.shape == b.shape == (*lead, R, G) and R % 8 == 0 and G <= 64 and R * G <= 0x7FFFFFFF
+            and (s.data_ptr() | b.data_ptr()) % 16 == 0):
         batch = math.prod(lead)
         pw = torch.empty((*lead, CW * 8, R // 8), dtype=torch.int32, device=w.device)
         ps = torch.empty((*lead, G, R), dtype=s.dtype, device=s.device)
