@@ -150,6 +150,17 @@ def ssm_rows(mixer: Mamba2Mixer, proj, cache: MambaCache, out=None, status=None,
     return y
 
 
+def _rows_into(block):
+    """block.rows_into, unless the block, or a class ahead of the one that defines it, has its
+    own rows()."""
+    for d in (getattr(block, "__dict__", {}), *map(vars, type(block).__mro__)):
+        if "rows_into" in d:
+            return block.rows_into
+        if "rows" in d:
+            return None
+    return None
+
+
 def mamba_verify(block, x3, cache, records):
     """hsd/mamba.py:19-44. One Mamba-2 block on x3 [1, L, *] with the cache advanced by L
     rows (the per-row checkpoints written), remembering in `records` what mamba_rollback
@@ -168,8 +179,9 @@ def mamba_verify(block, x3, cache, records):
         buf = dict(proj=torch.empty((L, block.in_proj.O), dtype=torch.bfloat16, device=x.device),
                    y_pre=torch.empty((L, m.intermediate_size + m.intermediate_size // 16), dtype=torch.float32,
                                      device=x.device))
-        if hasattr(block, "rows_into") and x.data_ptr() % 16 == 0:
-            out = block.rows_into(x, buf, cache, torch.empty_like(x))
+        into = _rows_into(block)
+        if into is not None and x.data_ptr() % 16 == 0:
+            out = into(x, buf, cache, torch.empty_like(x))
         else:
             out = x.clone()
             block.rows(out, buf, cache)
