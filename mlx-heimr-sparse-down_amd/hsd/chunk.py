@@ -42,6 +42,10 @@ def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
     """x [T, I]: bf16 rows (norm: the RMS norm's weight), or with gated_z mamba's z rows (f32,
     I + I/16 values per row) and the gated norm's weight. sums: for 4-bit weights."""
     T, I = x.shape
+    if x.dtype != (torch.float32 if gated_z else torch.bfloat16) or x.stride(1) != 1:
+        raise N.HSDError("prep takes unit-stride bf16 rows, or gated_z's f32 rows")
+    if gated_z and norm is None:
+        raise N.HSDError("gated_z takes a norm weight")
     kind = N.X_GATED_Z if gated_z else N.X_RMS if norm is not None else N.X_BF16
     xp = torch.empty((T, I), dtype=torch.bfloat16, device=x.device)
     hs = torch.empty((T, 3 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
@@ -53,7 +57,16 @@ def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
 def gemm(rows: Rows, W, residual=None, out=None):
     """bf16 y [T, O] = xn W^T (W: nn.QWeight); residual: y = bf16(residual + bf16(xn W^T))
     (4-bit weights; out may be residual)."""
-    T = rows.xp.shape[0]
+    T, I = rows.xp.shape
+    if I != W.I:
+        raise N.HSDError(f"gemm: the rows have {I} inputs, the weight {W.I}")
+    if W.q4 and rows.hs is None:
+        raise N.HSDError("gemm: a 4-bit weight takes rows prepared with their group sums")
+    if not W.q4 and residual is not None:
+        raise N.HSDError("gemm: a residual is added to a 4-bit weight's product only")
+    for t in (out, residual):
+        if t is not None and (t.dtype != torch.bfloat16 or t.shape != (T, W.O) or t.stride(1) != 1):
+            raise N.HSDError(f"gemm: out and residual must be unit-stride bf16 rows [{T}, {W.O}]")
     y = out if out is not None else torch.empty((T, W.O), dtype=torch.bfloat16, device=rows.xp.device)
     st = N.stream(rows.xp.device)
     if W.q4:
@@ -110,6 +123,8 @@ def scan(mixer, proj, cache, pos, total, status=None):
     T = proj.shape[0]
     H, P, Nst, G = mixer.num_heads, mixer.head_dim, mixer.ssm_state_size, mixer.n_groups
     DI, CD = mixer.intermediate_size, mixer.conv_dim
+    if proj.dtype != torch.bfloat16 or proj.shape[1] < DI + CD + H or proj.stride(1) != 1:
+        raise N.HSDError(f"proj needs {DI + CD + H} unit-stride bf16 columns")
     z = torch.empty((T, DI + DI // 16), dtype=torch.float32, device=proj.device)
     nb = N.call("hsd_mamba_scan_workspace_bytes", T, H, P, Nst, G)
     ws = torch.empty(nb, dtype=torch.uint8, device=proj.device)
