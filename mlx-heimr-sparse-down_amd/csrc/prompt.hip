@@ -307,6 +307,11 @@ __global__ __launch_bounds__(64 * kSW, 2) void k_scan(
 // ------------------------------------------------------------------ attention
 constexpr int kHD = 128;
 
+// A bf16 pair with zeros in place of infinities and NaNs.
+__device__ __forceinline__ uint32_t finite2(uint32_t v) {
+  return ((v & 0x7F80u) == 0x7F80u ? 0u : v & 0xFFFFu) | ((v & 0x7F800000u) == 0x7F800000u ? 0u : v & 0xFFFF0000u);
+}
+
 __device__ __forceinline__ bool bad_pos(int P, int V, int64_t smax) { return P < 0 || P + (int64_t)V > smax; }
 
 __global__ __launch_bounds__(256) void k_kv_append(const uint16_t* __restrict__ kv, int64_t ld,
@@ -335,7 +340,10 @@ __global__ __launch_bounds__(256) void k_kv_append(const uint16_t* __restrict__ 
 // probabilities are already a B operand), O^T = V^T P^T. The probabilities enter the second
 // product as three bf16 parts (all 24 bits of the fp32 value), three MFMAs per fragment. K rows are stored with their 16-byte pieces
 // swapped by (key % 16), V transposed with 8-byte pieces swapped by (dim / 2 % 16): no bank
-// conflicts. The last query tiles have the most keys and are launched first.
+// conflicts. The last query tiles have the most keys and are launched first. A masked key's
+// probability is zero, which the product turns into NaN where its V is not finite: a tile that
+// holds keys some row does not see (one or two per workgroup) is looked through for such values,
+// and they are left out of the product and added to the rows that do see them.
 __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restrict__ qkv, int64_t ld,
                                                         const uint16_t* __restrict__ kc,
                                                         const uint16_t* __restrict__ vc, int64_t smax,
@@ -391,6 +399,8 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
   load(0);
   for (int t = 0; t < ntile; ++t) {
     __syncthreads();                                 // the previous tile has been read
+    const bool diag = 64 * t + 63 > P + q0;          // uniform: a key that row q0 does not see
+    bool odd = false;                                // a value of this thread's that is not finite
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int key = 16 * i + (tid >> 4);
@@ -404,14 +414,24 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
       const uint32_t w1[4] = {vr[i][1].x, vr[i][1].y, vr[i][1].z, vr[i][1].w};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const uint32_t a0 = l0 ? w0[c] : 0u, a1 = l1 ? w1[c] : 0u;
+        uint32_t a0 = l0 ? w0[c] : 0u, a1 = l1 ? w1[c] : 0u;
+        if (diag) {
+          const uint32_t f0 = finite2(a0), f1 = finite2(a1);
+          odd = odd || f0 != a0 || f1 != a1;
+          a0 = f0;
+          a1 = f1;
+        }
         const int d = d0 + 2 * c;                     // dims d, d + 1 share (d / 2)
         const int pc = (kp >> 1) ^ ((d >> 1) & 15);
         *reinterpret_cast<uint32_t*>(vt + 128 * d + 8 * pc + 4 * (kp & 1)) = (a0 & 0xFFFFu) | (a1 << 16);
         *reinterpret_cast<uint32_t*>(vt + 128 * (d + 1) + 8 * pc + 4 * (kp & 1)) = (a0 >> 16) | (a1 & 0xFFFF0000u);
       }
     }
-    __syncthreads();
+    bool repair = false;                             // uniform
+    if (diag)
+      repair = __syncthreads_or(odd);
+    else
+      __syncthreads();
     load(t + 1);                                     // past the last tile: its last key, unused
     f32x16 s[2] = {};
 #pragma unroll
@@ -471,6 +491,21 @@ __global__ __launch_bounds__(256, 2) void k_attn_prompt(const uint16_t* __restri
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pm[st], o[d], 0, 0, 0);
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl[st], o[d], 0, 0, 0);
       }
+    if (repair) {
+#pragma unroll 1
+      for (int key = 64 * t; key <= min(64 * t + 63, last); ++key)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            const uint2 w = *reinterpret_cast<const uint2*>(vb + (size_t)key * kHD + 32 * d + 8 * b + 4 * kh);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const uint32_t x = ((u < 2 ? w.x : w.y) >> (16 * (u & 1))) & 0xFFFFu;
+              if ((x & 0x7F80u) == 0x7F80u && key <= qpos) o[d][4 * b + u] += bf16_bits_to_f32(x);
+            }
+          }
+    }
   }
   {
     const uint32_t c = __float_as_uint(l);

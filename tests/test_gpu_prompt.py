@@ -107,6 +107,31 @@ def test_attention_refuses_overflow(dev):
     assert float(kv.k.float().abs().max()) == 0 and float(o.float().abs().max()) == 0
 
 
+@pytest.mark.parametrize("T,pos0,row", [(40, 0, 39), (70, 0, 33), (70, 5, 64), (130, 100, 0), (64, 0, 63)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_attention_is_causal_for_values_that_are_not_finite(dev, T, pos0, row, value):
+    """One value of row `row` is infinite or NaN: the rows ahead of it are bit for bit what they
+    are without it, and so is every other dimension behind it; that one is not finite there."""
+    HQ, HKV, HD, smax = 8, 2, 128, 256
+    g = gen(dev, T)
+    qkv = torch.randn((T, (HQ + 2 * HKV) * HD), device=dev, generator=g).to(torch.bfloat16)
+    old = torch.randn((2, HKV, pos0, HD), device=dev, generator=g).to(torch.bfloat16)
+    dim = 77
+    odd = qkv.clone()
+    odd[row, (HQ + HKV) * HD + dim] = value          # kv head 0
+    out = []
+    for x in (qkv, odd):
+        kv = nn.KVCache(HKV, smax, dev, HD)
+        kv.k[:, :pos0], kv.v[:, :pos0] = old[0], old[1]
+        pos = torch.full((1,), pos0, dtype=torch.int32, device=dev)
+        out.append(chunk.attention(x, kv, pos, pos0 + T, n_heads=HQ, n_kv_heads=HKV, head_dim=HD).view(T, HQ, HD))
+    a, b = out
+    keep = torch.ones((T, HQ, HD), dtype=torch.bool, device=dev)
+    keep[row:, :HQ // HKV, dim] = False
+    assert torch.equal(a.view(torch.int16)[keep], b.view(torch.int16)[keep])
+    assert not bool(torch.isfinite(b.float())[~keep].any())
+
+
 CFG = Mdl.ModelConfig(hidden=512, pattern="MEM*EME", vocab=4096, n_experts=16, topk=6, moe_inter=256, shared_inter=512,
                       max_seq=256, mtp=True)
 
