@@ -204,3 +204,76 @@ def test_which_models_run_in_chunks(dev, change):
             assert float((u.double() - v.double()).norm() / v.double().norm()) < 0.26      # as test_chunked_prefill
         else:
             assert torch.equal(u.contiguous().view(torch.int16), v.contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,T", [(16, 33), (16, 70), (17, 35), (17, 70), (3, 8)])
+def test_prompt_of_several_chunks(dev, rows, T, monkeypatch):
+    """Conv window, recurrent state, earlier chunks' keys, token and head offsets across chunks,
+    a last chunk of one row (for which the head has none) and chunks of a multiple of the ring's
+    4 slabs (the state goes to the slab it came from): against one chunk and against steps of 3
+    rows. Without MoE layers (no ties between experts) two correct runs differ by bf16 roundings
+    alone: 2^-9 each, a dozen of them on a row's way through these layers, a few times that where
+    a norm follows. A lost state, window or key changes rows by a tenth of their size or more.
+    (A state is compared by heads: a state row is a sum of one channel's x times B, and a channel
+    whose x cancels in the conv has an x of nothing but roundings.)"""
+    cfg = Mdl.ModelConfig(hidden=512, pattern="M*MM*", vocab=4096, n_experts=16, topk=6, moe_inter=256, shared_inter=512,
+                          max_seq=256, mtp=True)
+    m = Mdl.NemotronModel(cfg, seed=5, device=dev, calibrate=False)
+    prompt = np.random.default_rng(T).integers(0, cfg.vocab, T).astype(np.int32)
+    runs = []
+    for mode in ("chunks", "one", "steps"):
+        monkeypatch.setattr(Mdl, "CHUNK_ROWS", rows if mode == "chunks" else 2048)
+        if mode == "steps":
+            m._chunkable = lambda: False
+        c = m.make_cache(cap=8)
+        x = m.prefill(prompt, c, graph=False).clone()
+        assert int(c.status.item()) == 0
+        assert c.state()[N.SEQ_POS] == T and c.state()[N.SEQ_HEAD_POS] == T - 1
+        cur = int(c.cur.item())
+        t = [x[0]] + [r for lc in c.layers for r in ((lc.ssm[cur].flatten(1), lc.conv[cur]) if hasattr(lc, "ssm") else
+                                                     (lc.k[:, :T], lc.v[:, :T]))]
+        assert not bool(c.head_kv.k[:, T - 1:].any()) or mode == "steps"
+        runs.append((cur, t + [c.head_kv.k[:, :T - 1], c.head_kv.v[:, :T - 1]]))
+    assert runs[0][0] == runs[1][0] == runs[2][0] == T % 4
+    for other in runs[1:]:
+        for i, (u, v) in enumerate(zip(runs[0][1], other[1])):
+            u, v = u.double(), v.double()
+            err = (u - v).norm(dim=-1) / v.norm(dim=-1).clamp_min(1e-3 * float(v.norm(dim=-1).max()))
+            assert float(err.max()) < 0.04, (i, float(err.max()))
+
+
+@pytest.mark.parametrize("T", [5, 33, 100])
+def test_blocks_on_the_same_rows(dev, T):
+    """Each block of the model on the same input rows, as a chunk and in steps of 3 rows: one
+    layer's roundings (2^-9 of a row's update, two or three of them, against the update itself);
+    MoE rows but the few whose last expert is nearly tied. 100 rows: 64-slot tiles (100 * 6 >= 32
+    * 16)."""
+    m = Mdl.NemotronModel(CFG, seed=5, device=dev, calibrate=False)
+    g = gen(dev, T)
+    x = torch.randn((T, CFG.hidden), device=dev, generator=g).to(torch.bfloat16)
+    x[:, 0] = m.c0
+    for t, blk in zip(CFG.pattern[:4], m.blocks):
+        a, b = m.make_cache(cap=8), m.make_cache(cap=8)
+        li = CFG.pattern.index(t)
+        u, v = x.clone(), x.clone()
+        if t == "E":
+            blk.chunk(u)
+        else:
+            blk.chunk(u, a.layers[li], a.pos, T, status=a.status)
+        buf = m._bufs[3]
+        for r in range(0, T, 3):
+            n = min(3, T - r)
+            if t == "E":
+                blk.rows(v[r:r + n], buf)
+                continue
+            if t == "M":
+                blk.rows(v[r:r + n], buf, b.layers[li], status=b.status)
+                N.call("hsd_mamba_select_row", b.cur, None, n, n, Mdl.NSLAB, None, N.stream(dev))
+            else:
+                blk.rows(v[r:r + n], buf, b.layers[li], b.pos, status=b.status)
+            N.call("hsd_seq_add", b.seq, N.SEQ_POS, n, N.stream(dev))
+        step = (v.double() - x.double()).norm(dim=-1)
+        err = (u.double() - v.double()).norm(dim=-1) / step
+        far = err > 0.03
+        assert float(far.double().mean()) <= (0.05 if t == "E" else 0.0), (t, float(err.max()))
+        assert int(a.status.item()) == 0 and int(b.status.item()) == 0
