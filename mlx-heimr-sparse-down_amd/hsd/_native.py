@@ -192,10 +192,13 @@ def ptr(t):
 
 def stream(device=None):
     """The current torch stream of `device` as a hipStream_t."""
-    d = device if device is None or isinstance(device, torch.device) else torch.device(device)
-    if d is not None and d.type != "cuda":
-        raise HSDError(f"libhsd takes device tensors only (got a {d.type.upper()} tensor)")
-    return _raw_stream(torch.cuda.current_device() if d is None or d.index is None else d.index)
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:                                    # no device, its name, or a CPU tensor's
+        d = torch.device("cuda" if device is None else device)
+        if d.type != "cuda":
+            raise HSDError(f"libhsd takes device tensors only (got a {d.type.upper()} tensor)")
+        index = torch.cuda.current_device() if d.index is None else d.index
+    return _raw_stream(index)
 
 
 _DT = {torch.bfloat16: DT_BF16, torch.float16: DT_F16, torch.float32: DT_F32}

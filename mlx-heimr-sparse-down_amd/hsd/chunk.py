@@ -42,39 +42,49 @@ def prep(x, norm=None, eps=1e-5, gated_z=False, sums=True):
     """x [T, I]: bf16 rows (norm: the RMS norm's weight), or with gated_z mamba's z rows (f32,
     I + I/16 values per row) and the gated norm's weight. sums: for 4-bit weights."""
     T, I = x.shape
-    if x.dtype != (torch.float32 if gated_z else torch.bfloat16) or x.stride(1) != 1:
+    ld, unit = x.stride()
+    if unit != 1 or x.dtype != (torch.float32 if gated_z else torch.bfloat16):
         raise N.HSDError("prep takes unit-stride bf16 rows, or gated_z's f32 rows")
     if gated_z and norm is None:
         raise N.HSDError("gated_z takes a norm weight")
     kind = N.X_GATED_Z if gated_z else N.X_RMS if norm is not None else N.X_BF16
     xp = torch.empty((T, I), dtype=torch.bfloat16, device=x.device)
     hs = torch.empty((T, 3 * group_pitch(I)), dtype=torch.bfloat16, device=x.device) if sums else None
-    N.call("hsd_rows_prep", x, x.stride(0), kind, norm, float(eps), xp, hs, T, I,
+    N.call("hsd_rows_prep", x, ld, kind, norm, float(eps), xp, hs, T, I,
            N.stream(x.device))
     return Rows(xp, hs)
+
+
+def _row_stride(t, T, O):
+    ld, unit = t.stride()
+    if t.dtype != torch.bfloat16 or unit != 1 or t.shape != (T, O):
+        raise N.HSDError(f"gemm: out and residual must be unit-stride bf16 rows [{T}, {O}]")
+    return ld
 
 
 def gemm(rows: Rows, W, residual=None, out=None):
     """bf16 y [T, O] = xn W^T (W: nn.QWeight); residual: y = bf16(residual + bf16(xn W^T))
     (4-bit weights; out may be residual)."""
-    T, I = rows.xp.shape
+    xp, hs = rows.xp, rows.hs
+    T, I = xp.shape
+    q4, y, rld = W.q4, out, 0
     if I != W.I:
         raise N.HSDError(f"gemm: the rows have {I} inputs, the weight {W.I}")
-    if W.q4 and rows.hs is None:
+    if q4 and hs is None:
         raise N.HSDError("gemm: a 4-bit weight takes rows prepared with their group sums")
-    if not W.q4 and residual is not None:
-        raise N.HSDError("gemm: a residual is added to a 4-bit weight's product only")
-    for t in (out, residual):
-        if t is not None and (t.dtype != torch.bfloat16 or t.shape != (T, W.O) or t.stride(1) != 1):
-            raise N.HSDError(f"gemm: out and residual must be unit-stride bf16 rows [{T}, {W.O}]")
-    y = out if out is not None else torch.empty((T, W.O), dtype=torch.bfloat16, device=rows.xp.device)
-    st = N.stream(rows.xp.device)
-    if W.q4:
-        N.call("hsd_gemm_q4", rows.xp, rows.hs, W.w, W.scales, W.biases, y,
-               y.stride(0), residual, 0 if residual is None else residual.stride(0), T, W.O, W.I, st)
+    if residual is not None:
+        if not q4:
+            raise N.HSDError("gemm: a residual is added to a 4-bit weight's product only")
+        rld = _row_stride(residual, T, W.O)
+    if out is None:
+        y, ld = torch.empty((T, W.O), dtype=torch.bfloat16, device=xp.device), W.O
     else:
-        N.call("hsd_gemm_bf16", rows.xp, rows.xp.stride(0), 0 if rows.hs is None else 1, W.w, y,
-               y.stride(0), T, W.O, W.I, st)
+        ld = rld if out is residual else _row_stride(out, T, W.O)
+    st = N.stream(xp.device)
+    if q4:
+        N.call("hsd_gemm_q4", xp, hs, W.w, W.scales, W.biases, y, ld, residual, rld, T, W.O, I, st)
+    else:
+        N.call("hsd_gemm_bf16", xp, I, 0 if hs is None else 1, W.w, y, ld, T, W.O, I, st)
     return y
 
 
@@ -123,12 +133,13 @@ def scan(mixer, proj, cache, pos, total, status=None):
     T = proj.shape[0]
     H, P, Nst, G = mixer.num_heads, mixer.head_dim, mixer.ssm_state_size, mixer.n_groups
     DI, CD = mixer.intermediate_size, mixer.conv_dim
-    if proj.dtype != torch.bfloat16 or proj.shape[1] < DI + CD + H or proj.stride(1) != 1:
+    ld, unit = proj.stride()
+    if unit != 1 or proj.dtype != torch.bfloat16 or proj.shape[1] < DI + CD + H:
         raise N.HSDError(f"proj needs {DI + CD + H} unit-stride bf16 columns")
     z = torch.empty((T, DI + DI // 16), dtype=torch.float32, device=proj.device)
     nb = N.call("hsd_mamba_scan_workspace_bytes", T, H, P, Nst, G)
     ws = torch.empty(nb, dtype=torch.uint8, device=proj.device)
-    base, es, ld = proj.data_ptr(), proj.element_size(), proj.stride(0)
+    base, es = proj.data_ptr(), 2
     lo, hi = mixer.time_step_limit
     N.call("hsd_mamba_scan", ctypes.c_void_p(base + DI * es), ld, ctypes.c_void_p(base + (DI + CD) * es), ld, proj,
            ld, N.contig(mixer.conv_w), N.contig(mixer.conv_b), N.contig(mixer.A_log),

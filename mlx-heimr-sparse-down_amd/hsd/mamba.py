@@ -153,11 +153,13 @@ def ssm_rows(mixer: Mamba2Mixer, proj, cache: MambaCache, out=None, status=None,
 def _rows_into(block):
     """block.rows_into, unless the block, or a class ahead of the one that defines it, has its
     own rows()."""
-    for d in (getattr(block, "__dict__", {}), *map(vars, type(block).__mro__)):
-        if "rows_into" in d:
-            return block.rows_into
-        if "rows" in d:
+    own = getattr(block, "__dict__", ())
+    for k in type(block).__mro__:
+        if "rows" in own:
             return None
+        own = k.__dict__
+        if "rows_into" in own:
+            return block.rows_into
     return None
 
 
