@@ -369,7 +369,8 @@ int hsd_gemm_q4(const uint16_t* xp, const uint16_t* hs, const uint32_t* w, const
 int hsd_gemm_bf16(const uint16_t* x, int64_t x_ld, int permuted, const uint16_t* w, uint16_t* y,
                   int64_t y_ld, int64_t T, int64_t O, int64_t I, void* stream);
 
-/* hsd_prefill_tiles without a workspace, with ntiles[0] = the routed tiles in use. */
+/* hsd_prefill_tiles without a workspace, for E <= 4096, with ntiles[0] = the routed tiles in
+ * use. */
 int hsd_moe_tiles(const int32_t* sel, int64_t T, int64_t topk, int64_t E, int64_t tt,
                   int32_t* tile_e, int32_t* tile_slot, int32_t* ntiles, int32_t* dev_status,
                   void* stream);
@@ -436,7 +437,8 @@ int hsd_prompt_advance(int32_t* seq, int64_t T, int64_t B, int64_t nslab, void* 
  * Replaces hsd/prefill.py:247-278 `build_tiles(sel, E, tt)`: slots t*topk+k stably
  * sorted by expert (ties by slot id), ceil(count/tt) tiles per expert, then
  * ceil(T/tt) shared tiles (expert E); fixed NT = T*topk/tt + E + ceil(T/tt), -1 pads.
- * tile_e [NT] int32, tile_slot [NT*tt] int32. workspace: hsd_prefill_tiles_workspace_bytes. */
+ * tile_e [NT] int32, tile_slot [NT*tt] int32. E <= 910. workspace:
+ * hsd_prefill_tiles_workspace_bytes (asked for, not used). */
 int64_t hsd_prefill_num_tiles(int64_t T, int64_t topk, int64_t E, int64_t tt);
 size_t hsd_prefill_tiles_workspace_bytes(int64_t T, int64_t topk, int64_t E);
 int hsd_prefill_tiles(const int32_t* sel, int64_t T, int64_t topk, int64_t E, int64_t tt,

@@ -517,9 +517,10 @@ __global__ __launch_bounds__(256, MT == 32 ? 3 : 2) void k_gemm_q4(GemmArgs a) {
 // each: a v_perm pairs two neurons' halves and a shift and an and-or make the bf16 pair, so
 // the lane's outputs are 4 consecutive columns, one per MFMA. The weight rows' 64-byte
 // quarters are swapped in neighbouring pairs for the upper 8 rows of every 16, so the two lane
-// halves read different banks. Every neuron of the layer is multiplied: a tile of 16 or more
-// tokens has a live token in nearly every row (90 % zeros: 1 - 0.9^24 = 92 %), where the
-// union lists (k_gemm in prefill.hip) save nothing for their passes over h.
+// halves read different banks. Every neuron of the layer is multiplied: a tile of 24 tokens has
+// a live token in nearly every row (90 % zeros: 1 - 0.9^24 = 92 %), where the union lists (k_gemm
+// in prefill.hip) save nothing for their passes over h. Tiles of few tokens read mostly dead rows
+// (2.8 tokens: 74 %): up to 12 rows a block takes the union lists (hsd/model.py).
 struct DownArgs {
   const uint16_t* h;       // [T, topk*F + FS]
   const uint16_t* hsum;    // [T * (topk + 1), 3 GPH]

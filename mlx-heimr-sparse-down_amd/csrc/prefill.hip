@@ -1007,7 +1007,8 @@ extern "C" int hsd_prefill_tiles(const int32_t* sel, int64_t T, int64_t topk, in
   const size_t need = hsd_prefill_tiles_workspace_bytes(T, topk, E);
   if (!workspace || workspace_bytes < need)
     return set_error(HSD_ERR_WORKSPACE, "%s: workspace needs %zu bytes", fn, need);
-  if ((18 * E + 1) * sizeof(int) > 65536) return set_error(HSD_ERR_SHAPE, "%s: E too large for LDS", fn);
+  // the entry point's bound (the kernel's LDS holds E counts); hsd_moe_tiles takes up to 4096
+  if (E > 910) return set_error(HSD_ERR_SHAPE, "%s: at most 910 experts", fn);
   hipLaunchKernelGGL(k_tiles, dim3((unsigned)E), dim3(kTT), (size_t)E * sizeof(int), as_stream(stream), sel, (int)T,
                      (int)topk, (int)E, (int)tt, tile_e, tile_slot, (int32_t*)nullptr, dev_status);
   return check_launch(fn);

@@ -373,8 +373,8 @@ class MoEBlock:
     def _chunk(self, x, tt, out=None, trace=None):
         """A prompt chunk's rows on the matrix cores (hsd.chunk): the projections run over the
         tiles of (token, slot) pairs sorted by expert, so an expert's weights are read once
-        per tile and not once per token, and every down row of a tile (with the tokens of a
-        tile nearly every row has a live one). No row's result depends on the zeros of another,
+        per tile and not once per token, and every down row for each tile (24 tokens of 90 %
+        zeros have a live one in 92 % of them). No row's result depends on the zeros of another,
         so both modes are the same bits."""
         c = self.cfg
         most = chunk.moe_rows(c.hidden, c.moe_inter, c.shared_inter, c.topk)
@@ -730,13 +730,15 @@ class NemotronModel:
     def prefill(self, tokens, cache: ModelCache, with_head=None, graph=True):
         """tokens [T] (host ints or a tensor) -> the residual stream of the last position
         [1, D] (pre norm_f), with every cache advanced by T rows (and, with the MTP head,
-        its cache holding the rows (h_p, tok_{p+1}), p < T-1)."""
+        its cache holding the rows (h_p, tok_{p+1}), p < T-1). graph: the 3-row steps replay
+        one captured graph (chunks are launched as they are, a few hundred kernels a prompt)."""
         with_head = (self.mtp is not None) if with_head is None else with_head
         prompt = torch.as_tensor(tokens, dtype=torch.int32).to(self.device)
         T = int(prompt.numel())
         nsteps = (T + 2) // 3
         if T < 1 or 3 * nsteps > self.cfg.max_seq:
-            # the last 3-row step writes attention rows up to 3 * nsteps - 1
+            # the last 3-row step writes attention rows up to 3 * nsteps - 1; a chunk writes T, but
+            # whether a prompt fits does not depend on which path its model's tensors take
             raise N.HSDError(f"a {T}-token prompt needs {3 * nsteps} attention cache rows (3-row prefill steps); "
                              f"max_seq is {self.cfg.max_seq}")
         if T > 3 and self._chunkable():
